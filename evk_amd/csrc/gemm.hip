@@ -1,15 +1,11 @@
 // fp16 GEMM / GEMV for gfx950: the kernels behind evk::ai::matmul
 // (reference: evk_ai.cpp:254-330 host side, shaders/matmul.comp:44-141).
 //
-// Tiled kernel: a workgroup computes a BM x BN tile of C with 4 waves; each
-// wave owns a (BM/WGM) x (BN/WGN) sub-tile made of 32x32 MFMA accumulators
-// (v_mfma_f32_32x32x16_f16, fp32 accumulation).  A and B tiles of BK along
-// K are staged in LDS, double-buffered, always stored k-contiguous
-// ([row][k], 16-byte chunks XOR-swizzled by row).  Operands that arrive
-// k-contiguous in memory (A row-major, B stored (N,K)) are copied as 16-byte
-// chunks; operands that arrive m/n-contiguous (A stored (K,M), B row-major
-// (K,N)) are transposed in registers in 8x8 blocks on the way to LDS.  The
-// global loads of tile t+1 are issued before the MFMAs of tile t.
+// MFMA kernel (gemm_mfma): BM x BN tiles of C, operand tiles of 64 along K in
+// LDS as they lie in memory, v_mfma_f32_16x16x32_f16 with fp32 accumulation.
+// Aligned operands go from HBM straight into LDS; any others (odd row
+// lengths, 2-byte aligned pointers, operands past the 2 GiB a buffer
+// descriptor spans) through registers.
 //
 // Skinny kernel (M <= 16, B row-major): bandwidth-bound, streams B once with
 // 16-byte coalesced loads, fp32 accumulation in registers, split-K across
@@ -22,190 +18,6 @@
 namespace evkhip {
 
 namespace {
-
-template <int BM_, int BN_, int BK_, int WGM_, int WGN_>
-struct TileCfg {
-    static constexpr int BM = BM_, BN = BN_, BK = BK_, WGM = WGM_, WGN = WGN_;
-    static constexpr int NT = WGM * WGN * 64;
-    static constexpr int WM = BM / WGM, WN = BN / WGN;
-    static constexpr int TM = WM / 32, TN = WN / 32;
-    static constexpr int KC = BK / 8;  // 16-byte chunks per LDS row
-    static_assert(TM >= 1 && TN >= 1, "wave tile must hold a 32x32 MFMA tile");
-    static_assert(BK % 16 == 0 && KC <= 8, "BK must be 16..64");
-};
-
-// Element offset (in halves) of chunk `c` of LDS row `r` (rows of BK halves).
-template <int BK>
-DEV int lds_off(int r, int c) {
-    constexpr int KC = BK / 8;
-    return r * BK + ((c ^ (r & (KC - 1))) << 3);
-}
-
-// ---- k-contiguous operand: ROWS x BK tile, chunk copies --------------------
-template <int ROWS, int BK, int NT>
-struct DirectLoader {
-    static constexpr int KC = BK / 8;
-    static constexpr int CHUNKS = ROWS * KC;
-    static constexpr int PER = (CHUNKS + NT - 1) / NT;
-    u32x4 r[PER];
-
-    DEV void load(const f16* __restrict__ src, int64_t ld, int row0, int nrows, int k0, int K) {
-#pragma unroll
-        for (int i = 0; i < PER; ++i) {
-            int c = threadIdx.x + i * NT;
-            int row = c / KC, kc = c % KC;
-            int gr = row0 + row, gk = k0 + kc * 8;
-            u32x4 v = {0u, 0u, 0u, 0u};
-            if ((CHUNKS % NT == 0 || c < CHUNKS) && gr < nrows && gk < K)
-                v = *reinterpret_cast<const u32x4*>(src + (int64_t)gr * ld + gk);
-            r[i] = v;
-        }
-    }
-    DEV void store(f16* lds) const {
-#pragma unroll
-        for (int i = 0; i < PER; ++i) {
-            int c = threadIdx.x + i * NT;
-            if (CHUNKS % NT == 0 || c < CHUNKS) {
-                int row = c / KC, kc = c % KC;
-                *reinterpret_cast<u32x4*>(lds + lds_off<BK>(row, kc)) = r[i];
-            }
-        }
-    }
-};
-
-// ---- m/n-contiguous operand: memory holds BK rows of ROWS contiguous halves;
-// LDS wants ROWS rows of BK.  8x8 register transposes. ------------------------
-template <int ROWS, int BK, int NT>
-struct TransLoader {
-    static constexpr int NB = ROWS / 8, KB = BK / 8;
-    static constexpr int BLOCKS = NB * KB;
-    static constexpr int PER = (BLOCKS + NT - 1) / NT;
-    u32x4 r[PER][8];
-
-    DEV void load(const f16* __restrict__ src, int64_t ld, int row0, int nrows, int k0, int K) {
-#pragma unroll
-        for (int i = 0; i < PER; ++i) {
-            int q = threadIdx.x + i * NT;
-            int kb = q / NB, nb = q % NB;
-            int gn = row0 + nb * 8;
-            bool okb = (BLOCKS % NT == 0 || q < BLOCKS) && gn < nrows;
-#pragma unroll
-            for (int rr = 0; rr < 8; ++rr) {
-                int gk = k0 + kb * 8 + rr;
-                u32x4 v = {0u, 0u, 0u, 0u};
-                if (okb && gk < K) v = *reinterpret_cast<const u32x4*>(src + (int64_t)gk * ld + gn);
-                r[i][rr] = v;
-            }
-        }
-    }
-    DEV void store(f16* lds) const {
-#pragma unroll
-        for (int i = 0; i < PER; ++i) {
-            int q = threadIdx.x + i * NT;
-            if (BLOCKS % NT == 0 || q < BLOCKS) {
-                int kb = q / NB, nb = q % NB;
-                u32x4 t[8];
-                transpose8x8(r[i], t);
-#pragma unroll
-                for (int c = 0; c < 8; ++c)
-                    *reinterpret_cast<u32x4*>(lds + lds_off<BK>(nb * 8 + c, kb)) = t[c];
-            }
-        }
-    }
-};
-
-template <bool TRANS, int ROWS, int BK, int NT>
-using LoaderFor = typename std::conditional<TRANS, TransLoader<ROWS, BK, NT>, DirectLoader<ROWS, BK, NT>>::type;
-
-// TA: A stored (K,M).  TB: B stored (N,K).
-template <class Cfg, bool TA, bool TB>
-__global__ __launch_bounds__(Cfg::NT) void gemm_tiled(GemmArgs p) {
-    constexpr int BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK, NT = Cfg::NT;
-    constexpr int TM = Cfg::TM, TN = Cfg::TN;
-    __shared__ __attribute__((aligned(16))) f16 sA[2][BM * BK];
-    __shared__ __attribute__((aligned(16))) f16 sB[2][BN * BK];
-
-    const int M = p.M, N = p.N, K = p.K;
-    const int bz = blockIdx.z;
-    const f16* __restrict__ A = p.A + (int64_t)bz * p.sA;
-    const f16* __restrict__ B = p.B + (int64_t)bz * p.sB;
-    f16* __restrict__ Cp = p.C + (int64_t)bz * p.sC;
-
-    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int wm0 = (wave / Cfg::WGN) * Cfg::WM, wn0 = (wave % Cfg::WGN) * Cfg::WN;
-    const int l32 = lane & 31, lg = lane >> 5;
-
-    // A: logical (M,K).  !TA: row-major ld=K, rows m.  TA: memory (K,M), ld=M.
-    LoaderFor<TA, BM, BK, NT> la;
-    LoaderFor<!TB, BN, BK, NT> lb;
-    const int64_t ldA = TA ? M : K;
-    const int64_t ldB = TB ? K : N;
-
-    floatx16 acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
-
-    const int KT = (K + BK - 1) / BK;
-    la.load(A, ldA, m0, M, 0, K);
-    lb.load(B, ldB, n0, N, 0, K);
-    la.store(sA[0]);
-    lb.store(sB[0]);
-    __syncthreads();
-
-    for (int kt = 0; kt < KT; ++kt) {
-        const int cur = kt & 1;
-        const bool more = kt + 1 < KT;
-        if (more) {
-            la.load(A, ldA, m0, M, (kt + 1) * BK, K);
-            lb.load(B, ldB, n0, N, (kt + 1) * BK, K);
-        }
-        const f16* a_s = sA[cur];
-        const f16* b_s = sB[cur];
-#pragma unroll
-        for (int ks = 0; ks < BK / 16; ++ks) {
-            half8 af[TM], bf[TN];
-#pragma unroll
-            for (int i = 0; i < TM; ++i)
-                af[i] = *reinterpret_cast<const half8*>(a_s + lds_off<BK>(wm0 + i * 32 + l32, ks * 2 + lg));
-#pragma unroll
-            for (int j = 0; j < TN; ++j)
-                bf[j] = *reinterpret_cast<const half8*>(b_s + lds_off<BK>(wn0 + j * 32 + l32, ks * 2 + lg));
-#pragma unroll
-            for (int i = 0; i < TM; ++i)
-#pragma unroll
-                for (int j = 0; j < TN; ++j) acc[i][j] = mfma32(af[i], bf[j], acc[i][j]);
-        }
-        if (more) {
-            la.store(sA[cur ^ 1]);
-            lb.store(sB[cur ^ 1]);
-        }
-        __syncthreads();
-    }
-
-    // Epilogue: D element e of lane l -> row 8*(e/4)+4*lg+(e%4), col l32.
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            const int col = n0 + wn0 + j * 32 + l32;
-            if (col >= N) continue;
-#pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const int row = m0 + wm0 + i * 32 + 8 * (e >> 2) + 4 * lg + (e & 3);
-                if (row < M) {
-                    f16* dst = Cp + (int64_t)row * N + col;
-                    float v = acc[i][j][e];
-                    if (p.acc) v += (float)*dst;
-                    *dst = (f16)v;
-                }
-            }
-        }
-}
 
 // ---- MFMA kernel: BM x BN tiles; 4 waves of (BM/2) x (BN/2), or for 256x256
 // tiles 8 waves of 128 x 64 (two waves per SIMD: one wave's LDS reads and
@@ -290,6 +102,54 @@ DEV half8 frag_t(const f16* t, int k0, int c0, int g, int trow, int tcol) {
     return cat4(lds_read_tr(at(k)), lds_read_tr(at(k + 4)));
 }
 
+// The same tile through registers, for operands of any alignment and size:
+// load() requests the 16-byte chunks (global loads at 2-byte aligned 64-bit
+// addresses; the last, partial chunk of a row element by element, so that
+// nothing past the row enters the sums), store() writes them to LDS in
+// tile_to_lds's layout.
+template <int ROWS, int COLS, bool KCONTIG, int NT>
+struct RagTile {
+    static constexpr int CPR = COLS / 8, PER = ROWS * CPR / NT;
+    static_assert(PER >= 1 && ROWS * CPR % NT == 0, "tile shape");
+    u32x4 r[PER];
+
+    DEV void load(const f16* src, int64_t ld, int64_t r0, int64_t c0, int nr, int nc, int tid) {
+        const int row = tid / CPR, col = (tid % CPR) * 8;  // chunk i: NT / CPR rows further each
+        const f16* p = src + (r0 + row) * ld + c0 + col;
+        if (r0 + ROWS <= nr && c0 + COLS <= nc) {  // workgroup-uniform: the tile is whole
+#pragma unroll
+            for (int i = 0; i < PER; ++i) __builtin_memcpy(&r[i], p + (int64_t)i * (NT / CPR) * ld, 16);
+            return;
+        }
+        const int64_t left = nc - (c0 + col);
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const f16* q = p + (int64_t)i * (NT / CPR) * ld;
+            u32x4 v = {0u, 0u, 0u, 0u};
+            if (r0 + row + i * (NT / CPR) < nr && left > 0) {
+                if (left >= 8) {
+                    __builtin_memcpy(&v, q, 16);
+                } else {
+                    half8 h = {};
+#pragma unroll
+                    for (int e = 0; e < 7; ++e)
+                        if (e < left) h[e] = q[e];
+                    v = as_u32x4(h);
+                }
+            }
+            r[i] = v;
+        }
+    }
+    DEV void store(f16* lds, int tid) const {
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const int row = tid / CPR + i * (NT / CPR), ch = tid % CPR;
+            const int slot = KCONTIG ? (ch ^ (row & 7)) : (ch ^ (2 * (row & 3)));
+            *reinterpret_cast<u32x4*>(lds + row * COLS + slot * 8) = r[i];
+        }
+    }
+};
+
 DEV int xcd_tile(int w, int total) {
     if (total % 8) return w;
     return (w % 8) * (total / 8) + w / 8;  // XCD w%8 gets a contiguous range
@@ -312,12 +172,12 @@ DEV void wait_vmcnt(int n) {
     }
 }
 
-template <int BM, int BN, bool TA, bool TB, int NWV = 4, int KG = 1>
+template <int BM, int BN, bool TA, bool TB, int NWV = 4, int KG = 1, bool RAG = false>
 __global__ __launch_bounds__(64 * NWV * KG, 1) void gemm_mfma(GemmArgs p, int tiles_m, int tiles_n) {
     constexpr int WGN = NWV / 2;  // waves along N (2 along M)
     constexpr int BK = MB_K, WM = BM / 2, WN = BN / WGN, FM = WM / 16, FN = WN / 16;
     constexpr int A_EL = BM * BK, B_EL = BN * BK, STAGE = A_EL + B_EL;
-    constexpr int NST = KG > 1 ? 2 : mfma_stages<BM>();  // per K group
+    constexpr int NST = KG > 1 || RAG ? 2 : mfma_stages<BM>();  // per K group
     constexpr int LPT = (BM * BK / 512 + BN * BK / 512) / NWV;  // DMA loads per wave per tile
     constexpr int OUT_LD = WN + 8;
     constexpr int OUT_EL = NWV * WM * OUT_LD;
@@ -349,8 +209,19 @@ __global__ __launch_bounds__(64 * NWV * KG, 1) void gemm_mfma(GemmArgs p, int ti
     const int wm0 = (wave / WGN) * WM, wn0 = (wave % WGN) * WN;
     const int trow = l16 >> 2, tcol = (l16 & 3) * 4;
 
-    const __amdgpu_buffer_rsrc_t ares = buf_rsrc(A, (uint32_t)((int64_t)M * K * 2));
-    const __amdgpu_buffer_rsrc_t bres = buf_rsrc(B, (uint32_t)((int64_t)K * N * 2));
+    // RAG: every chunk is bounds-checked against the matrix; the descriptors
+    // (whose sizes are 32-bit) serve the other form only
+    const __amdgpu_buffer_rsrc_t ares = buf_rsrc(A, RAG ? 0u : (uint32_t)((int64_t)M * K * 2));
+    const __amdgpu_buffer_rsrc_t bres = buf_rsrc(B, RAG ? 0u : (uint32_t)((int64_t)K * N * 2));
+    RagTile<TA ? BK : BM, TA ? BM : BK, !TA, 64 * NWV> ra;
+    RagTile<TB ? BN : BK, TB ? BK : BN, TB, 64 * NWV> rb;
+    const int gtid = wave * 64 + lane;
+    auto fetch = [&](int k0) {
+        if (TA) ra.load(A, M, k0, m0, K, M, gtid);
+        else ra.load(A, K, m0, k0, M, K, gtid);
+        if (TB) rb.load(B, K, n0, k0, N, K, gtid);
+        else rb.load(B, N, k0, n0, K, N, gtid);
+    };
     auto issue = [&](int k0, f16* sa, f16* sb) {
         if (TA) tile_to_lds<BK, BM, false, NWV>(ares, M, k0, m0, K, M, sa, wave, lane);
         else tile_to_lds<BM, BK, true, NWV>(ares, K, m0, k0, M, K, sa, wave, lane);
@@ -407,21 +278,44 @@ __global__ __launch_bounds__(64 * NWV * KG, 1) void gemm_mfma(GemmArgs p, int ti
     const int KT_ALL = (K + BK - 1) / BK, per = (KT_ALL + KG - 1) / KG;
     const int kt_base = kg * per, KT = max(0, min(KT_ALL - kt_base, per));
     f16* gsm = smem + kg * NST * STAGE;
-#pragma unroll
-    for (int t2 = 0; t2 < NST - 1; ++t2)
-        if (t2 < KT) issue((kt_base + t2) * BK, gsm + t2 * STAGE, gsm + t2 * STAGE + A_EL);
-    for (int kt = 0; kt < per; ++kt) {
-        // this wave's loads of tile kt are in LDS once at most the loads of
-        // the younger tiles in flight remain (loads complete in order)
-        wait_vmcnt(LPT * max(0, min(NST - 2, KT - 1 - kt)));
-        __syncthreads();  // everyone's; the stage of tile kt-1 is free again
-        if (kt + NST - 1 < KT) {
-            f16* nxt = gsm + ((kt + NST - 1) % NST) * STAGE;
-            issue((kt_base + kt + NST - 1) * BK, nxt, nxt + A_EL);
+    if constexpr (RAG) {
+        // two stages: tile kt + 1 is requested before tile kt is multiplied
+        // and written to the other stage after (everyone has left that stage
+        // once the barrier that published tile kt is passed)
+        if (KT > 0) {
+            fetch(kt_base * BK);
+            ra.store(gsm, gtid);
+            rb.store(gsm + A_EL, gtid);
         }
-        if (kt >= KT) continue;
-        const f16* cur = gsm + (kt % NST) * STAGE;
-        compute(cur, cur + A_EL);
+        for (int kt = 0; kt < per; ++kt) {
+            if (kt + 1 < KT) fetch((kt_base + kt + 1) * BK);
+            __syncthreads();
+            if (kt >= KT) continue;
+            const f16* cur = gsm + (kt % 2) * STAGE;
+            compute(cur, cur + A_EL);
+            if (kt + 1 < KT) {
+                f16* nxt = gsm + ((kt + 1) % 2) * STAGE;
+                ra.store(nxt, gtid);
+                rb.store(nxt + A_EL, gtid);
+            }
+        }
+    } else {
+#pragma unroll
+        for (int t2 = 0; t2 < NST - 1; ++t2)
+            if (t2 < KT) issue((kt_base + t2) * BK, gsm + t2 * STAGE, gsm + t2 * STAGE + A_EL);
+        for (int kt = 0; kt < per; ++kt) {
+            // this wave's loads of tile kt are in LDS once at most the loads of
+            // the younger tiles in flight remain (loads complete in order)
+            wait_vmcnt(LPT * max(0, min(NST - 2, KT - 1 - kt)));
+            __syncthreads();  // everyone's; the stage of tile kt-1 is free again
+            if (kt + NST - 1 < KT) {
+                f16* nxt = gsm + ((kt + NST - 1) % NST) * STAGE;
+                issue((kt_base + kt + NST - 1) * BK, nxt, nxt + A_EL);
+            }
+            if (kt >= KT) continue;
+            const f16* cur = gsm + (kt % NST) * STAGE;
+            compute(cur, cur + A_EL);
+        }
     }
 
     if constexpr (KG > 1) {
@@ -481,29 +375,22 @@ __global__ __launch_bounds__(64 * NWV * KG, 1) void gemm_mfma(GemmArgs p, int ti
         const int r = q / CPR, cc = (q % CPR) * 8;
         const int row = m0 + wm0 + r, col = n0 + wn0 + cc;
         const u32x4 v = *reinterpret_cast<const u32x4*>(ot + r * OUT_LD + cc);
+        if constexpr (RAG) {
+            if (row >= M || col >= N) continue;
+            f16* dst = Cp + (int64_t)row * N + col;
+            if (col + 8 <= N) {
+                __builtin_memcpy(dst, &v, 16);
+            } else {
+                const half8 h = as_half8(v);
+#pragma unroll
+                for (int e = 0; e < 7; ++e)
+                    if (col + e < N) dst[e] = h[e];
+            }
+            continue;
+        }
         // nontemporal: C is written once (QKV shape 0.785 -> 0.763 ms)
         if (row < M && col < N) __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(Cp + (int64_t)row * N + col));
     }
-}
-
-// ---- any-alignment fallback: one thread per C element, fp32 FMA ------------
-__global__ __launch_bounds__(256) void gemm_scalar(GemmArgs p, int ta, int tb) {
-    const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int bz = blockIdx.y;
-    if (idx >= (int64_t)p.M * p.N) return;
-    const int r = (int)(idx / p.N), c = (int)(idx % p.N);
-    const f16* A = p.A + (int64_t)bz * p.sA;
-    const f16* B = p.B + (int64_t)bz * p.sB;
-    f16* Cp = p.C + (int64_t)bz * p.sC;
-    float s = 0.0f;
-    for (int k = 0; k < p.K; ++k) {
-        float a = (float)(ta ? A[(int64_t)k * p.M + r] : A[(int64_t)r * p.K + k]);
-        float b = (float)(tb ? B[(int64_t)c * p.K + k] : B[(int64_t)k * p.N + c]);
-        s += a * b;
-    }
-    f16* dst = Cp + (int64_t)r * p.N + c;
-    if (p.acc) s += (float)*dst;
-    *dst = (f16)s;
 }
 
 // ---- skinny GEMV: C(M,N) = A(M,K) B(K,N), M <= 16, B row-major -------------
@@ -804,7 +691,7 @@ __global__ __launch_bounds__(256) void gemv_mf(GemmArgs p, float* __restrict__ p
 
 
 
-template <int BM, int BN, bool TA, bool TB>
+template <int BM, int BN, bool TA, bool TB, bool RAG>
 hipError_t launch_mfma(const GemmArgs& a, int batch, hipStream_t st) {
     const int tm = (a.M + BM - 1) / BM, tn = (a.N + BN - 1) / BN;
     dim3 grid((unsigned)(tm * tn), 1, batch);
@@ -813,40 +700,21 @@ hipError_t launch_mfma(const GemmArgs& a, int batch, hipStream_t st) {
         // at most one tile per CU and a long K: four K groups per workgroup
         // (16 waves), so that four shorter load/compute chains overlap
         if ((int64_t)tm * tn * batch <= device_cu_count() && a.K >= 16 * MB_K) {
-            hipLaunchKernelGGL((gemm_mfma<BM, BN, TA, TB, NWV, 4>), grid, dim3(64 * NWV * 4), 0, st, a, tm, tn);
+            hipLaunchKernelGGL((gemm_mfma<BM, BN, TA, TB, NWV, 4, RAG>), grid, dim3(64 * NWV * 4), 0, st, a, tm, tn);
             return hipGetLastError();
         }
     }
-    hipLaunchKernelGGL((gemm_mfma<BM, BN, TA, TB, NWV>), grid, dim3(64 * NWV), 0, st, a, tm, tn);
+    hipLaunchKernelGGL((gemm_mfma<BM, BN, TA, TB, NWV, 1, RAG>), grid, dim3(64 * NWV), 0, st, a, tm, tn);
     return hipGetLastError();
 }
 
-template <int BM, int BN>
+template <int BM, int BN, bool RAG>
 hipError_t launch_mfma_t(const GemmArgs& a, int batch, bool ta, bool tb, hipStream_t st) {
-    if (!ta && !tb) return launch_mfma<BM, BN, false, false>(a, batch, st);
-    if (!ta && tb) return launch_mfma<BM, BN, false, true>(a, batch, st);
-    if (ta && !tb) return launch_mfma<BM, BN, true, false>(a, batch, st);
-    return launch_mfma<BM, BN, true, true>(a, batch, st);
+    if (!ta && !tb) return launch_mfma<BM, BN, false, false, RAG>(a, batch, st);
+    if (!ta && tb) return launch_mfma<BM, BN, false, true, RAG>(a, batch, st);
+    if (ta && !tb) return launch_mfma<BM, BN, true, false, RAG>(a, batch, st);
+    return launch_mfma<BM, BN, true, true, RAG>(a, batch, st);
 }
-
-template <class Cfg, bool TA, bool TB>
-hipError_t launch_tiled(const GemmArgs& a, int batch, hipStream_t st) {
-    dim3 grid((a.N + Cfg::BN - 1) / Cfg::BN, (a.M + Cfg::BM - 1) / Cfg::BM, batch);
-    hipLaunchKernelGGL((gemm_tiled<Cfg, TA, TB>), grid, dim3(Cfg::NT), 0, st, a);
-    return hipGetLastError();
-}
-
-template <class Cfg>
-hipError_t launch_tiled_t(const GemmArgs& a, int batch, bool ta, bool tb, hipStream_t st) {
-    if (!ta && !tb) return launch_tiled<Cfg, false, false>(a, batch, st);
-    if (!ta && tb) return launch_tiled<Cfg, false, true>(a, batch, st);
-    if (ta && !tb) return launch_tiled<Cfg, true, false>(a, batch, st);
-    return launch_tiled<Cfg, true, true>(a, batch, st);
-}
-
-using CfgL = TileCfg<256, 256, 64, 2, 2>;  // 4 waves of 128x128
-using CfgM = TileCfg<128, 128, 64, 2, 2>;  // 4 waves of 64x64
-using CfgS = TileCfg<64, 64, 64, 2, 2>;    // 4 waves of 32x32
 
 // Library workspace for the split-K GEMV (grow-only): partials, and the
 // per-column-block arrival counters in an allocation of their own (zeroed
@@ -922,13 +790,7 @@ int gemm_dispatch(const GemmArgs& a, int batch, bool ta, bool tb, bool vec_ok, h
                   const GemvScratch* fixed) {
     if (a.M == 0 || a.N == 0) return EVKHIP_OK;
     hipError_t e;
-    if (!vec_ok) {
-        dim3 grid((unsigned)(((int64_t)a.M * a.N + 255) / 256), batch);
-        hipLaunchKernelGGL(gemm_scalar, grid, dim3(256), 0, st, a, (int)ta, (int)tb);
-        e = hipGetLastError();
-        return e == hipSuccess ? EVKHIP_OK : check_hip(e, "gemm_scalar launch");
-    }
-    if (a.M <= 16 && !ta && !tb && a.K > 0 && (int64_t)a.K * a.N * 2 < INT32_MAX &&
+    if (vec_ok && a.M <= 16 && !ta && !tb && a.K > 0 && (int64_t)a.K * a.N * 2 < INT32_MAX &&
         (int64_t)a.M * a.K * 2 < INT32_MAX) {
         const int ncb = (a.N + SK_CB - 1) / SK_CB;
         const int nks = (a.K + SK_KC - 1) / SK_KC;
@@ -968,19 +830,25 @@ int gemm_dispatch(const GemmArgs& a, int batch, bool ta, bool tb, bool vec_ok, h
     auto tiles = [&](int bm, int bn) {
         return (int64_t)((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn) * batch;
     };
-    // the MFMA kernel addresses each operand through a buffer descriptor
-    const bool fits = (int64_t)a.M * a.K * 2 < INT32_MAX && (int64_t)a.K * a.N * 2 < INT32_MAX &&
-                      (int64_t)a.M * a.N < INT32_MAX;
-    if (fits) {
-        if (tiles(256, 256) >= cus) e = launch_mfma_t<256, 256>(a, batch, ta, tb, st);
-        else if (tiles(128, 128) >= cus / 2) e = launch_mfma_t<128, 128>(a, batch, ta, tb, st);
-        else e = launch_mfma_t<64, 64>(a, batch, ta, tb, st);
-    } else if (tiles(256, 256) >= cus) {
-        e = launch_tiled_t<CfgL>(a, batch, ta, tb, st);
+    // The LDS-direct loads address each operand through a buffer descriptor
+    // and take whole, aligned 16-byte chunks; every other operand (odd row
+    // lengths, pointers off a 16-byte boundary, 2 GiB and more) goes through
+    // registers, in 128- or 64-wide tiles: with 256 the staging registers no
+    // longer fit beside the accumulators.  Against the kernels that served
+    // such calls before, one thread per element (odd rows) and a tiled one
+    // with register transposes (2 GiB): 1000 x 1001 x 777 336 -> 18.2 us,
+    // 3000 x 1501 x 801 1116 -> 53 us, 51 x 50 x 1481 179 -> 13.7 us;
+    // 131136 x 256 x 8192 1240 -> 1222 us, A stored (K,M) 1425 -> 1176 us.
+    const bool direct = vec_ok && (int64_t)a.M * a.K * 2 < INT32_MAX && (int64_t)a.K * a.N * 2 < INT32_MAX &&
+                        (int64_t)a.M * a.N < INT32_MAX;
+    if (direct) {
+        if (tiles(256, 256) >= cus) e = launch_mfma_t<256, 256, false>(a, batch, ta, tb, st);
+        else if (tiles(128, 128) >= cus / 2) e = launch_mfma_t<128, 128, false>(a, batch, ta, tb, st);
+        else e = launch_mfma_t<64, 64, false>(a, batch, ta, tb, st);
     } else if (tiles(128, 128) >= cus / 2) {
-        e = launch_tiled_t<CfgM>(a, batch, ta, tb, st);
+        e = launch_mfma_t<128, 128, true>(a, batch, ta, tb, st);
     } else {
-        e = launch_tiled_t<CfgS>(a, batch, ta, tb, st);
+        e = launch_mfma_t<64, 64, true>(a, batch, ta, tb, st);
     }
     return e == hipSuccess ? EVKHIP_OK : check_hip(e, "gemm launch");
 }

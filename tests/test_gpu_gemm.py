@@ -234,3 +234,47 @@ def test_operand_over_2gib_takes_tiled_path(dev, orc, ta):
     assert np.abs(got_cs - want_cs).max() <= 2e-3 * np.abs(want_cs).max() + 1.0
     del A, B, C
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)])
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (65, 63, 64), (64, 66, 129), (130, 71, 1031), (1000, 1001, 77), (9, 3000, 515)])
+def test_any_row_length(dev, orc, ta, tb, M, N, K):
+    """Row lengths that are no multiple of a 16-byte chunk, in every operand
+    order: tile edges, a K tail of one element, grids of one and of many
+    tiles, the four-group K split (K >= 1024)."""
+    import evk_amd as evk
+    a = orc.uniform_f16((K, M) if ta else (M, K), 91 + M)
+    b = orc.uniform_f16((N, K) if tb else (K, N), 92 + N)
+    got = run_mm(evk, dev, a, b, (M, N), ta, tb)
+    assert_close_f16(got, orc.matmul(a, b, transpose_a=ta, transpose_b=tb), what=f"{ta}{tb} {M}x{N}x{K}")
+
+
+@pytest.mark.parametrize("shift", [(1, 0, 0), (0, 3, 0), (0, 0, 5), (7, 1, 2)])
+def test_two_byte_aligned_operands(dev, orc, shift):
+    """Operands that start off a 16-byte boundary (batched, accumulating, so
+    each batch starts elsewhere), guarded by sentinels around C."""
+    import torch
+    import evk_amd as evk
+    B, M, N, K = 3, 70, 88, 72
+    a, b, c0 = orc.uniform_f16((B, M, K), 95), orc.uniform_f16((K, N), 96), orc.uniform_f16((B, M, N), 97)
+
+    def at(x, off):
+        buf = torch.full((x.size + 16,), 7.0, dtype=torch.float16, device=dev)
+        buf[off:off + x.size] = to_dev(x, dev).reshape(-1)
+        return buf, buf[off:off + x.size].view(x.shape)
+
+    (_, A), (_, W), (buf, C) = at(a, shift[0]), at(b, shift[1]), at(c0, shift[2])
+    evk.matmul(A, W, C, acc_c=True)
+    torch.cuda.synchronize()
+    assert_close_f16(from_dev(C), orc.matmul(a, b, c=c0, acc_c=True), what=f"shift {shift}")
+    assert bool((buf[:shift[2]] == 7).all()) and bool((buf[shift[2] + c0.size:] == 7).all())
+
+
+@pytest.mark.parametrize("K", [1, 63, 2741])
+def test_weight_gradient_of_ragged_token_count(dev, orc, K):
+    """X^T dY over K tokens: K is the row count of both operands and needs no
+    multiple; the rows past K must not enter the sums (LDS-direct loads)."""
+    import evk_amd as evk
+    a, b, c0 = orc.uniform_f16((K, 136), 98), orc.uniform_f16((K, 264), 99), orc.uniform_f16((136, 264), 100)
+    got = run_mm(evk, dev, a, b, None, True, False, True, c0)
+    assert_close_f16(got, orc.matmul(a, b, c=c0, transpose_a=True, acc_c=True), what=f"K={K}")
