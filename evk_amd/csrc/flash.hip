@@ -860,7 +860,7 @@ __global__ __launch_bounds__(512, 1) void flash_fwd_ks(FlashArgs p) {
 }
 
 // ---------------------------------------------------------------------------
-// Backward dK, dV for head dims 32 and 64.
+// Backward dK, dV for head dims 32, 64 and 128.
 //
 // Workgroup: 4 waves and 128 keys; wave w owns keys [32w, 32w+32) of the
 // block, with K^T and V^T as B-operand registers for the whole kernel.  The
@@ -973,11 +973,12 @@ DEV void bwd_kv_body(const FlashArgs& p, float* part_ws, int parts_per_batch, in
     const __amdgpu_buffer_rsrc_t gres = buf_rsrc(p.dO + (int64_t)b * NH * DH, (uint32_t)NH * DH * 2);
     const __amdgpu_buffer_rsrc_t ores = buf_rsrc(p.o + (int64_t)b * NH * DH, (uint32_t)NH * DH * 2);
     const __amdgpu_buffer_rsrc_t lres = buf_rsrc(p.lse + (int64_t)b * H * N, (uint32_t)(H * N) * 4u);
-    // A thread holds at most one dO piece (DH <= 64); with it the O piece at
-    // the same place, so that D = rowsum(dO * O) comes from the DH/8 lanes
-    // of a row.  Rows past NH read as zeros: D = 0, lse2 = 0 (their Q and
-    // dO rows are zero too, so they add nothing).
-    u32x4 pr[PPT], po = {0u, 0u, 0u, 0u};
+    // With each dO piece a thread holds the O piece at the same place, so
+    // that D = rowsum(dO * O) comes from the DH/8 lanes of a row.  Rows past
+    // NH read as zeros: D = 0, lse2 = 0 (their Q and dO rows are zero too, so
+    // they add nothing).
+    constexpr int OPT = PIECES >= 256 ? PIECES / 256 : 1;  // dO pieces per thread
+    u32x4 pr[PPT], po[OPT] = {};
     float sr = 0.0f;
     int spos = 0;
     // Row (position, head) of thread t's statistics row (t mod BRC), advanced
@@ -1008,7 +1009,7 @@ DEV void bwd_kv_body(const FlashArgs& p, float* part_ws, int parts_per_batch, in
             if (2 * PIECES % 256 == 0 || pc < 2 * PIECES) {
                 if (which) {
                     pr[i] = buf_load16(gres, off, 0);
-                    po = buf_load16(ores, off, 0);
+                    po[i % OPT] = buf_load16(ores, off, 0);
                 } else {
                     pr[i] = buf_load16(qres, off, 0);
                 }
@@ -1031,29 +1032,36 @@ DEV void bwd_kv_body(const FlashArgs& p, float* part_ws, int parts_per_batch, in
     };
     auto lstore = [&](int stage) {
         f16* cs = chunk_s + stage * L::STAGE;
-        float dsum = 0.0f;
+        float dsum[OPT] = {};
 #pragma unroll
         for (int i = 0; i < PPT; ++i) {
             const int pc = threadIdx.x + 256 * i;
             const int which = __builtin_amdgcn_readfirstlane(pc / PIECES), pi = pc % PIECES;
             if (2 * PIECES % 256 == 0 || pc < 2 * PIECES) {
                 *reinterpret_cast<u32x4*>(cs + which * L::CHUNK + (pi / (DH / 8)) * RW + (pi % (DH / 8)) * 8) = pr[i];
-                if (which) dsum = dot8(as_half8(pr[i]), as_half8(po));
+                if (which) dsum[i % OPT] = dot8(as_half8(pr[i]), as_half8(po[i % OPT]));
             }
         }
-        // the DH/8 lanes of a row are adjacent (a quad or two): DPP sums
-        dsum += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, dsum), 0xB1, 0xF, 0xF, false));
-        if (DH / 8 >= 4)
-            dsum += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, dsum), 0x4E, 0xF, 0xF, false));
-        if (DH / 8 >= 8)
-            dsum += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, dsum), 0x141, 0xF, 0xF, false));
-        static_assert(DH / 8 <= 8, "a row's lanes within a half row");
+        // the DH/8 lanes of a row are adjacent (a quad, a half row or a row of
+        // 16 lanes): DPP sums
+        auto dpp_add = [](float& v, auto ctrl) {
+            v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), decltype(ctrl)::value,
+                                                                       0xF, 0xF, false));
+        };
+        static_assert(DH / 8 <= 16, "a row's lanes within 16 lanes");
+#pragma unroll
+        for (int o = 0; o < OPT; ++o) {
+            dpp_add(dsum[o], std::integral_constant<int, 0xB1>{});
+            if (DH / 8 >= 4) dpp_add(dsum[o], std::integral_constant<int, 0x4E>{});
+            if (DH / 8 >= 8) dpp_add(dsum[o], std::integral_constant<int, 0x141>{});
+            if (DH / 8 >= 16) dpp_add(dsum[o], std::integral_constant<int, 0x140>{});
+        }
 #pragma unroll
         for (int i = 0; i < PPT; ++i) {
             const int pc = threadIdx.x + 256 * i;
             const int pi = pc % PIECES;
             if (pc >= PIECES && pc < 2 * PIECES && pi % (DH / 8) == 0)
-                stats_s[stage * L::STATS + BRC + pi / (DH / 8)] = dsum;
+                stats_s[stage * L::STATS + BRC + pi / (DH / 8)] = dsum[i % OPT];
         }
         const float l2 = sr * kLog2e;  // base-2 LSE
         if (threadIdx.x < BRC) stats_s[stage * L::STATS + threadIdx.x] = l2;
@@ -1238,7 +1246,7 @@ __global__ __launch_bounds__(256) void flash_bwd_kv_reduce(FlashArgs p, const fl
 }
 
 // ---------------------------------------------------------------------------
-// Backward dQ for head dims 32 and 64: the key-split forward's structure
+// Backward dQ for head dims 32, 64 and 128: the key-split forward's structure
 // without the online softmax (P comes from the saved row statistics).
 // Workgroup: 64 flattened query rows, 4 waves; wave w takes 32-key chunks
 // w, w+4, ... for all 64 rows:
@@ -1429,8 +1437,16 @@ DEV void bwd_q_body(const FlashArgs& p, int blk, char* lds) {
 // the latter, heavy row tiles first.  The two halves are independent (both
 // read only Q, K, V, dO and the row statistics), so the dQ tiles fill the
 // CUs that the short dK/dV parts free.
+// DH = 128 runs one wave per SIMD (450 registers: both bodies hold 128
+// accumulators and as many operand values).  It is a latency chain, about
+// 1.9 us per 32-row chunk of a dK/dV part, but its parts fill the chip where
+// one workgroup per 32 keys (the kernels below) leaves most CUs idle: with
+// the forward, B=2 N=2000 H=8 causal 834 -> 203 us, B=1 N=1740 H=12 1035 ->
+// 125 us, B=1 N=130 H=2 40.5 -> 32.7 us.  Longer parts halve the fp32
+// partials but not the chain: parts of 32 chunks 201, 116 and (B=1 N=600
+// H=4) 85.6 us against 203, 125 and 54.9 us with 16.
 template <int DH, bool CAUSAL>
-__global__ __launch_bounds__(256, 2) void flash_bwd_kvq(FlashArgs p, float* part_ws, int parts_per_batch, int n_kv) {
+__global__ __launch_bounds__(256, DH <= 64 ? 2 : 1) void flash_bwd_kvq(FlashArgs p, float* part_ws, int parts_per_batch, int n_kv) {
     constexpr int KVB = KvLayout<DH>::LDS_BYTES, QB = DqLayout<DH>::LDS_BYTES;
     __shared__ __attribute__((aligned(16))) char lds[KVB > QB ? KVB : QB];
     if ((int)blockIdx.x < n_kv) {
@@ -1914,7 +1930,7 @@ hipError_t launch_bwd(const FlashArgs& a, bool causal, bool have_lse, hipStream_
     return hipGetLastError();
 }
 
-// dK/dV by key blocks and row parts, then dQ by row tiles (head dims 32, 64).
+// dK/dV by key blocks and row parts, then dQ by row tiles (head dims 32, 64, 128).
 template <int DH>
 hipError_t launch_bwd_split(const FlashArgs& a, bool causal, float* parts, int parts_per_batch,
                             hipStream_t st) {
@@ -1981,7 +1997,7 @@ int flash_backward(FlashArgs a, int dh, bool mfma, bool causal, hipStream_t st) 
     a.scale_log2 = a.scale * kLog2e;
     const size_t rows = (size_t)a.B * a.N * a.H;
     const bool have_lse = a.lse != nullptr;
-    const bool split = mfma && dh <= 64 && !flash_wide_head(dh) && (int64_t)a.N * a.H * dh * 2 < (int64_t)INT32_MAX;
+    const bool split = mfma && dh <= 128 && !flash_wide_head(dh) && (int64_t)a.N * a.H * dh * 2 < (int64_t)INT32_MAX;
     const bool wide = mfma && flash_wide_head(dh) && flash_wide_fits(a.N, a.H, dh);
     // arena layout (256-byte aligned pieces)
     auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
@@ -2012,13 +2028,16 @@ int flash_backward(FlashArgs a, int dh, bool mfma, bool causal, hipStream_t st) 
             float* l_ws = reinterpret_cast<float*>(g_bwd_ws + stats_b + part_b + al(rows * dh * 2));
             f.out = o_ws;
             f.lse = l_ws;
-            e = (dh == 32) ? launch_fwd<32>(f, causal, 0, st) : launch_fwd<64>(f, causal, 0, st);
+            e = (dh == 32)   ? launch_fwd<32>(f, causal, 0, st)
+                : (dh == 64) ? launch_fwd<64>(f, causal, 0, st)
+                             : launch_fwd<128>(f, causal, 0, st);
             if (e != hipSuccess) return check_hip(e, "flash backward: forward recompute");
             a.o = o_ws;
             a.lse = l_ws;
         }
-        e = (dh == 32) ? launch_bwd_split<32>(a, causal, parts, parts_per_batch, st)
-                       : launch_bwd_split<64>(a, causal, parts, parts_per_batch, st);
+        e = (dh == 32)   ? launch_bwd_split<32>(a, causal, parts, parts_per_batch, st)
+            : (dh == 64) ? launch_bwd_split<64>(a, causal, parts, parts_per_batch, st)
+                         : launch_bwd_split<128>(a, causal, parts, parts_per_batch, st);
     } else if (wide) {
         if (!have_lse) {
             // recompute the forward's O and LSE into the arena

@@ -143,6 +143,28 @@ def test_flash_backward_dh32_split_parts(dev, orc, causal):
     assert_close_f16(dv, wv, what=f"dV dh32 causal={causal}")
 
 
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("use_lse", [True, False])
+@pytest.mark.parametrize("B,N,H", [(2, 300, 8), (1, 127, 4), (1, 129, 5), (8, 64, 8)])
+def test_flash_backward_dh128(dev, orc, B, N, H, causal, use_lse):
+    """Head size 128 at the edges of its tiles: several row parts per key
+    block, one key short of and one key past a 128-key block, heads that do
+    not divide the 32-row chunks, one part (written without partials)."""
+    import evk_amd as evk
+    import torch
+    Dh = 128
+    q, g = orc.normal_f16((B, N, H * Dh), 281 + N), orc.normal_f16((B, N, H * Dh), 284 + N)
+    k, v = orc.normal_f16((B, N, Dh), 282 + N), orc.normal_f16((B, N, Dh), 283 + N)
+    Q, K, V, G = (to_dev(x, dev) for x in (q, k, v, g))
+    O, L = torch.empty_like(Q), torch.empty((B, H, N), dtype=torch.float32, device=dev)
+    evk.flash_attention(Q, K, V, O, causal=causal, lse=L)
+    dQ, dK, dV = torch.empty_like(Q), torch.empty_like(K), torch.empty_like(V)
+    evk.flash_attention_bwd(Q, K, V, O, G, dQ, dK, dV, causal=causal, lse=L if use_lse else None)
+    torch.cuda.synchronize()
+    for got, want, what in zip((dQ, dK, dV), orc.attention_bwd(q, k, v, g, causal), ("dQ", "dK", "dV")):
+        assert_close_f16(from_dev(got), want, what=f"{what} B={B} N={N} H={H}")
+
+
 @pytest.mark.parametrize("Dh", [32, 64, 128, 16, 48, 96, 256])
 @pytest.mark.parametrize("N", [16, 45, 96])
 def test_flash_backward_ragged(dev, orc, Dh, N):
