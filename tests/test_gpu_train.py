@@ -220,3 +220,19 @@ def test_empty_inputs(dev):
     evk.sgd(e, e, 0.1)
     evk.sum_batch(e, e, 3, 0)
     sync()
+
+
+@pytest.mark.parametrize("n,dim,vocab,distinct", [(1, 1, 2, 1), (2048, 6, 50, 3), (2049, 513, 300, 40), (5000, 2, 9, 1),
+                                                 (66000, 3, 70, 200)])
+def test_embed_backward_order(dev, orc, n, dim, vocab, distinct):
+    """Every addition rounded to fp16, in row order, bit for bit: ids that
+    repeat within and across the 2048-row chunks, one id everywhere, ids past
+    the vocabulary, odd dimensions, more rows than the grid is high."""
+    import torch
+    import evk_amd as evk
+    idx = (orc.tokens_u16(n, 701 + n, 65536).astype(np.uint32) % distinct).astype(np.uint16)
+    g, base = orc.normal_f16((n, dim), 702 + n), orc.normal_f16((vocab, dim), 703 + n)
+    GE = to_dev(base, dev)
+    evk.embed_backward(to_dev(g, dev), torch.from_numpy(idx.view(np.int16)).to(dev), GE)
+    torch.cuda.synchronize()
+    assert np.array_equal(from_dev(GE), orc.embed_backward(g, idx, base))
