@@ -187,6 +187,29 @@ DEV float gelu_f(float x) {
     return 0.5f * x * (1.0f + tanhf(u));
 }
 
+// tanh on the hardware exponential and reciprocal: 1 - 2 / (e^(2|u|) + 1) with
+// u's sign, about 1e-7 absolute everywhere (what 1 + tanh u needs: it takes
+// the same rounding as with tanhf next to -1).  For whole tensors, where
+// tanhf's branches and polynomial take longer than the memory accesses; the
+// decode kernels keep gelu_f.
+DEV float tanh_fast(float u) {
+    constexpr float k2Log2e = 2.0f * 1.4426950408889634f;
+    const float r = 2.0f * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(k2Log2e * fabsf(u)) + 1.0f);
+    return copysignf(1.0f - r, u);
+}
+DEV float gelu_fast(float x) {
+    const float ka = 0.7978845608028654f, kb = 0.044715f;
+    return 0.5f * x * (1.0f + tanh_fast(ka * (x + kb * x * x * x)));
+}
+
+// 16-byte accesses at any fp16 address
+DEV half8 ld_h8(const f16* p) {
+    half8 v;
+    __builtin_memcpy(&v, p, 16);
+    return v;
+}
+DEV void st_h8(f16* p, const half8& v) { __builtin_memcpy(p, &v, 16); }
+
 // greedy_sample.comp's winner is the maximum under the total order
 // (value desc, bitrev8(j mod 256) asc, j asc); rank encodes the last two.
 DEV uint32_t greedy_rank(uint32_t j) {

@@ -222,8 +222,48 @@ __global__ __launch_bounds__(256) void kv_write_k(const f16* src, f16* cache, in
 }
 
 // ---------------------------------------------------------------------------
-// rms_norm: one wave per row, 4 rows per workgroup.
+// rms_norm: one wave per row, 4 rows per workgroup.  Rows of D <= 512 * NV
+// whose length is a multiple of 8 stay in registers (16-byte accesses at any
+// alignment, one read and one write of each value); longer or odd rows are
+// walked element by element, twice.  Launch-bound at 1000 rows of 768: 3.4 us
+// (walked, 2-byte accesses: 7.7).
 // ---------------------------------------------------------------------------
+DEV float clamp_f16(float v) { return fminf(fmaxf(v, -65504.0f), 65504.0f); }
+
+template <int NV>
+__global__ __launch_bounds__(256) void rms_norm_reg_k(const f16* in, f16* out, int64_t rows, int D, float eps) {
+    const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    if (row >= rows) return;
+    const f16* x = in + row * D;
+    half8 r[NV];
+#pragma unroll
+    for (int u = 0; u < NV; ++u) {
+        const int c = (lane + 64 * u) * 8;
+        r[u] = half8{};
+        if (c < D) r[u] = ld_h8(x + c);
+    }
+    float ss = 0.0f;
+#pragma unroll
+    for (int u = 0; u < NV; ++u)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const float v = clamp_f16((float)r[u][e]);
+            ss += v * v;
+        }
+    ss = wave_sum(ss);
+    const float inv = 1.0f / sqrtf(ss / (float)D + eps);
+#pragma unroll
+    for (int u = 0; u < NV; ++u) {
+        const int c = (lane + 64 * u) * 8;
+        if (c >= D) continue;
+        half8 o;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = (f16)(clamp_f16((float)r[u][e]) * inv);
+        st_h8(out + row * D + c, o);
+    }
+}
+
 __global__ __launch_bounds__(256) void rms_norm_k(const f16* in, f16* out, int64_t rows, int D, float eps) {
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
@@ -231,15 +271,12 @@ __global__ __launch_bounds__(256) void rms_norm_k(const f16* in, f16* out, int64
     const f16* x = in + row * D;
     float ss = 0.0f;
     for (int j = lane; j < D; j += 64) {
-        float v = fminf(fmaxf((float)x[j], -65504.0f), 65504.0f);
+        const float v = clamp_f16((float)x[j]);
         ss += v * v;
     }
     ss = wave_sum(ss);
     const float inv = 1.0f / sqrtf(ss / (float)D + eps);
-    for (int j = lane; j < D; j += 64) {
-        float v = fminf(fmaxf((float)x[j], -65504.0f), 65504.0f);
-        out[row * D + j] = (f16)(v * inv);
-    }
+    for (int j = lane; j < D; j += 64) out[row * D + j] = (f16)(clamp_f16((float)x[j]) * inv);
 }
 
 // rope: one thread per rotated pair.
@@ -263,24 +300,57 @@ __global__ __launch_bounds__(256) void rope_k(const f16* in, f16* out, int B, in
 }
 
 
+// Elementwise: 8 consecutive values per thread in 16-byte accesses (at any
+// alignment), the last thread value by value.  Memory-bound: gelu over 2560 x
+// 3072 7.7 us = 4.1 TB/s (19.2 us with one value per thread and tanhf).
+template <class F>
+DEV void each8(int64_t n, F&& f) {
+    const int64_t i0 = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8;
+    if (i0 < n) f(i0, n - i0 < 8 ? (int)(n - i0) : 8);
+}
+DEV half8 ld_n(const f16* p, int n) {
+    if (n == 8) return ld_h8(p);
+    half8 v = {};
+#pragma unroll
+    for (int e = 0; e < 7; ++e)
+        if (e < n) v[e] = p[e];
+    return v;
+}
+DEV void st_n(f16* p, const half8& v, int n) {
+    if (n == 8) return st_h8(p, v);
+#pragma unroll
+    for (int e = 0; e < 7; ++e)
+        if (e < n) p[e] = v[e];
+}
+
 __global__ __launch_bounds__(256) void gelu_k(const f16* in, f16* out, int64_t n) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) out[i] = (f16)gelu_f((float)in[i]);
+    each8(n, [&](int64_t i, int k) {
+        half8 v = ld_n(in + i, k);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = (f16)gelu_fast((float)v[e]);
+        st_n(out + i, v, k);
+    });
 }
 
 __global__ __launch_bounds__(256) void add_k(const f16* a, const f16* b, f16* c, int64_t n) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) c[i] = (f16)((float)a[i] + (float)b[i]);
+    each8(n, [&](int64_t i, int k) {
+        const half8 x = ld_n(a + i, k), y = ld_n(b + i, k);
+        half8 v;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = (f16)((float)x[e] + (float)y[e]);
+        st_n(c + i, v, k);
+    });
 }
 
+// One thread per 8 values of a row (dim / 8 rounded up pieces a row).
 __global__ __launch_bounds__(256) void embed_k(const f16* table, const uint16_t* idx, f16* out, int64_t n_idx,
-                                                int dim, int vocab) {
+                                                int dim, int pieces, int vocab) {
     const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (gid >= n_idx * dim) return;
-    const int64_t i = gid / dim;
-    const int d = (int)(gid % dim);
+    if (gid >= n_idx * pieces) return;
+    const int64_t i = gid / pieces;
+    const int d = (int)(gid % pieces) * 8, k = min(8, dim - d);
     const int tok = min((int)idx[i], vocab - 1);
-    out[gid] = table[(int64_t)tok * dim + d];
+    st_n(out + i * dim + d, ld_n(table + (int64_t)tok * dim + d, k), k);
 }
 
 // ---------------------------------------------------------------------------
@@ -290,18 +360,38 @@ __global__ __launch_bounds__(256) void embed_k(const f16* table, const uint16_t*
 // token_base.  Any reduction tree over this order gives the same winner.
 // ---------------------------------------------------------------------------
 
-__global__ __launch_bounds__(256) void greedy_k(const f16* logits, uint16_t* out, int S, int V, int position,
-                                                 int token_base, int token_count) {
-    __shared__ float s_v[4];
-    __shared__ uint32_t s_r[4];
+// One workgroup per sequence; a thread requests GR_LD 16-byte pieces of the
+// row before it looks at any (the row may start at any fp16 address): 32000
+// logits 39.7 -> 6.1 us against 2-byte loads by 256 threads.
+constexpr int GR_NT = 1024, GR_LD = 4;
+
+__global__ __launch_bounds__(GR_NT) void greedy_k(const f16* logits, uint16_t* out, int S, int V, int position,
+                                                   int token_base, int token_count) {
+    __shared__ float s_v[GR_NT / 64];
+    __shared__ uint32_t s_r[GR_NT / 64];
     const int b = blockIdx.x, tid = threadIdx.x;
     const f16* row = logits + ((int64_t)b * S + position) * V + token_base;
     float bv = -3.402823466e+38f;
     uint32_t br = 0u;  // rank of j = 0 (token_base)
-    for (int j = tid; j < token_count; j += 256) {
-        float v = (float)row[j];
-        uint32_t r = greedy_rank((uint32_t)j);
-        if (v > -3.402823466e+38f && greedy_better(v, r, bv, br)) { bv = v; br = r; }
+    for (int j0 = tid * 8; j0 < token_count; j0 += GR_NT * 8 * GR_LD) {
+        half8 v[GR_LD];
+#pragma unroll
+        for (int u = 0; u < GR_LD; ++u) {
+            const int j = j0 + u * GR_NT * 8;
+            v[u] = ld_n(row + j, max(0, min(8, token_count - j)));
+        }
+#pragma unroll
+        for (int u = 0; u < GR_LD; ++u)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int j = j0 + u * GR_NT * 8 + e;
+                const float x = (float)v[u][e];
+                const uint32_t r = greedy_rank((uint32_t)j);
+                if (j < token_count && x > -3.402823466e+38f && greedy_better(x, r, bv, br)) {
+                    bv = x;
+                    br = r;
+                }
+            }
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
@@ -312,12 +402,9 @@ __global__ __launch_bounds__(256) void greedy_k(const f16* logits, uint16_t* out
     if ((tid & 63) == 0) { s_v[tid >> 6] = bv; s_r[tid >> 6] = br; }
     __syncthreads();
     if (tid == 0) {
-        for (int w = 1; w < 4; ++w)
+        for (int w = 1; w < GR_NT / 64; ++w)
             if (greedy_better(s_v[w], s_r[w], bv, br)) { bv = s_v[w]; br = s_r[w]; }
-        // rank -> j: low 16 bits hold j >> 8, high bits bitrev8(j & 255)
-        uint32_t lo = __builtin_bitreverse32(br >> 16) >> 24;
-        uint32_t j = ((br & 0xFFFFu) << 8) | lo;
-        out[b] = (uint16_t)(token_base + j);
+        out[b] = (uint16_t)(token_base + greedy_index(br));
     }
 }
 
@@ -415,7 +502,12 @@ int kv_cache_write_launch(const f16* src, f16* cache, int batch, int n, int D, i
 
 int rms_norm_launch(const f16* in, f16* out, int64_t rows, int D, float eps, hipStream_t st) {
     if (rows == 0) return EVKHIP_OK;
-    hipLaunchKernelGGL(rms_norm_k, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, st, in, out, rows, D, eps);
+    const dim3 grid((unsigned)((rows + 3) / 4));
+    if (D % 8 || D > 4096) hipLaunchKernelGGL(rms_norm_k, grid, dim3(256), 0, st, in, out, rows, D, eps);
+    else if (D <= 512) hipLaunchKernelGGL(rms_norm_reg_k<1>, grid, dim3(256), 0, st, in, out, rows, D, eps);
+    else if (D <= 1024) hipLaunchKernelGGL(rms_norm_reg_k<2>, grid, dim3(256), 0, st, in, out, rows, D, eps);
+    else if (D <= 2048) hipLaunchKernelGGL(rms_norm_reg_k<4>, grid, dim3(256), 0, st, in, out, rows, D, eps);
+    else hipLaunchKernelGGL(rms_norm_reg_k<8>, grid, dim3(256), 0, st, in, out, rows, D, eps);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? EVKHIP_OK : check_hip(e, "rms_norm launch");
 }
@@ -431,24 +523,24 @@ int rope_launch(const f16* in, f16* out, int B, int S, int E, float base, int po
 
 int gelu_launch(const f16* in, f16* out, int64_t n, hipStream_t st) {
     if (n == 0) return EVKHIP_OK;
-    hipLaunchKernelGGL(gelu_k, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, in, out, n);
+    hipLaunchKernelGGL(gelu_k, dim3((unsigned)((n + 2047) / 2048)), dim3(256), 0, st, in, out, n);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? EVKHIP_OK : check_hip(e, "gelu launch");
 }
 
 int add_launch(const f16* a, const f16* b, f16* c, int64_t n, hipStream_t st) {
     if (n == 0) return EVKHIP_OK;
-    hipLaunchKernelGGL(add_k, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a, b, c, n);
+    hipLaunchKernelGGL(add_k, dim3((unsigned)((n + 2047) / 2048)), dim3(256), 0, st, a, b, c, n);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? EVKHIP_OK : check_hip(e, "add launch");
 }
 
 int embed_launch(const f16* table, const uint16_t* idx, f16* out, int64_t n_idx, int dim, int vocab,
                  hipStream_t st) {
-    int64_t n = n_idx * dim;
-    if (n == 0) return EVKHIP_OK;
-    hipLaunchKernelGGL(embed_k, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, table, idx, out, n_idx, dim,
-                       vocab);
+    if (n_idx == 0 || dim == 0) return EVKHIP_OK;
+    const int pieces = (dim + 7) / 8;
+    hipLaunchKernelGGL(embed_k, dim3((unsigned)((n_idx * pieces + 255) / 256)), dim3(256), 0, st, table, idx, out,
+                       n_idx, dim, pieces, vocab);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? EVKHIP_OK : check_hip(e, "embed launch");
 }
@@ -456,7 +548,7 @@ int embed_launch(const f16* table, const uint16_t* idx, f16* out, int64_t n_idx,
 int greedy_launch(const f16* logits, uint16_t* out, int B, int S, int V, int position, int token_base,
                   int token_count, hipStream_t st) {
     if (B == 0) return EVKHIP_OK;
-    hipLaunchKernelGGL(greedy_k, dim3(B), dim3(256), 0, st, logits, out, S, V, position, token_base, token_count);
+    hipLaunchKernelGGL(greedy_k, dim3(B), dim3(GR_NT), 0, st, logits, out, S, V, position, token_base, token_count);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? EVKHIP_OK : check_hip(e, "greedy_sample launch");
 }

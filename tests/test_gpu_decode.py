@@ -430,3 +430,85 @@ def test_prefill_in_two_parts(dev, orc):
     stop = check_ids([int(from_dev(tok)[0])], [int(want_ids[0])], want_logits)
     if stop is None:
         assert_close_f16(from_dev(cache), want_cache, what="kv cache")
+
+
+def shifted(x, dev, off):
+    """x on the device, `off` fp16 elements past a 16-byte boundary."""
+    import torch
+    buf = torch.zeros(x.size + 8, dtype=torch.float16, device=dev)
+    t = buf[off:off + x.size].view(x.shape)
+    t.copy_(to_dev(x, dev))
+    return t
+
+
+@pytest.mark.parametrize("off", [0, 3])
+@pytest.mark.parametrize("D", [8, 504, 512, 520, 1024, 1032, 2048, 2056, 4096, 4104, 777])
+def test_rms_norm_row_lengths(dev, orc, D, off):
+    """Row lengths at the edges of the register kernels (512 * 1, 2, 4, 8),
+    past them and odd, five rows (one past a workgroup), any alignment."""
+    import evk_amd as evk
+    import torch
+    x = orc.normal_f16((5, D), 320 + D, 0, 2)
+    X, Y = shifted(x, dev, off), shifted(np.zeros_like(x), dev, off)
+    evk.rms_norm(X, Y, 1e-4)
+    torch.cuda.synchronize()
+    assert ulp_close(from_dev(Y), orc.rms_norm(x, 1e-4))
+
+
+@pytest.mark.parametrize("off", [0, 5])
+@pytest.mark.parametrize("n", [1, 7, 8, 9, 2047, 2049])
+def test_elementwise_tails(dev, orc, n, off):
+    """gelu and add at the last, partial 8 values and past a workgroup; the
+    values behind the output stay as they were."""
+    import evk_amd as evk
+    import torch
+    x, y = orc.normal_f16((n,), 330 + n, 0, 3), orc.normal_f16((n,), 331 + n)
+    X, Y = shifted(x, dev, off), shifted(y, dev, off)
+    buf = torch.full((n + 16,), 7.0, dtype=torch.float16, device=dev)
+    O = buf[off:off + n]
+    evk.gelu(X, O)
+    torch.cuda.synchronize()
+    # half an fp16 ulp, and 0.5 x times the 1e-7 that tanh may be off
+    v = f32(x).astype(np.float64)
+    want = v / (1.0 + np.exp(-2.0 * 0.7978845608028654 * (v + 0.044715 * v ** 3)))
+    got = from_dev(O)
+    assert np.all(np.abs(f32(got) - want) <= 2.0 ** -11 * np.abs(want) + 2.0 ** -25 + 1e-7 * np.abs(v))
+    evk.add(X, Y, O)
+    torch.cuda.synchronize()
+    assert np.array_equal(from_dev(O), orc.add(x, y))
+    assert bool((buf[:off] == 7).all()) and bool((buf[off + n:] == 7).all())
+
+
+@pytest.mark.parametrize("dim", [1, 7, 8, 13, 768])
+def test_embed_row_lengths(dev, orc, dim):
+    import evk_amd as evk
+    import torch
+    table = orc.normal_f16((50, dim), 340 + dim)
+    idx = np.array([0, 49, 3, 3, 60, 7, 65535], np.uint16)  # ids past the table take its last row
+    O = torch.empty((len(idx), dim), dtype=torch.float16, device=dev)
+    evk.embed(to_dev(table, dev), torch.from_numpy(idx.view(np.int16)).to(dev), O)
+    torch.cuda.synchronize()
+    assert np.array_equal(from_dev(O), table[np.minimum(idx, 49)])
+
+
+@pytest.mark.parametrize("V,base,count", [(40000, 0, 40000), (40001, 3, 39990), (33000, 1, 32769), (100, 7, 9), (8, 0, 0)])
+def test_greedy_long_rows(dev, orc, V, base, count):
+    """Rows longer than one pass of the workgroup, ranges off a 16-byte
+    boundary and with a partial last piece, ties (few distinct values),
+    infinities and NaN."""
+    import evk_amd as evk
+    logits = (orc.normal_f16((3, 2, V), 350 + V) & np.uint16(0xFC00))
+    logits[1, 1, base:base + count:5] = 0x7E00   # NaN never wins
+    logits[2, 1, :] = 0xFC00                     # -inf everywhere: no candidate
+    got = greedy_dev(evk, dev, logits, 1, base, count)
+    want = []
+    for b in range(3):
+        best, bj = None, 0
+        for j, v in enumerate(f32(logits[b, 1, base:base + count])):
+            if not v > -3.402823466e+38:
+                continue
+            key = (-v, int(f"{j & 255:08b}"[::-1], 2), j)
+            if best is None or key < best:
+                best, bj = key, j
+        want.append(base + bj)
+    assert list(got) == want

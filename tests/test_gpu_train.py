@@ -236,3 +236,25 @@ def test_embed_backward_order(dev, orc, n, dim, vocab, distinct):
     evk.embed_backward(to_dev(g, dev), torch.from_numpy(idx.view(np.int16)).to(dev), GE)
     torch.cuda.synchronize()
     assert np.array_equal(from_dev(GE), orc.embed_backward(g, idx, base))
+
+
+@pytest.mark.parametrize("off", [0, 3])
+@pytest.mark.parametrize("D", [8, 512, 520, 1024, 1032, 2048, 2056, 777])
+def test_rms_norm_backward_row_lengths(dev, orc, D, off):
+    """Row lengths at the edges of the register kernels, past them and odd,
+    five rows (one past a workgroup), any alignment."""
+    import torch
+
+    import evk_amd as evk
+    x, g, a = rnd(91, (5, D)), rnd(92, (5, D)), rnd(93, (5, D))
+
+    def at(v):
+        buf = torch.zeros(v.size + 8, dtype=torch.float16, device=dev)
+        t = buf[off:off + v.size].view(v.shape)
+        t.copy_(to_dev(v, dev))
+        return t
+
+    X, G, A = at(x), at(g), at(a)
+    evk.rms_norm_backward(X, G, A, 1e-4)
+    sync()
+    assert_close_f16(from_dev(A), orc.rms_norm_backward(x, g, a, 1e-4), what=f"rms_norm_backward D={D}")
