@@ -19,13 +19,10 @@ namespace evkhip {
 
 namespace {
 
-// ---- MFMA kernel: BM x BN tiles; 4 waves of (BM/2) x (BN/2), or for 256x256
-// tiles 8 waves of 128 x 64 (two waves per SIMD: one wave's LDS reads and
-// waits overlap the other's MFMAs; measured 2-5 % faster than 4 waves of
-// 128 x 128 at 4096^3 and QKV, while 4 waves of 64 x 128 were slower).
-// 64x64 tiles of a grid that fits the CUs once with a long K run go as four
-// K groups of 4 waves (16 waves), whose fp32 sums are added in group order
-// in LDS, so the result does not depend on timing: 1024^3 8.6 -> 7.1 us ----
+// ---- MFMA kernel: BM x BN tiles; NWV waves of (BM/2) x (BN/(NWV/2)) per K
+// group, KG K groups (each takes a range of the K tiles; their fp32 sums are
+// added in group order in LDS, so the result does not depend on timing) and
+// NST LDS stages; which instance serves a product: kPlans ----
 // v_mfma_f32_16x16x32_f16 (lane l: A row l%16 / B column l%16, k 8(l/16)..+8;
 // D column l%16, rows 4(l/16)..+3).  Each operand tile of BK = 64 along K
 // goes from global memory straight into LDS (buffer_load_dwordx4 ... lds: a
@@ -38,9 +35,9 @@ namespace {
 //     halves, chunk c of row r at slot c ^ 2 (r & 3); fragments by
 //     ds_read_b64_tr_b16 (4 consecutive k of one column per lane).
 // The loads choose their global chunk per lane to realise the permutation;
-// chunks outside the matrix read as zeros (buffer descriptors).  Two LDS
-// stages for 256x256 tiles, four for smaller ones: the loads of the next
-// tiles fly during the MFMAs of tile t; one barrier per tile.  Workgroups are ordered so that the
+// chunks outside the matrix read as zeros (buffer descriptors).  The loads of
+// the next NST - 1 tiles fly during the MFMAs of tile t; one barrier per
+// tile.  Workgroups are ordered so that the
 // ones an XCD runs (workgroup id mod 8) cover a compact block of C tiles and
 // share A/B panels in that XCD's L2.  The epilogue stages each wave's fp16
 // tile in LDS and writes 16-byte row chunks (accumulating calls add C per
@@ -150,34 +147,31 @@ struct RagTile {
     }
 };
 
+// Workgroup w runs on XCD w % 8; each XCD takes a contiguous range of tiles
+// (the first total % 8 XCDs one more than the others).
 DEV int xcd_tile(int w, int total) {
-    if (total % 8) return w;
-    return (w % 8) * (total / 8) + w / 8;  // XCD w%8 gets a contiguous range
+    const int x = w % 8;
+    return x * (total / 8) + min(x, total % 8) + w / 8;
 }
-
-// LDS stages of gemm_mfma: two for 256x256 tiles (128 KB), four for the
-// smaller tiles, whose short K loops need more tiles in flight.
-template <int BM>
-constexpr int mfma_stages() { return BM >= 256 ? 2 : 4; }
 
 // s_waitcnt with vmcnt(n) (n < 64) and the other counters left alone
 DEV void wait_vmcnt(int n) {
     switch (n) {
 #define EVK_VMCNT_CASE(v) \
     case v: __builtin_amdgcn_s_waitcnt(((v) & 15) | (((v) >> 4) << 14) | 0x0f70); break;
-        EVK_VMCNT_CASE(0) EVK_VMCNT_CASE(4) EVK_VMCNT_CASE(8) EVK_VMCNT_CASE(12) EVK_VMCNT_CASE(16)
-        EVK_VMCNT_CASE(24) EVK_VMCNT_CASE(32)
+        EVK_VMCNT_CASE(0) EVK_VMCNT_CASE(2) EVK_VMCNT_CASE(3) EVK_VMCNT_CASE(4) EVK_VMCNT_CASE(6) EVK_VMCNT_CASE(8)
+        EVK_VMCNT_CASE(9) EVK_VMCNT_CASE(12) EVK_VMCNT_CASE(16) EVK_VMCNT_CASE(18) EVK_VMCNT_CASE(24) EVK_VMCNT_CASE(32)
 #undef EVK_VMCNT_CASE
         default: __builtin_amdgcn_s_waitcnt(0x0f70); break;
     }
 }
 
-template <int BM, int BN, bool TA, bool TB, int NWV = 4, int KG = 1, bool RAG = false>
+template <int BM, int BN, bool TA, bool TB, int NWV, int KG, int NST, bool RAG>
 __global__ __launch_bounds__(64 * NWV * KG, 1) void gemm_mfma(GemmArgs p, int tiles_m, int tiles_n) {
     constexpr int WGN = NWV / 2;  // waves along N (2 along M)
     constexpr int BK = MB_K, WM = BM / 2, WN = BN / WGN, FM = WM / 16, FN = WN / 16;
     constexpr int A_EL = BM * BK, B_EL = BN * BK, STAGE = A_EL + B_EL;
-    constexpr int NST = KG > 1 || RAG ? 2 : mfma_stages<BM>();  // per K group
+    static_assert(!RAG || NST == 2, "two stages through registers");
     constexpr int LPT = (BM * BK / 512 + BN * BK / 512) / NWV;  // DMA loads per wave per tile
     constexpr int OUT_LD = WN + 8;
     constexpr int OUT_EL = NWV * WM * OUT_LD;
@@ -217,15 +211,15 @@ __global__ __launch_bounds__(64 * NWV * KG, 1) void gemm_mfma(GemmArgs p, int ti
     RagTile<TB ? BN : BK, TB ? BK : BN, TB, 64 * NWV> rb;
     const int gtid = wave * 64 + lane;
     auto fetch = [&](int k0) {
-        if (TA) ra.load(A, M, k0, m0, K, M, gtid);
+        if constexpr (TA) ra.load(A, M, k0, m0, K, M, gtid);
         else ra.load(A, K, m0, k0, M, K, gtid);
-        if (TB) rb.load(B, K, n0, k0, N, K, gtid);
+        if constexpr (TB) rb.load(B, K, n0, k0, N, K, gtid);
         else rb.load(B, N, k0, n0, K, N, gtid);
     };
     auto issue = [&](int k0, f16* sa, f16* sb) {
-        if (TA) tile_to_lds<BK, BM, false, NWV>(ares, M, k0, m0, K, M, sa, wave, lane);
+        if constexpr (TA) tile_to_lds<BK, BM, false, NWV>(ares, M, k0, m0, K, M, sa, wave, lane);
         else tile_to_lds<BM, BK, true, NWV>(ares, K, m0, k0, M, K, sa, wave, lane);
-        if (TB) tile_to_lds<BN, BK, true, NWV>(bres, K, n0, k0, N, K, sb, wave, lane);
+        if constexpr (TB) tile_to_lds<BN, BK, true, NWV>(bres, K, n0, k0, N, K, sb, wave, lane);
         else tile_to_lds<BK, BN, false, NWV>(bres, N, k0, n0, K, N, sb, wave, lane);
     };
 
@@ -691,29 +685,116 @@ __global__ __launch_bounds__(256) void gemv_mf(GemmArgs p, float* __restrict__ p
 
 
 
-template <int BM, int BN, bool TA, bool TB, bool RAG>
-hipError_t launch_mfma(const GemmArgs& a, int batch, hipStream_t st) {
-    const int tm = (a.M + BM - 1) / BM, tn = (a.N + BN - 1) / BN;
-    dim3 grid((unsigned)(tm * tn), 1, batch);
-    constexpr int NWV = (BM >= 256 && BN >= 256) ? 8 : 4;  // the large tile: two waves per SIMD
-    if constexpr (BM == 64) {
-        // at most one tile per CU and a long K: four K groups per workgroup
-        // (16 waves), so that four shorter load/compute chains overlap
-        if ((int64_t)tm * tn * batch <= device_cu_count() && a.K >= 16 * MB_K) {
-            hipLaunchKernelGGL((gemm_mfma<BM, BN, TA, TB, NWV, 4, RAG>), grid, dim3(64 * NWV * 4), 0, st, a, tm, tn);
-            return hipGetLastError();
+// The instances of gemm_mfma and what one costs, for choosing among them:
+// a CU that holds j tiles at once (j <= resident, what LDS allows) spends
+// fixed + steps * (step1 .. step_r, linear in j) us on them, steps being the
+// 64-deep K tiles of one K group; the launch ends with its fullest CU, and
+// the part of a last round that leaves CUs idle runs up to `slack` faster
+// (less traffic beside it).  The constants are a least-squares fit to 470
+// random products (17 <= M <= 8192, N up to 12288, K up to 8192, every
+// operand order): the instance it picks is within 1.4 % of the fastest of
+// the nine on average, and 20 % faster than the three tile sizes (128 x 128
+// by 4 waves, four LDS stages) that were chosen by tile count alone before.
+// 8 waves on 128 x 128 tiles, or two K groups of 4, keep two waves on a SIMD
+// so that one's LDS reads and waits overlap the other's MFMAs; two stages
+// instead of four let two workgroups share a CU.
+//   us, before -> now: 2560 x 3072 x 768 28.7 -> 17.3, its weight gradient
+//   (3072 x 768 over 2560) 39.5 -> 26.1, 1000 x 2304 x 768 13.8 -> 9.4,
+//   512 x 4096 x 4096 58.5 -> 27.3, 2048^3 32.4 -> 23.6, 40 x 11008 x 4096
+//   21.0 -> 17.9, 2560 x 768 x 32000 (B transposed) 247 -> 173
+struct GemmPlan {
+    int bm, bn, kg, resident;
+    float launch, fixed, step1, step_r, slack;
+};
+constexpr GemmPlan kPlans[] = {
+    {256, 256, 1, 1, 0.0f, 7.81f, 1.74f, 1.74f, 0.30f},   // 0: 8 waves
+    {128, 128, 1, 2, 0.0f, 4.22f, 0.72f, 1.09f, 0.28f},   // 1: 8 waves
+    {128, 128, 2, 1, 2.24f, 2.99f, 1.19f, 1.19f, 0.26f},  // 2: 2 groups of 4 waves
+    {128, 64, 2, 1, 1.85f, 2.17f, 0.79f, 0.79f, 0.19f},   // 3: 2 groups of 4, three stages
+    {64, 64, 1, 4, 0.75f, 2.05f, 0.43f, 0.91f, 0.18f},    // 4: 4 waves
+    {64, 64, 2, 2, 2.19f, 1.16f, 0.72f, 0.94f, 0.46f},    // 5: 2 groups of 4, two stages
+    {64, 64, 2, 1, 1.82f, 1.63f, 0.50f, 0.50f, 0.16f},    // 6: 2 groups of 4, four stages
+    {64, 64, 4, 1, 2.54f, 1.57f, 1.19f, 1.19f, 0.46f},    // 7: 4 groups of 4
+    {32, 64, 4, 1, 2.35f, 1.32f, 0.95f, 0.95f, 0.48f},    // 8: 4 groups of 4
+};
+constexpr int kPlanCount = sizeof(kPlans) / sizeof(kPlans[0]);
+// A row-major (8 undercuts 7 everywhere), A stored (K,M) (whose LDS rows of
+// BM halves need 64), and tiles through registers
+constexpr unsigned kRowPlans = 0x1ffu & ~(1u << 7), kColPlans = 0x1ffu & ~(1u << 8);
+constexpr unsigned kRagPlans = 1u << 1 | 1u << 4 | 1u << 5 | 1u << 7;
+
+float plan_cost(const GemmPlan& p, const GemmArgs& a, int batch, int cus) {
+    const int64_t tiles = (int64_t)((a.M + p.bm - 1) / p.bm) * ((a.N + p.bn - 1) / p.bn) * batch;
+    const int64_t m = (tiles + cus - 1) / cus;  // tiles of the fullest CU
+    const float steps = (float)(((a.K + MB_K - 1) / MB_K + p.kg - 1) / p.kg);
+    auto round_us = [&](int64_t j) {
+        if (j == 0) return 0.0f;
+        const float step =
+            p.resident == 1 ? p.step1 : p.step1 + (p.step_r - p.step1) * (float)(j - 1) / (float)(p.resident - 1);
+        return p.fixed + steps * step;
+    };
+    auto upto = [&](int64_t q) { return (float)(q / p.resident) * round_us(p.resident) + round_us(q % p.resident); };
+    const float busy = (float)(tiles - (m - 1) * cus) / (float)cus;
+    return p.launch + upto(m - 1) + (upto(m) - upto(m - 1)) * (1.0f - p.slack * (1.0f - busy));
+}
+
+int choose_plan(const GemmArgs& a, int batch, unsigned allowed) {
+    const int cus = device_cu_count();
+    int best = -1;
+    float best_us = 0.0f;
+    for (int i = 0; i < kPlanCount; ++i) {
+        if (!(allowed >> i & 1u)) continue;
+        const float us = plan_cost(kPlans[i], a, batch, cus);
+        if (best < 0 || us < best_us) {
+            best = i;
+            best_us = us;
         }
     }
-    hipLaunchKernelGGL((gemm_mfma<BM, BN, TA, TB, NWV, 1, RAG>), grid, dim3(64 * NWV), 0, st, a, tm, tn);
+    return best;
+}
+
+template <int PLAN, bool TA, bool TB, bool RAG>
+hipError_t launch_mfma(const GemmArgs& a, int batch, hipStream_t st) {
+    constexpr GemmPlan P = kPlans[PLAN];
+    constexpr int NWV = PLAN <= 1 ? 8 : 4, NST = PLAN == 3 ? 3 : PLAN == 6 ? 4 : 2;
+    const int tm = (a.M + P.bm - 1) / P.bm, tn = (a.N + P.bn - 1) / P.bn;
+    hipLaunchKernelGGL((gemm_mfma<P.bm, P.bn, TA, TB, NWV, P.kg, NST, RAG>), dim3((unsigned)(tm * tn), 1, batch),
+                       dim3(64 * NWV * P.kg), 0, st, a, tm, tn);
     return hipGetLastError();
 }
 
-template <int BM, int BN, bool RAG>
+template <int PLAN, bool RAG>
 hipError_t launch_mfma_t(const GemmArgs& a, int batch, bool ta, bool tb, hipStream_t st) {
-    if (!ta && !tb) return launch_mfma<BM, BN, false, false, RAG>(a, batch, st);
-    if (!ta && tb) return launch_mfma<BM, BN, false, true, RAG>(a, batch, st);
-    if (ta && !tb) return launch_mfma<BM, BN, true, false, RAG>(a, batch, st);
-    return launch_mfma<BM, BN, true, true, RAG>(a, batch, st);
+    if (ta) {
+        if constexpr (RAG || PLAN != 8)
+            return tb ? launch_mfma<PLAN, true, true, RAG>(a, batch, st) : launch_mfma<PLAN, true, false, RAG>(a, batch, st);
+    } else {
+        if constexpr (RAG || PLAN != 7)
+            return tb ? launch_mfma<PLAN, false, true, RAG>(a, batch, st) : launch_mfma<PLAN, false, false, RAG>(a, batch, st);
+    }
+    return hipErrorInvalidValue;  // outside kRowPlans / kColPlans
+}
+
+hipError_t launch_plan(int plan, const GemmArgs& a, int batch, bool ta, bool tb, hipStream_t st) {
+    switch (plan) {
+        case 0: return launch_mfma_t<0, false>(a, batch, ta, tb, st);
+        case 1: return launch_mfma_t<1, false>(a, batch, ta, tb, st);
+        case 2: return launch_mfma_t<2, false>(a, batch, ta, tb, st);
+        case 3: return launch_mfma_t<3, false>(a, batch, ta, tb, st);
+        case 4: return launch_mfma_t<4, false>(a, batch, ta, tb, st);
+        case 5: return launch_mfma_t<5, false>(a, batch, ta, tb, st);
+        case 6: return launch_mfma_t<6, false>(a, batch, ta, tb, st);
+        case 7: return launch_mfma_t<7, false>(a, batch, ta, tb, st);
+        default: return launch_mfma_t<8, false>(a, batch, ta, tb, st);
+    }
+}
+hipError_t launch_plan_rag(int plan, const GemmArgs& a, int batch, bool ta, bool tb, hipStream_t st) {
+    switch (plan) {
+        case 1: return launch_mfma_t<1, true>(a, batch, ta, tb, st);
+        case 4: return launch_mfma_t<4, true>(a, batch, ta, tb, st);
+        case 5: return launch_mfma_t<5, true>(a, batch, ta, tb, st);
+        default: return launch_mfma_t<7, true>(a, batch, ta, tb, st);
+    }
 }
 
 // Library workspace for the split-K GEMV (grow-only): partials, and the
@@ -826,15 +907,10 @@ int gemm_dispatch(const GemmArgs& a, int batch, bool ta, bool tb, bool vec_ok, h
         e = hipGetLastError();
         return e == hipSuccess ? EVKHIP_OK : check_hip(e, "gemv launch");
     }
-    const int64_t cus = device_cu_count();
-    auto tiles = [&](int bm, int bn) {
-        return (int64_t)((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn) * batch;
-    };
     // The LDS-direct loads address each operand through a buffer descriptor
     // and take whole, aligned 16-byte chunks; every other operand (odd row
     // lengths, pointers off a 16-byte boundary, 2 GiB and more) goes through
-    // registers, in 128- or 64-wide tiles: with 256 the staging registers no
-    // longer fit beside the accumulators.  Against the kernels that served
+    // registers (kRagPlans).  Against the kernels that served
     // such calls before, one thread per element (odd rows) and a tiled one
     // with register transposes (2 GiB): 1000 x 1001 x 777 336 -> 18.2 us,
     // 3000 x 1501 x 801 1116 -> 53 us, 51 x 50 x 1481 179 -> 13.7 us;
@@ -842,13 +918,9 @@ int gemm_dispatch(const GemmArgs& a, int batch, bool ta, bool tb, bool vec_ok, h
     const bool direct = vec_ok && (int64_t)a.M * a.K * 2 < INT32_MAX && (int64_t)a.K * a.N * 2 < INT32_MAX &&
                         (int64_t)a.M * a.N < INT32_MAX;
     if (direct) {
-        if (tiles(256, 256) >= cus) e = launch_mfma_t<256, 256, false>(a, batch, ta, tb, st);
-        else if (tiles(128, 128) >= cus / 2) e = launch_mfma_t<128, 128, false>(a, batch, ta, tb, st);
-        else e = launch_mfma_t<64, 64, false>(a, batch, ta, tb, st);
-    } else if (tiles(128, 128) >= cus / 2) {
-        e = launch_mfma_t<128, 128, true>(a, batch, ta, tb, st);
+        e = launch_plan(choose_plan(a, batch, ta ? kColPlans : kRowPlans), a, batch, ta, tb, st);
     } else {
-        e = launch_mfma_t<64, 64, true>(a, batch, ta, tb, st);
+        e = launch_plan_rag(choose_plan(a, batch, kRagPlans), a, batch, ta, tb, st);
     }
     return e == hipSuccess ? EVKHIP_OK : check_hip(e, "gemm launch");
 }

@@ -278,3 +278,22 @@ def test_weight_gradient_of_ragged_token_count(dev, orc, K):
     a, b, c0 = orc.uniform_f16((K, 136), 98), orc.uniform_f16((K, 264), 99), orc.uniform_f16((136, 264), 100)
     got = run_mm(evk, dev, a, b, None, True, False, True, c0)
     assert_close_f16(got, orc.matmul(a, b, c=c0, transpose_a=True, acc_c=True), what=f"K={K}")
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)])
+@pytest.mark.parametrize("M,N,K", [(2888, 2880, 552), (2320, 1736, 24), (1968, 1080, 720), (2384, 520, 400), (40, 24, 24),
+                                   (24, 24, 264), (136, 2584, 328), (24, 88, 1248), (200, 24, 4104)])
+def test_each_instance(dev, orc, ta, tb, M, N, K):
+    """One product per instance of the MFMA kernel (256 x 256 down to 32 x 64
+    tiles, one to four K groups, two to four LDS stages): ragged last tiles, K
+    ranges of unequal length and groups without any; a sample of rows in every
+    row tile against the oracle, accumulating into C."""
+    import evk_amd as evk
+    a = orc.uniform_f16((K, M) if ta else (M, K), 111 + M)
+    b = orc.uniform_f16((N, K) if tb else (K, N), 112 + N)
+    c0 = orc.uniform_f16((M, N), 113)
+    got = run_mm(evk, dev, a, b, None, ta, tb, True, c0)
+    rows = np.unique(np.r_[np.arange(0, M, 29), M - 1])
+    A = f32(a[:, rows].T if ta else a[rows])
+    want = (A @ f32(b.T if tb else b) + f32(c0[rows])).astype(np.float16).view(np.uint16)
+    assert_close_f16(got[rows], want, what=f"{ta}{tb} {M}x{N}x{K}")
