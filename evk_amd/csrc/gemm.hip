@@ -159,8 +159,7 @@ DEV void wait_vmcnt(int n) {
     switch (n) {
 #define EVK_VMCNT_CASE(v) \
     case v: __builtin_amdgcn_s_waitcnt(((v) & 15) | (((v) >> 4) << 14) | 0x0f70); break;
-        EVK_VMCNT_CASE(0) EVK_VMCNT_CASE(2) EVK_VMCNT_CASE(3) EVK_VMCNT_CASE(4) EVK_VMCNT_CASE(6) EVK_VMCNT_CASE(8)
-        EVK_VMCNT_CASE(9) EVK_VMCNT_CASE(12) EVK_VMCNT_CASE(16) EVK_VMCNT_CASE(18) EVK_VMCNT_CASE(24) EVK_VMCNT_CASE(32)
+        EVK_VMCNT_CASE(0) EVK_VMCNT_CASE(3) EVK_VMCNT_CASE(4) EVK_VMCNT_CASE(6) EVK_VMCNT_CASE(8)
 #undef EVK_VMCNT_CASE
         default: __builtin_amdgcn_s_waitcnt(0x0f70); break;
     }
@@ -228,6 +227,40 @@ __global__ __launch_bounds__(64 * NWV * KG, 1) void gemm_mfma(GemmArgs p, int ti
     for (int i = 0; i < FM; ++i)
 #pragma unroll
         for (int j = 0; j < FN; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+    // The wave's part of C in 16-byte row chunks, chunk q of a lane staged at
+    // its place in the wave's LDS tile (the epilogue's).  A call that adds to C
+    // requests its chunks before the first operand tile, where the registers
+    // allow it, so that they are there when the last product is (C
+    // read at the end: 3072 x 768 over 2560 rows 33.4 us, now 30.0; the whole
+    // MLP step 184 us with 2-byte reads and writes of C, 171, now 162).
+    constexpr int CPR = WN / 8, CQ = WM * CPR / 64;
+    constexpr bool C_EARLY = CQ <= 8;
+    f16* ot = smem + wave * WM * OUT_LD;
+    auto each_chunk = [&](auto&& f) {  // f(q, C address, LDS address, columns inside C)
+#pragma unroll
+        for (int q = 0; q < CQ; ++q) {
+            const int r = (lane + 64 * q) / CPR, cc = ((lane + 64 * q) % CPR) * 8;
+            const int row = m0 + wm0 + r, col = n0 + wn0 + cc;
+            if (row < M && col < N) f(q, Cp + (int64_t)row * N + col, ot + r * OUT_LD + cc, N - col);
+        }
+    };
+    const bool adds = p.acc || p.epi == GEMM_RESIDUAL;
+    u32x4 prior[CQ];
+    auto load_c = [&] {
+        each_chunk([&](int q, const f16* c, f16*, int left) {
+            if (!RAG || left >= 8) {
+                __builtin_memcpy(&prior[q], c, 16);
+            } else {
+                half8 h = {};
+#pragma unroll
+                for (int e = 0; e < 7; ++e)
+                    if (e < left) h[e] = c[e];
+                prior[q] = as_u32x4(h);
+            }
+        });
+    };
+    if (C_EARLY && adds && kg == 0) load_c();
 
     // One LDS tile: 2 k-steps x FM fragment rows, FN MFMAs per row, run as
     // 2 FM steps.  A fragments are read AD steps ahead (ring of AD + 1); the
@@ -331,60 +364,55 @@ __global__ __launch_bounds__(64 * NWV * KG, 1) void gemm_mfma(GemmArgs p, int ti
                     for (int j = 0; j < FN; ++j) acc[i][j] += red[((((q - 1) * NWV + wave) * FM + i) * FN + j) * 64 + lane];
         }
     }
-    if (p.acc) {  // C += A B: one rounding of the fp32 sum per element
-        if (kg > 0) return;
+    // Each wave stages its fp16 tile in LDS: the prior C first where the call
+    // adds to it, then the results, then 16-byte row chunks to C.  The staging
+    // area overlaps the stages, which every wave has finished reading once all
+    // have passed this barrier.
+    __syncthreads();
+    if (kg > 0) return;  // past the last barrier: group 0 stores the tile
+    auto wave_lds = [] {  // this wave's LDS accesses so far are done
+        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+        __builtin_amdgcn_wave_barrier();
+    };
+    auto stage = [&](auto&& f) {  // LDS tile = fp16(f(sum, what it holds))
 #pragma unroll
         for (int i = 0; i < FM; ++i)
 #pragma unroll
-            for (int j = 0; j < FN; ++j) {
-                const int col = n0 + wn0 + 16 * j + l16;
+            for (int j = 0; j < FN; ++j)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const int row = m0 + wm0 + 16 * i + 4 * g + e;
-                    if (row < M && col < N) {
-                        f16* dst = Cp + (int64_t)row * N + col;
-                        *dst = (f16)(acc[i][j][e] + (float)*dst);
-                    }
+                    f16* o = ot + (16 * i + 4 * g + e) * OUT_LD + 16 * j + l16;
+                    *o = (f16)f(acc[i][j][e], o);
                 }
-            }
-        return;
+    };
+    if (adds) {
+        if constexpr (!C_EARLY) load_c();
+        each_chunk([&](int q, f16*, f16* o, int) { *reinterpret_cast<u32x4*>(o) = prior[q]; });
+        wave_lds();
+        if (p.acc) stage([](float v, const f16* o) { return v + (float)*o; });  // one rounding of the fp32 sum
+        else stage([](float v, const f16* o) { return (float)(f16)v + (float)*o; });
+    } else if (p.epi == GEMM_GELU) {
+        stage([](float v, const f16*) { return gelu_fast((float)(f16)v); });
+    } else {
+        stage([](float v, const f16*) { return v; });
     }
-    // stage the wave's tile as fp16 rows, then 16-byte row chunks to C; the
-    // staging area overlaps the stages, which every wave has finished
-    // reading once all have passed this barrier
-    __syncthreads();
-    if (kg > 0) return;  // past the last barrier: group 0 stores the tile
-    f16* ot = smem + wave * WM * OUT_LD;
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) ot[(16 * i + 4 * g + e) * OUT_LD + 16 * j + l16] = (f16)acc[i][j][e];
-    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's LDS writes
-    __builtin_amdgcn_wave_barrier();
-    constexpr int CPR = WN / 8;
-#pragma unroll 4
-    for (int q = lane; q < WM * CPR; q += 64) {
-        const int r = q / CPR, cc = (q % CPR) * 8;
-        const int row = m0 + wm0 + r, col = n0 + wn0 + cc;
-        const u32x4 v = *reinterpret_cast<const u32x4*>(ot + r * OUT_LD + cc);
+    wave_lds();
+    each_chunk([&](int, f16* c, const f16* o, int left) {
+        const u32x4 v = *reinterpret_cast<const u32x4*>(o);
         if constexpr (RAG) {
-            if (row >= M || col >= N) continue;
-            f16* dst = Cp + (int64_t)row * N + col;
-            if (col + 8 <= N) {
-                __builtin_memcpy(dst, &v, 16);
+            if (left >= 8) {
+                __builtin_memcpy(c, &v, 16);
             } else {
                 const half8 h = as_half8(v);
 #pragma unroll
                 for (int e = 0; e < 7; ++e)
-                    if (col + e < N) dst[e] = h[e];
+                    if (e < left) c[e] = h[e];
             }
-            continue;
+        } else {
+            // nontemporal: C is written once (QKV shape 0.785 -> 0.763 ms)
+            __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(c));
         }
-        // nontemporal: C is written once (QKV shape 0.785 -> 0.763 ms)
-        if (row < M && col < N) __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(Cp + (int64_t)row * N + col));
-    }
+    });
 }
 
 // ---- skinny GEMV: C(M,N) = A(M,K) B(K,N), M <= 16, B row-major -------------
@@ -690,38 +718,40 @@ __global__ __launch_bounds__(256) void gemv_mf(GemmArgs p, float* __restrict__ p
 // fixed + steps * (step1 .. step_r, linear in j) us on them, steps being the
 // 64-deep K tiles of one K group; the launch ends with its fullest CU, and
 // the part of a last round that leaves CUs idle runs up to `slack` faster
-// (less traffic beside it).  The constants are a least-squares fit to 470
+// (less traffic beside it).  The constants are a least-squares fit to 300
 // random products (17 <= M <= 8192, N up to 12288, K up to 8192, every
-// operand order): the instance it picks is within 1.4 % of the fastest of
-// the nine on average, and 20 % faster than the three tile sizes (128 x 128
-// by 4 waves, four LDS stages) that were chosen by tile count alone before.
-// 8 waves on 128 x 128 tiles, or two K groups of 4, keep two waves on a SIMD
-// so that one's LDS reads and waits overlap the other's MFMAs; two stages
-// instead of four let two workgroups share a CU.
+// operand order) whose operands come from outside the L2, as between the
+// layers of a model: the instance it picks is within 1.6 % of the fastest of
+// 17 on average.  Before, three tile sizes were chosen by tile count alone;
+// 128 x 128 ran on 4 waves with four LDS stages, one wave per SIMD.  8 waves,
+// or two K groups of 4 or 8, put two or more on a SIMD so that one's LDS
+// reads and waits overlap the other's MFMAs; two stages instead of four let
+// two workgroups share a CU, and more stages pay where a grid fits the CUs
+// once and the operands' latency shows.
 //   us, before -> now: 2560 x 3072 x 768 28.7 -> 17.3, its weight gradient
-//   (3072 x 768 over 2560) 39.5 -> 26.1, 1000 x 2304 x 768 13.8 -> 9.4,
-//   512 x 4096 x 4096 58.5 -> 27.3, 2048^3 32.4 -> 23.6, 40 x 11008 x 4096
-//   21.0 -> 17.9, 2560 x 768 x 32000 (B transposed) 247 -> 173
+//   (3072 x 768 over 2560) 39.5 -> 25.1, 1000 x 2304 x 768 13.8 -> 10.1,
+//   512 x 4096 x 4096 58.5 -> 28.0, 2048^3 32.4 -> 24.0, 40 x 11008 x 4096
+//   21.0 -> 18.1, 2560 x 768 x 32000 (B transposed) 247 -> 173
 struct GemmPlan {
-    int bm, bn, kg, resident;
+    int bm, bn, waves, kg, stages, resident;
     float launch, fixed, step1, step_r, slack;
 };
 constexpr GemmPlan kPlans[] = {
-    {256, 256, 1, 1, 0.0f, 7.81f, 1.74f, 1.74f, 0.30f},   // 0: 8 waves
-    {128, 128, 1, 2, 0.0f, 4.22f, 0.72f, 1.09f, 0.28f},   // 1: 8 waves
-    {128, 128, 2, 1, 2.24f, 2.99f, 1.19f, 1.19f, 0.26f},  // 2: 2 groups of 4 waves
-    {128, 64, 2, 1, 1.85f, 2.17f, 0.79f, 0.79f, 0.19f},   // 3: 2 groups of 4, three stages
-    {64, 64, 1, 4, 0.75f, 2.05f, 0.43f, 0.91f, 0.18f},    // 4: 4 waves
-    {64, 64, 2, 2, 2.19f, 1.16f, 0.72f, 0.94f, 0.46f},    // 5: 2 groups of 4, two stages
-    {64, 64, 2, 1, 1.82f, 1.63f, 0.50f, 0.50f, 0.16f},    // 6: 2 groups of 4, four stages
-    {64, 64, 4, 1, 2.54f, 1.57f, 1.19f, 1.19f, 0.46f},    // 7: 4 groups of 4
-    {32, 64, 4, 1, 2.35f, 1.32f, 0.95f, 0.95f, 0.48f},    // 8: 4 groups of 4
+    {256, 256, 8, 1, 2, 1, 0.0f, 8.04f, 1.79f, 1.79f, 0.31f},   // 0
+    {128, 128, 8, 1, 2, 2, 0.0f, 4.11f, 0.79f, 1.19f, 0.22f},   // 1
+    {128, 128, 8, 2, 2, 1, 1.87f, 3.08f, 1.23f, 1.23f, 0.22f},  // 2
+    {128, 64, 4, 2, 3, 1, 1.96f, 2.20f, 0.82f, 0.82f, 0.16f},   // 3
+    {64, 64, 4, 1, 2, 4, 0.30f, 2.59f, 0.47f, 0.94f, 0.06f},    // 4
+    {128, 128, 8, 1, 4, 1, 1.64f, 2.75f, 0.65f, 0.65f, 0.24f},  // 5
+    {64, 64, 4, 2, 3, 1, 1.89f, 1.66f, 0.53f, 0.53f, 0.12f},    // 6
+    {32, 64, 4, 2, 4, 1, 1.85f, 1.39f, 0.46f, 0.46f, 0.07f},    // 7
 };
 constexpr int kPlanCount = sizeof(kPlans) / sizeof(kPlans[0]);
-// A row-major (8 undercuts 7 everywhere), A stored (K,M) (whose LDS rows of
-// BM halves need 64), and tiles through registers
-constexpr unsigned kRowPlans = 0x1ffu & ~(1u << 7), kColPlans = 0x1ffu & ~(1u << 8);
-constexpr unsigned kRagPlans = 1u << 1 | 1u << 4 | 1u << 5 | 1u << 7;
+// A row-major, A stored (K,M) (whose LDS rows of BM halves need 64), and
+// tiles through registers (two stages: 128 x 128, and 64 x 64 by one and two
+// K groups)
+constexpr unsigned kRowPlans = 0xffu, kColPlans = 0x7fu;
+constexpr unsigned kRagPlans = 1u << 1 | 1u << 4 | 1u << 6;
 
 float plan_cost(const GemmPlan& p, const GemmArgs& a, int batch, int cus) {
     const int64_t tiles = (int64_t)((a.M + p.bm - 1) / p.bm) * ((a.N + p.bn - 1) / p.bn) * batch;
@@ -756,23 +786,19 @@ int choose_plan(const GemmArgs& a, int batch, unsigned allowed) {
 template <int PLAN, bool TA, bool TB, bool RAG>
 hipError_t launch_mfma(const GemmArgs& a, int batch, hipStream_t st) {
     constexpr GemmPlan P = kPlans[PLAN];
-    constexpr int NWV = PLAN <= 1 ? 8 : 4, NST = PLAN == 3 ? 3 : PLAN == 6 ? 4 : 2;
     const int tm = (a.M + P.bm - 1) / P.bm, tn = (a.N + P.bn - 1) / P.bn;
-    hipLaunchKernelGGL((gemm_mfma<P.bm, P.bn, TA, TB, NWV, P.kg, NST, RAG>), dim3((unsigned)(tm * tn), 1, batch),
-                       dim3(64 * NWV * P.kg), 0, st, a, tm, tn);
+    hipLaunchKernelGGL((gemm_mfma<P.bm, P.bn, TA, TB, P.waves, P.kg, RAG ? 2 : P.stages, RAG>),
+                       dim3((unsigned)(tm * tn), 1, batch), dim3(64 * P.waves * P.kg), 0, st, a, tm, tn);
     return hipGetLastError();
 }
 
 template <int PLAN, bool RAG>
 hipError_t launch_mfma_t(const GemmArgs& a, int batch, bool ta, bool tb, hipStream_t st) {
-    if (ta) {
-        if constexpr (RAG || PLAN != 8)
-            return tb ? launch_mfma<PLAN, true, true, RAG>(a, batch, st) : launch_mfma<PLAN, true, false, RAG>(a, batch, st);
-    } else {
-        if constexpr (RAG || PLAN != 7)
-            return tb ? launch_mfma<PLAN, false, true, RAG>(a, batch, st) : launch_mfma<PLAN, false, false, RAG>(a, batch, st);
-    }
-    return hipErrorInvalidValue;  // outside kRowPlans / kColPlans
+    if (!ta)
+        return tb ? launch_mfma<PLAN, false, true, RAG>(a, batch, st) : launch_mfma<PLAN, false, false, RAG>(a, batch, st);
+    if constexpr (PLAN != 7)
+        return tb ? launch_mfma<PLAN, true, true, RAG>(a, batch, st) : launch_mfma<PLAN, true, false, RAG>(a, batch, st);
+    return hipErrorInvalidValue;  // not in kColPlans
 }
 
 hipError_t launch_plan(int plan, const GemmArgs& a, int batch, bool ta, bool tb, hipStream_t st) {
@@ -784,16 +810,14 @@ hipError_t launch_plan(int plan, const GemmArgs& a, int batch, bool ta, bool tb,
         case 4: return launch_mfma_t<4, false>(a, batch, ta, tb, st);
         case 5: return launch_mfma_t<5, false>(a, batch, ta, tb, st);
         case 6: return launch_mfma_t<6, false>(a, batch, ta, tb, st);
-        case 7: return launch_mfma_t<7, false>(a, batch, ta, tb, st);
-        default: return launch_mfma_t<8, false>(a, batch, ta, tb, st);
+        default: return launch_mfma_t<7, false>(a, batch, ta, tb, st);
     }
 }
 hipError_t launch_plan_rag(int plan, const GemmArgs& a, int batch, bool ta, bool tb, hipStream_t st) {
     switch (plan) {
         case 1: return launch_mfma_t<1, true>(a, batch, ta, tb, st);
         case 4: return launch_mfma_t<4, true>(a, batch, ta, tb, st);
-        case 5: return launch_mfma_t<5, true>(a, batch, ta, tb, st);
-        default: return launch_mfma_t<7, true>(a, batch, ta, tb, st);
+        default: return launch_mfma_t<6, true>(a, batch, ta, tb, st);
     }
 }
 
@@ -871,7 +895,7 @@ int gemm_dispatch(const GemmArgs& a, int batch, bool ta, bool tb, bool vec_ok, h
                   const GemvScratch* fixed) {
     if (a.M == 0 || a.N == 0) return EVKHIP_OK;
     hipError_t e;
-    if (vec_ok && a.M <= 16 && !ta && !tb && a.K > 0 && (int64_t)a.K * a.N * 2 < INT32_MAX &&
+    if (vec_ok && a.epi == GEMM_STORE && a.M <= 16 && !ta && !tb && a.K > 0 && (int64_t)a.K * a.N * 2 < INT32_MAX &&
         (int64_t)a.M * a.K * 2 < INT32_MAX) {
         const int ncb = (a.N + SK_CB - 1) / SK_CB;
         const int nks = (a.K + SK_KC - 1) / SK_KC;

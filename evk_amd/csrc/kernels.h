@@ -12,8 +12,12 @@ struct GemmArgs {
     f16* C;
     int M, N, K;
     int64_t sA, sB, sC;  // per-batch element strides (0 = broadcast)
-    int acc;
+    int acc;             // C = fp16(C + A B)
+    int epi;             // GEMM_*, without acc
 };
+// Ops folded into the store of a product, with the roundings of the separate
+// ops: C = fp16(C + fp16(A B)) and C = fp16(gelu(fp16(A B))).
+enum { GEMM_STORE = 0, GEMM_RESIDUAL = 1, GEMM_GELU = 2 };
 // Caller-provided split-K scratch of the skinny (M <= 16) path: partials and
 // arrival counters.  With it, gemm_dispatch allocates nothing.
 struct GemvScratch {
@@ -46,6 +50,8 @@ struct FlashArgs {
     float scale_log2;  // scale * log2(e)
     float scale;
     int spin_limit;    // iterations of a bounded in-kernel wait before it gives up
+    int64_t out_bstride;  // forward, flash_out_strided head sizes only: elements between the O of consecutive
+    int out_rstride;      // batches and query rows; 0, 0 = contiguous (B, N, H*Dh)
 };
 // flash_wide.hip: MFMA forward / backward for the other multiples of 16 up
 // to 256.  The backward takes the forward's O and LSE in a.o / a.lse (no
@@ -59,6 +65,10 @@ inline bool flash_mfma_head(uint32_t dh) { return dh == 32 || dh == 64 || dh == 
 // buffer offsets: they run only while that batch stays below 2 GiB.
 inline bool flash_wide_fits(uint64_t N, uint64_t H, uint32_t dh) {
     return N * H * dh * 2u < (uint64_t)INT32_MAX;
+}
+// Whether flash_forward takes out_bstride / out_rstride at this size.
+inline bool flash_out_strided(uint64_t N, uint32_t dh) {
+    return (dh == 32 || dh == 64) && N * dh * 2 < (uint64_t)INT32_MAX;
 }
 int flash_forward(FlashArgs a, int dh, bool mfma, bool causal, hipStream_t st);
 int flash_backward(FlashArgs a, int dh, bool mfma, bool causal, hipStream_t st);

@@ -281,11 +281,11 @@ def test_weight_gradient_of_ragged_token_count(dev, orc, K):
 
 
 @pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)])
-@pytest.mark.parametrize("M,N,K", [(2888, 2880, 552), (2320, 1736, 24), (1968, 1080, 720), (2384, 520, 400), (40, 24, 24),
-                                   (24, 24, 264), (136, 2584, 328), (24, 88, 1248), (200, 24, 4104)])
+@pytest.mark.parametrize("M,N,K", [(2888, 2880, 552), (2320, 1736, 24), (1120, 1952, 1376), (336, 2752, 328), (40, 24, 24),
+                                   (1136, 1824, 336), (1680, 264, 208), (24, 24, 72), (24, 88, 1248), (200, 24, 4104)])
 def test_each_instance(dev, orc, ta, tb, M, N, K):
     """One product per instance of the MFMA kernel (256 x 256 down to 32 x 64
-    tiles, one to four K groups, two to four LDS stages): ragged last tiles, K
+    tiles, one or two K groups, two to four LDS stages): ragged last tiles, K
     ranges of unequal length and groups without any; a sample of rows in every
     row tile against the oracle, accumulating into C."""
     import evk_amd as evk
