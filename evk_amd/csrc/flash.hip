@@ -847,10 +847,11 @@ __global__ __launch_bounds__(512, 1) void flash_fwd_ks(FlashArgs p) {
     const int row = R0 + q;
     const float inv_l = l > 0.0f ? 1.0f / l : 0.0f;
     if (active && row < NH) {
+        f16* orow = p.out + b * p.out_bstride + (int64_t)row * p.out_rstride;
 #pragma unroll
         for (int d = 0; d < DB; ++d) {
             const uint2 o = {pack_h2(a[d][0] * inv_l, a[d][1] * inv_l), pack_h2(a[d][2] * inv_l, a[d][3] * inv_l)};
-            *reinterpret_cast<uint2*>(p.out + ((int64_t)b * NH + row) * DH + d * 16 + mg * 4) = o;
+            *reinterpret_cast<uint2*>(orow + d * 16 + mg * 4) = o;
         }
         if (p.lse && mg == 0) {
             const float lse = l > 0.0f ? (m + log2f(l)) * kLn2 : -INFINITY;
@@ -1893,8 +1894,13 @@ hipError_t launch_fwd(const FlashArgs& a, bool causal, int mode, hipStream_t st)
             constexpr int QB = FWD_KS_QB;
             const int64_t nrg_ks = ((int64_t)a.N * a.H + 16 * QB - 1) / (16 * QB);
             dim3 gk((unsigned)((nrg_ks + 1) / 2 * a.B));
-            if (causal) hipLaunchKernelGGL((flash_fwd_ks<DH, QB, true>), gk, dim3(512), 0, st, a);
-            else hipLaunchKernelGGL((flash_fwd_ks<DH, QB, false>), gk, dim3(512), 0, st, a);
+            FlashArgs s = a;
+            if (s.out_rstride == 0) {
+                s.out_rstride = DH;
+                s.out_bstride = (int64_t)a.N * a.H * DH;
+            }
+            if (causal) hipLaunchKernelGGL((flash_fwd_ks<DH, QB, true>), gk, dim3(512), 0, st, s);
+            else hipLaunchKernelGGL((flash_fwd_ks<DH, QB, false>), gk, dim3(512), 0, st, s);
             return hipGetLastError();
         }
     }
