@@ -14,6 +14,7 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+import struct
 from typing import Optional
 
 __all__ = [
@@ -162,17 +163,54 @@ def desc(t, shape=None) -> Tensor:
     return d
 
 
+# Calls of the op wrappers.  A small op takes a few us on the GPU, so the time
+# to describe its tensors in Python counts: packed bytes of an evkhip_tensor
+# (0.7 us against 1.5 for filling a ctypes structure field by field), passed as
+# a plain pointer, and the raw handle of torch's current stream instead of a
+# Stream object.
+_PACK = [struct.Struct("@QI%dI%dx" % (n, C.sizeof(Tensor) - 12 - 4 * n)).pack for n in range(MAX_DIMS + 1)]
+
+
+class _Calls:
+    """The library's functions with tensor descriptors as packed bytes."""
+
+    def __getattr__(self, name):
+        fn = lib()[name]  # an object of its own: lib().<name> keeps its argument types
+        fn.restype, args = SIGNATURES[name]
+        fn.argtypes = [C.c_char_p if a is TP else a for a in args]
+        setattr(self, name, fn)
+        return fn
+
+
+_calls = _Calls()
+
+
+def _D(t) -> bytes:
+    """desc(t) as bytes."""
+    if isinstance(t, tuple):
+        return bytes(desc(t))
+    if not t.is_contiguous():
+        raise ValueError("evk_amd ops take contiguous tensors")
+    shape = t.shape
+    try:
+        return _PACK[len(shape)](t.data_ptr(), len(shape), *shape)
+    except (struct.error, IndexError):  # sizes past 32 bits, rank > 8: as desc has it
+        return bytes(desc(t))
+
+
+_torch = None
+
+
 def _stream(stream=None):
     if stream is not None:
-        return C.c_void_p(int(stream))
-    import torch
-    if torch.cuda.is_available():
-        return C.c_void_p(torch.cuda.current_stream().cuda_stream)
-    return C.c_void_p(0)
-
-
-def _ref(d: Tensor):
-    return C.byref(d)
+        return int(stream)
+    global _torch
+    if _torch is None:
+        import torch
+        _torch = torch
+    if _torch.cuda.is_initialized():  # current_stream() of the current device, as its handle
+        return _torch._C._cuda_getCurrentRawStream(_torch._C._cuda_getDevice())
+    return _torch.cuda.current_stream().cuda_stream if _torch.cuda.is_available() else 0
 
 
 # ---------------------------------------------------------------------------
@@ -218,8 +256,7 @@ def debug_set_spin_limit(iterations: int) -> None:
 def matmul(a, b, c, transpose_a=False, transpose_b=False, acc_c=False, TILE_M=80, TILE_N=80,
            stream=None):
     """evk::ai::matmul (evk_ai.h:495): C (+)= op(A) . op(B) with batch broadcast."""
-    da, db, dc = desc(a), desc(b), desc(c)
-    _check(lib().evkhip_matmul(_ref(da), _ref(db), _ref(dc), int(transpose_a), int(transpose_b),
+    _check(_calls.evkhip_matmul(_D(a), _D(b), _D(c), int(transpose_a), int(transpose_b),
                                int(acc_c), int(TILE_M), int(TILE_N), _stream(stream)))
     return c
 
@@ -229,167 +266,161 @@ def flash_attention(q, k, v, o, causal=False, lse=None, stream=None):
 
     q, o: (B, N, H*Dh) fp16; k, v: (B, N, Dh) fp16; lse: optional (B, H, N) fp32.
     """
-    dq, dk, dv, do = desc(q), desc(k), desc(v), desc(o)
     lp = None
     if lse is not None:
         if not lse.is_contiguous():
             raise ValueError("lse must be contiguous")
         lp = C.c_void_p(lse.data_ptr())
-    _check(lib().evkhip_flash_attention(_ref(dq), _ref(dk), _ref(dv), _ref(do), int(causal), lp,
+    _check(_calls.evkhip_flash_attention(_D(q), _D(k), _D(v), _D(o), int(causal), lp,
                                         _stream(stream)))
     return o
 
 
 def flash_attention_bwd(q, k, v, o, dO, dQ, dK, dV, heads=0, causal=False, lse=None, stream=None):
     """evk::ai::flash_attention_bwd (evk_ai.h:503) + causal/LSE extensions."""
-    ds = [desc(t) for t in (q, k, v, o, dO, dQ, dK, dV)]
     lp = C.c_void_p(lse.data_ptr()) if lse is not None else None
-    _check(lib().evkhip_flash_attention_bwd(*[_ref(d) for d in ds], int(heads), int(causal), lp,
+    _check(_calls.evkhip_flash_attention_bwd(*[_D(t) for t in (q, k, v, o, dO, dQ, dK, dV)], int(heads), int(causal), lp,
                                             _stream(stream)))
 
 
 def single_query_attention(q, k_cache, v_cache, out, current_length, heads=1, stream=None):
     """Decode-step attention (single_query_attention.comp, generalised)."""
-    _check(lib().evkhip_single_query_attention(_ref(desc(q)), _ref(desc(k_cache)),
-                                               _ref(desc(v_cache)), _ref(desc(out)),
+    _check(_calls.evkhip_single_query_attention(_D(q), _D(k_cache),
+                                               _D(v_cache), _D(out),
                                                int(current_length), int(heads), _stream(stream)))
     return out
 
 
 def kv_cache_write(src, cache, pos0, stream=None):
     """Rows [pos0, pos0+n) of each sequence's cache (B, max_seq, D) <- src (B, n, D)."""
-    _check(lib().evkhip_kv_cache_write(_ref(desc(src)), _ref(desc(cache)), int(pos0), _stream(stream)))
+    _check(_calls.evkhip_kv_cache_write(_D(src), _D(cache), int(pos0), _stream(stream)))
 
 
 def rms_norm(inp, out, eps=1e-4, stream=None):
-    _check(lib().evkhip_rms_norm(_ref(desc(inp)), _ref(desc(out)), float(eps), _stream(stream)))
+    _check(_calls.evkhip_rms_norm(_D(inp), _D(out), float(eps), _stream(stream)))
     return out
 
 
 def rope(inp, out, batch_size, seq_len, embed_dim, rotary_base=10000.0, position_offset=0,
          head_dim=0, stream=None):
-    _check(lib().evkhip_rope(_ref(desc(inp)), _ref(desc(out)), int(batch_size), int(seq_len),
+    _check(_calls.evkhip_rope(_D(inp), _D(out), int(batch_size), int(seq_len),
                              int(embed_dim), float(rotary_base), int(position_offset),
                              int(head_dim), _stream(stream)))
     return out
 
 
 def gelu(inp, out, stream=None):
-    _check(lib().evkhip_gelu(_ref(desc(inp)), _ref(desc(out)), _stream(stream)))
+    _check(_calls.evkhip_gelu(_D(inp), _D(out), _stream(stream)))
     return out
 
 
 def add(a, b, c, stream=None):
-    _check(lib().evkhip_add(_ref(desc(a)), _ref(desc(b)), _ref(desc(c)), _stream(stream)))
+    _check(_calls.evkhip_add(_D(a), _D(b), _D(c), _stream(stream)))
     return c
 
 
 def embed(embeddings, indices, out, stream=None):
-    _check(lib().evkhip_embed(_ref(desc(embeddings)), _ref(desc(indices)), _ref(desc(out)),
+    _check(_calls.evkhip_embed(_D(embeddings), _D(indices), _D(out),
                               _stream(stream)))
     return out
 
 
 # ---- training ops (evk_ai.h:507-614); *_backward accumulate into grad_in ----
 
-def _D(t):
-    return _ref(desc(t))
-
-
 def scale(t, factor, stream=None):
-    _check(lib().evkhip_scale(_D(t), float(factor), _stream(stream)))
+    _check(_calls.evkhip_scale(_D(t), float(factor), _stream(stream)))
     return t
 
 
 def relu(inp, out, stream=None):
-    _check(lib().evkhip_relu(_D(inp), _D(out), _stream(stream)))
+    _check(_calls.evkhip_relu(_D(inp), _D(out), _stream(stream)))
     return out
 
 
 def relu_backward(grad_out, inp, grad_in, stream=None):
-    _check(lib().evkhip_relu_backward(_D(grad_out), _D(inp), _D(grad_in), _stream(stream)))
+    _check(_calls.evkhip_relu_backward(_D(grad_out), _D(inp), _D(grad_in), _stream(stream)))
     return grad_in
 
 
 def gelu_backward(grad_out, inp, grad_in, stream=None):
-    _check(lib().evkhip_gelu_backward(_D(grad_out), _D(inp), _D(grad_in), _stream(stream)))
+    _check(_calls.evkhip_gelu_backward(_D(grad_out), _D(inp), _D(grad_in), _stream(stream)))
     return grad_in
 
 
 def mse_loss(predicted, target, pred_grad, result, stream=None):
-    _check(lib().evkhip_mse_loss(_D(predicted), _D(target), _D(pred_grad), _D(result), _stream(stream)))
+    _check(_calls.evkhip_mse_loss(_D(predicted), _D(target), _D(pred_grad), _D(result), _stream(stream)))
     return result
 
 
 def sgd(param, gradient, learning_rate, stream=None):
-    _check(lib().evkhip_sgd(_D(param), _D(gradient), float(learning_rate), _stream(stream)))
+    _check(_calls.evkhip_sgd(_D(param), _D(gradient), float(learning_rate), _stream(stream)))
     return param
 
 
 def adam(param, gradient, m_state, v_state, learning_rate, beta1, beta2, beta1_correction_inv,
          beta2_correction_inv, epsilon, stream=None):
-    _check(lib().evkhip_adam(_D(param), _D(gradient), _D(m_state), _D(v_state), float(learning_rate),
+    _check(_calls.evkhip_adam(_D(param), _D(gradient), _D(m_state), _D(v_state), float(learning_rate),
                              float(beta1), float(beta2), float(beta1_correction_inv),
                              float(beta2_correction_inv), float(epsilon), _stream(stream)))
     return param
 
 
 def softmax(inp, out, input_scale=1.0, stream=None):
-    _check(lib().evkhip_softmax(_D(inp), _D(out), float(input_scale), _stream(stream)))
+    _check(_calls.evkhip_softmax(_D(inp), _D(out), float(input_scale), _stream(stream)))
     return out
 
 
 def softmax_backward(probs, grad_out, grad_in, scale=1.0, stream=None):
-    _check(lib().evkhip_softmax_backward(_D(probs), _D(grad_out), _D(grad_in), float(scale),
+    _check(_calls.evkhip_softmax_backward(_D(probs), _D(grad_out), _D(grad_in), float(scale),
                                          _stream(stream)))
     return grad_in
 
 
 def rms_norm_backward(inp, grad_out, grad_in, eps=1e-4, stream=None):
-    _check(lib().evkhip_rms_norm_backward(_D(inp), _D(grad_out), _D(grad_in), float(eps), _stream(stream)))
+    _check(_calls.evkhip_rms_norm_backward(_D(inp), _D(grad_out), _D(grad_in), float(eps), _stream(stream)))
     return grad_in
 
 
 def cross_entropy_loss(logits, targets, grad, result, stream=None):
-    _check(lib().evkhip_cross_entropy_loss(_D(logits), _D(targets), _D(grad), _D(result), _stream(stream)))
+    _check(_calls.evkhip_cross_entropy_loss(_D(logits), _D(targets), _D(grad), _D(result), _stream(stream)))
     return result
 
 
 def sum_batch(inp, out, batch_count, size_per_batch, stream=None):
-    _check(lib().evkhip_sum_batch(_D(inp), _D(out), int(batch_count), int(size_per_batch), _stream(stream)))
+    _check(_calls.evkhip_sum_batch(_D(inp), _D(out), int(batch_count), int(size_per_batch), _stream(stream)))
     return out
 
 
 def apply_causal_mask(scores, stream=None):
-    _check(lib().evkhip_apply_causal_mask(_D(scores), _stream(stream)))
+    _check(_calls.evkhip_apply_causal_mask(_D(scores), _stream(stream)))
     return scores
 
 
 def position_add(inp, pos_emb, out, batch_size, seq_len, embed_dim, stream=None):
-    _check(lib().evkhip_position_add(_D(inp), _D(pos_emb), _D(out), int(batch_size), int(seq_len),
+    _check(_calls.evkhip_position_add(_D(inp), _D(pos_emb), _D(out), int(batch_size), int(seq_len),
                                      int(embed_dim), _stream(stream)))
     return out
 
 
 def position_add_backward(grad_out, grad_in, grad_pos, batch_size, seq_len, embed_dim, stream=None):
-    _check(lib().evkhip_position_add_backward(_D(grad_out), _D(grad_in), _D(grad_pos), int(batch_size),
+    _check(_calls.evkhip_position_add_backward(_D(grad_out), _D(grad_in), _D(grad_pos), int(batch_size),
                                               int(seq_len), int(embed_dim), _stream(stream)))
     return grad_in, grad_pos
 
 
 def rope_backward(grad_out, grad_in, batch_size, seq_len, embed_dim, rotary_base=10000.0, stream=None):
-    _check(lib().evkhip_rope_backward(_D(grad_out), _D(grad_in), int(batch_size), int(seq_len),
+    _check(_calls.evkhip_rope_backward(_D(grad_out), _D(grad_in), int(batch_size), int(seq_len),
                                       int(embed_dim), float(rotary_base), _stream(stream)))
     return grad_in
 
 
 def embed_backward(grad_out, indices, grad_embeddings, stream=None):
-    _check(lib().evkhip_embed_backward(_D(grad_out), _D(indices), _D(grad_embeddings), _stream(stream)))
+    _check(_calls.evkhip_embed_backward(_D(grad_out), _D(indices), _D(grad_embeddings), _stream(stream)))
     return grad_embeddings
 
 
 def greedy_sample(logits, out_tokens, position, token_base, token_count, stream=None):
-    _check(lib().evkhip_greedy_sample(_ref(desc(logits)), _ref(desc(out_tokens)), int(position),
+    _check(_calls.evkhip_greedy_sample(_D(logits), _D(out_tokens), int(position),
                                       int(token_base), int(token_count), _stream(stream)))
     return out_tokens
 

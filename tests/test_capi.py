@@ -189,3 +189,19 @@ def test_model_validation(L):
     bad = evk_amd.ModelCfg(32000, 768, 12, 60, 12, 3072, 1056, 1e-4, 1e4)  # heads*dh != d
     assert L.evkhip_model_decode(C.byref(bad), p, p, p, 1, 0, p, None) == SHAPE
     assert L.evkhip_model_prefill(C.byref(cfg), p, p, None, 4, 0, p, p, None) == INVALID
+
+
+def test_packed_descriptors():
+    """The descriptors the wrappers pass are those that desc() builds, for
+    every rank, and what desc() refuses is refused."""
+    import torch
+
+    import evk_amd as evk
+    for rank in range(evk.MAX_DIMS + 1):
+        t = torch.empty([r + 2 for r in range(rank)][::-1], dtype=torch.float16)
+        assert evk._D(t) == bytes(evk.desc(t))
+    assert evk._D((4096, (3, 5))) == bytes(evk.desc((4096, (3, 5))))
+    with pytest.raises(ValueError):
+        evk._D(torch.empty([1] * (evk.MAX_DIMS + 1)))
+    with pytest.raises(ValueError):
+        evk._D(torch.empty(4, 6).t())
