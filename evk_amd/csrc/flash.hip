@@ -482,7 +482,8 @@ struct KsLayout {
     static constexpr int LDS_BYTES = VBYTES + MERGE * 4;
 };
 
-template <int DH, int QB, bool CAUSAL>
+// STRIDED: O rows at out_bstride / out_rstride instead of contiguous.
+template <int DH, int QB, bool CAUSAL, bool STRIDED = false>
 __global__ __launch_bounds__(512, 1) void flash_fwd_ks(FlashArgs p) {
     using L = KsLayout<DH, QB>;
     constexpr int ROWS = L::ROWS;
@@ -847,7 +848,8 @@ __global__ __launch_bounds__(512, 1) void flash_fwd_ks(FlashArgs p) {
     const int row = R0 + q;
     const float inv_l = l > 0.0f ? 1.0f / l : 0.0f;
     if (active && row < NH) {
-        f16* orow = p.out + b * p.out_bstride + (int64_t)row * p.out_rstride;
+        f16* orow = STRIDED ? p.out + b * p.out_bstride + (int64_t)row * p.out_rstride
+                            : p.out + ((int64_t)b * NH + row) * DH;
 #pragma unroll
         for (int d = 0; d < DB; ++d) {
             const uint2 o = {pack_h2(a[d][0] * inv_l, a[d][1] * inv_l), pack_h2(a[d][2] * inv_l, a[d][3] * inv_l)};
@@ -861,7 +863,7 @@ __global__ __launch_bounds__(512, 1) void flash_fwd_ks(FlashArgs p) {
 }
 
 // ---------------------------------------------------------------------------
-// Backward dK, dV for head dims 32, 64 and 128.
+// Backward dK, dV for head dims 32 and 64 (128: bwd_kv_pair_body).
 //
 // Workgroup: 4 waves and 128 keys; wave w owns keys [32w, 32w+32) of the
 // block, with K^T and V^T as B-operand registers for the whole kernel.  The
@@ -875,7 +877,7 @@ __global__ __launch_bounds__(512, 1) void flash_fwd_ks(FlashArgs p) {
 //   dV += P^T dO, dK += dS^T Q: the probabilities of two 16-row blocks are
 //       the A operand as they are (slot s <-> row 4g+s, 16+4g+s-4), and dO, Q
 //       come transposed from the LDS chunk through ds_read_b64_tr_b16.
-// The query rows of a key block are split into parts of at most PART_CHUNKS
+// The query rows of a key block are split into parts of at most 2^part_log2
 // chunks, one part per workgroup, so that causal key blocks near the start
 // (which see every row) do not serialise the grid.  A key block with one
 // part writes dK, dV directly; otherwise every part stores an fp32 partial
@@ -890,18 +892,47 @@ DEV float dot8(const half8& x, const half8& y) {
     for (int e = 0; e < 8; ++e) acc = __builtin_fmaf((float)x[e], (float)y[e], acc);
     return acc;
 }
+// the same on v_dot2_f32_f16 (products and sums in fp32): 4 instructions
+// instead of 24
+DEV float dot8_pairs(const half8& x, const half8& y) {
+    float acc = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 8; e += 2)
+        acc = __builtin_amdgcn_fdot2(half2_t{x[e], x[e + 1]}, half2_t{y[e], y[e + 1]}, acc, false);
+    return acc;
+}
+
+// v += v of the lane that DPP control CTRL names (0xB1, 0x4E: lanes 1 and 2
+// apart in a quad; 0x141: the mirrored lane of 8; 0x140: of 16)
+template <int CTRL>
+DEV void dpp_add(float& v) {
+    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
+}
 
 constexpr int BKB = 128;       // keys per workgroup (4 waves x 32)
 constexpr int BRC = 32;        // flattened query rows per chunk
-constexpr int PART_CHUNKS = 16;
+// Chunks per row part, as a power of two: as long as leaves about 128 parts
+// (fewer fp32 partials to write and read) and short enough that a small call
+// still spreads over the chip.  Head sizes up to 64 stop at 16: two workgroups
+// share a CU there, and longer parts lengthen the launch.  Forward and
+// backward, us with this rule and with parts of 16 throughout: Dh 128, B=2
+// N=2000 H=8 163 and 177, B=16 N=160 H=4 27.5 and 40.1, B=1 N=130 H=2 22.3
+// and 26.6; Dh 64, B=1 N=600 H=4 24.5 and 33.7, B=16 N=160 H=4 20.9 and 32.3;
+// Dh 32, B=1 N=888 H=1 19.9 and 27.7.
+inline int bwd_part_log2(int dh, int64_t chunks) {
+    const int most = dh <= 64 ? 4 : 6;
+    int l = 2;
+    while (l < most && (chunks >> (l + 1)) >= 96) ++l;
+    return l;
+}
 
 // Chunks of flattened rows that key block kb of a batch interacts with.
 __host__ __device__ inline int bwd_kv_chunks(int kb, int N, int H, bool causal) {
     const int64_t r_lo = causal ? (int64_t)kb * BKB * H : 0;
     return (int)(((int64_t)N * H - r_lo + BRC - 1) / BRC);
 }
-__host__ __device__ inline int bwd_kv_parts(int kb, int N, int H, bool causal) {
-    return (bwd_kv_chunks(kb, N, H, causal) + PART_CHUNKS - 1) / PART_CHUNKS;
+__host__ __device__ inline int bwd_kv_parts(int kb, int N, int H, bool causal, int part_log2) {
+    return (bwd_kv_chunks(kb, N, H, causal) + (1 << part_log2) - 1) >> part_log2;
 }
 
 template <int DH>
@@ -915,7 +946,7 @@ struct KvLayout {
     static constexpr int LDS_BYTES = CHUNK_BYTES + STATS_BYTES + 2 * BRC * 4;
 };
 
-template <int DH, bool CAUSAL>
+template <int DH, bool CAUSAL, int PL>
 DEV void bwd_kv_body(const FlashArgs& p, float* part_ws, int parts_per_batch, int blk, char* lds) {
     using L = KvLayout<DH>;
     constexpr int KS = DH / 32, DB = DH / 16, RW = L::RW;
@@ -926,19 +957,20 @@ DEV void bwd_kv_body(const FlashArgs& p, float* part_ws, int parts_per_batch, in
     int* pos_s = reinterpret_cast<int*>(lds + L::CHUNK_BYTES + L::STATS_BYTES);  // position of each row
 
     const int H = p.H, N = p.N, NH = N * H;
+    const int part_log2 = PL > 0 ? PL : p.part_log2;
     const int nkb = (N + BKB - 1) / BKB;
     // workgroup -> (batch, key block, part); heavy key blocks first
     const int b = blk / parts_per_batch;
     int rem = blk % parts_per_batch, kb = 0, nparts = 0, slot0 = 0;
     for (; kb < nkb; ++kb) {
-        nparts = bwd_kv_parts(kb, N, H, CAUSAL);
+        nparts = bwd_kv_parts(kb, N, H, CAUSAL, part_log2);
         if (rem < nparts) break;
         rem -= nparts;
         slot0 += nparts;
     }
     const int part = rem;
     const int nch_all = bwd_kv_chunks(kb, N, H, CAUSAL);
-    const int c_lo = part * PART_CHUNKS, c_hi = min(nch_all, c_lo + PART_CHUNKS);
+    const int c_lo = part << part_log2, c_hi = min(nch_all, c_lo + (1 << part_log2));
     const int r_lo = CAUSAL ? kb * BKB * H : 0;
 
     const int lane = threadIdx.x & 63;
@@ -974,12 +1006,11 @@ DEV void bwd_kv_body(const FlashArgs& p, float* part_ws, int parts_per_batch, in
     const __amdgpu_buffer_rsrc_t gres = buf_rsrc(p.dO + (int64_t)b * NH * DH, (uint32_t)NH * DH * 2);
     const __amdgpu_buffer_rsrc_t ores = buf_rsrc(p.o + (int64_t)b * NH * DH, (uint32_t)NH * DH * 2);
     const __amdgpu_buffer_rsrc_t lres = buf_rsrc(p.lse + (int64_t)b * H * N, (uint32_t)(H * N) * 4u);
-    // With each dO piece a thread holds the O piece at the same place, so
-    // that D = rowsum(dO * O) comes from the DH/8 lanes of a row.  Rows past
-    // NH read as zeros: D = 0, lse2 = 0 (their Q and dO rows are zero too, so
-    // they add nothing).
-    constexpr int OPT = PIECES >= 256 ? PIECES / 256 : 1;  // dO pieces per thread
-    u32x4 pr[PPT], po[OPT] = {};
+    // A thread holds at most one dO piece (DH <= 64); with it the O piece at
+    // the same place, so that D = rowsum(dO * O) comes from the DH/8 lanes
+    // of a row.  Rows past NH read as zeros: D = 0, lse2 = 0 (their Q and
+    // dO rows are zero too, so they add nothing).
+    u32x4 pr[PPT], po = {0u, 0u, 0u, 0u};
     float sr = 0.0f;
     int spos = 0;
     // Row (position, head) of thread t's statistics row (t mod BRC), advanced
@@ -1010,7 +1041,7 @@ DEV void bwd_kv_body(const FlashArgs& p, float* part_ws, int parts_per_batch, in
             if (2 * PIECES % 256 == 0 || pc < 2 * PIECES) {
                 if (which) {
                     pr[i] = buf_load16(gres, off, 0);
-                    po[i % OPT] = buf_load16(ores, off, 0);
+                    po = buf_load16(ores, off, 0);
                 } else {
                     pr[i] = buf_load16(qres, off, 0);
                 }
@@ -1033,36 +1064,27 @@ DEV void bwd_kv_body(const FlashArgs& p, float* part_ws, int parts_per_batch, in
     };
     auto lstore = [&](int stage) {
         f16* cs = chunk_s + stage * L::STAGE;
-        float dsum[OPT] = {};
+        float dsum = 0.0f;
 #pragma unroll
         for (int i = 0; i < PPT; ++i) {
             const int pc = threadIdx.x + 256 * i;
             const int which = __builtin_amdgcn_readfirstlane(pc / PIECES), pi = pc % PIECES;
             if (2 * PIECES % 256 == 0 || pc < 2 * PIECES) {
                 *reinterpret_cast<u32x4*>(cs + which * L::CHUNK + (pi / (DH / 8)) * RW + (pi % (DH / 8)) * 8) = pr[i];
-                if (which) dsum[i % OPT] = dot8(as_half8(pr[i]), as_half8(po[i % OPT]));
+                if (which) dsum = dot8(as_half8(pr[i]), as_half8(po));
             }
         }
-        // the DH/8 lanes of a row are adjacent (a quad, a half row or a row of
-        // 16 lanes): DPP sums
-        auto dpp_add = [](float& v, auto ctrl) {
-            v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), decltype(ctrl)::value,
-                                                                       0xF, 0xF, false));
-        };
-        static_assert(DH / 8 <= 16, "a row's lanes within 16 lanes");
-#pragma unroll
-        for (int o = 0; o < OPT; ++o) {
-            dpp_add(dsum[o], std::integral_constant<int, 0xB1>{});
-            if (DH / 8 >= 4) dpp_add(dsum[o], std::integral_constant<int, 0x4E>{});
-            if (DH / 8 >= 8) dpp_add(dsum[o], std::integral_constant<int, 0x141>{});
-            if (DH / 8 >= 16) dpp_add(dsum[o], std::integral_constant<int, 0x140>{});
-        }
+        // the DH/8 lanes of a row are adjacent (a quad or two): DPP sums
+        static_assert(DH / 8 <= 8, "a row's lanes within a half row");
+        dpp_add<0xB1>(dsum);
+        if (DH / 8 >= 4) dpp_add<0x4E>(dsum);
+        if (DH / 8 >= 8) dpp_add<0x141>(dsum);
 #pragma unroll
         for (int i = 0; i < PPT; ++i) {
             const int pc = threadIdx.x + 256 * i;
             const int pi = pc % PIECES;
             if (pc >= PIECES && pc < 2 * PIECES && pi % (DH / 8) == 0)
-                stats_s[stage * L::STATS + BRC + pi / (DH / 8)] = dsum[i % OPT];
+                stats_s[stage * L::STATS + BRC + pi / (DH / 8)] = dsum;
         }
         const float l2 = sr * kLog2e;  // base-2 LSE
         if (threadIdx.x < BRC) stats_s[stage * L::STATS + threadIdx.x] = l2;
@@ -1203,19 +1225,270 @@ DEV void bwd_kv_body(const FlashArgs& p, float* part_ws, int parts_per_batch, in
         }
 }
 
+// The same part for head size 128 on 8 waves (two per SIMD within 256
+// registers).  Waves w and w + 4 share keys [32 (w % 4), +32): each contracts S
+// and dP for one 16-row block of the chunk (half w / 4) and accumulates dK, dV
+// for one half of Dh.  The probabilities of the other row block come through
+// LDS: they are written in iteration c and multiplied in iteration c + 1, so
+// an iteration holds the score products of one chunk and the gradient
+// products of the one before, which do not depend on each other, and needs
+// one barrier.  Three LDS stages (chunk c + 1 arrives, c is scored, c - 1 is
+// multiplied).
+template <int DH>
+struct KvPairLayout {
+    static constexpr int RW = DH + 8;
+    static constexpr int CHUNK = BRC * RW, STAGE = 2 * CHUNK;  // halves: Q, then dO
+    static constexpr int STATS = 2 * BRC;                      // floats: lse2, D per row
+    static constexpr int STATS_AT = 3 * STAGE * 2, POS_AT = STATS_AT + 3 * STATS * 4, X_AT = POS_AT + 3 * BRC * 4;
+    static constexpr int XW = 8 * 4 * 64;  // half4 of one exchange buffer: [wave][P k2 | dS k2][lane]
+    static constexpr int LDS_BYTES = X_AT + 2 * XW * 8;
+};
+
+template <int DH, bool CAUSAL>
+DEV void bwd_kv_pair_body(const FlashArgs& p, float* part_ws, int parts_per_batch, int blk, char* lds) {
+    using L = KvPairLayout<DH>;
+    constexpr int KS = DH / 32, DB = DH / 16, DW = DB / 2, RW = L::RW, NT = 512;
+    static_assert(BRC * DH / 8 == NT, "one Q and one dO piece per thread");
+    f16* chunk_s = reinterpret_cast<f16*>(lds);
+    float* stats_s = reinterpret_cast<float*>(lds + L::STATS_AT);
+    int* pos_s = reinterpret_cast<int*>(lds + L::POS_AT);
+    half4* x_s = reinterpret_cast<half4*>(lds + L::X_AT);
+
+    const int H = p.H, N = p.N, NH = N * H;
+    const int nkb = (N + BKB - 1) / BKB;
+    const int b = blk / parts_per_batch;
+    int rem = blk % parts_per_batch, kb = 0, nparts = 0, slot0 = 0;
+    for (; kb < nkb; ++kb) {
+        nparts = bwd_kv_parts(kb, N, H, CAUSAL, p.part_log2);
+        if (rem < nparts) break;
+        rem -= nparts;
+        slot0 += nparts;
+    }
+    const int part = rem;
+    const int nch_all = bwd_kv_chunks(kb, N, H, CAUSAL);
+    const int c_lo = part << p.part_log2, c_hi = min(nch_all, c_lo + (1 << p.part_log2));
+    const int r_lo = CAUSAL ? kb * BKB * H : 0;
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kp = wave & 3, hf = wave >> 2;
+    const int l16 = lane & 15, g = lane >> 4, trow = l16 >> 2, tcol = (l16 & 3) * 4;
+    const int k0 = kb * BKB + kp * 32;
+    const float c2 = p.scale_log2;
+
+    const __amdgpu_buffer_rsrc_t kres = buf_rsrc(p.k + (int64_t)b * N * DH, (uint32_t)N * DH * 2);
+    const __amdgpu_buffer_rsrc_t vres = buf_rsrc(p.v + (int64_t)b * N * DH, (uint32_t)N * DH * 2);
+    half8 kt[2][KS], vt[2][KS];
+#pragma unroll
+    for (int k2 = 0; k2 < 2; ++k2)
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const uint32_t off = (uint32_t)((k0 + 16 * k2 + l16) * DH + ks * 32 + g * 8) * 2;
+            kt[k2][ks] = as_half8(buf_load16(kres, off, 0));
+            vt[k2][ks] = as_half8(buf_load16(vres, off, 0));
+        }
+    floatx4 dk[2][DW], dv[2][DW];
+#pragma unroll
+    for (int k2 = 0; k2 < 2; ++k2)
+#pragma unroll
+        for (int d = 0; d < DW; ++d) {
+            dk[k2][d] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+            dv[k2][d] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+
+    // staging as in bwd_kv_body: thread t holds piece t of Q, dO and O; the
+    // statistics row t mod BRC advances without dividing
+    const __amdgpu_buffer_rsrc_t qres = buf_rsrc(p.q + (int64_t)b * NH * DH, (uint32_t)NH * DH * 2);
+    const __amdgpu_buffer_rsrc_t gres = buf_rsrc(p.dO + (int64_t)b * NH * DH, (uint32_t)NH * DH * 2);
+    const __amdgpu_buffer_rsrc_t ores = buf_rsrc(p.o + (int64_t)b * NH * DH, (uint32_t)NH * DH * 2);
+    const __amdgpu_buffer_rsrc_t lres = buf_rsrc(p.lse + (int64_t)b * H * N, (uint32_t)(H * N) * 4u);
+    u32x4 rq, rg, ro;
+    float sr = 0.0f;
+    int spos = 0;
+    const int h_step = BRC % H, p_step = BRC / H;
+    int st_head, st_pos, st_next = c_lo;
+    {
+        const int row = r_lo + c_lo * BRC + (int)(threadIdx.x % BRC);
+        st_head = row % H;
+        st_pos = row / H;
+    }
+    auto gload = [&](int c) {
+        const uint32_t row0 = (uint32_t)(r_lo + c * BRC);
+        const uint32_t off = (row0 * DH + threadIdx.x * 8) * 2;
+        rq = buf_load16(qres, off, 0);
+        rg = buf_load16(gres, off, 0);
+        ro = buf_load16(ores, off, 0);
+        for (; st_next < c; ++st_next) {
+            st_head += h_step;
+            st_pos += p_step;
+            if (st_head >= H) {
+                st_head -= H;
+                st_pos += 1;
+            }
+        }
+        sr = buf_load_f32(lres, oob_or(threadIdx.x < BRC && row0 + threadIdx.x < (uint32_t)NH,
+                                       (uint32_t)(st_head * N + st_pos) * 4u));
+        if (threadIdx.x >= BRC && threadIdx.x < 2 * BRC) spos = st_pos;
+    };
+    auto lstore = [&](int stage) {
+        f16* cs = chunk_s + stage * L::STAGE + (threadIdx.x / (DH / 8)) * RW + (threadIdx.x % (DH / 8)) * 8;
+        *reinterpret_cast<u32x4*>(cs) = rq;
+        *reinterpret_cast<u32x4*>(cs + L::CHUNK) = rg;
+        float dsum = dot8_pairs(as_half8(rg), as_half8(ro));
+        static_assert(DH / 8 == 16, "a row's pieces on 16 adjacent lanes");
+        dpp_add<0xB1>(dsum);
+        dpp_add<0x4E>(dsum);
+        dpp_add<0x141>(dsum);
+        dpp_add<0x140>(dsum);
+        if (threadIdx.x % (DH / 8) == 0) stats_s[stage * L::STATS + BRC + threadIdx.x / (DH / 8)] = dsum;
+        if (threadIdx.x < BRC) stats_s[stage * L::STATS + threadIdx.x] = sr * kLog2e;
+        else if (threadIdx.x < 2 * BRC) pos_s[stage * BRC + threadIdx.x - BRC] = spos;
+    };
+
+    if (c_lo < c_hi) {
+        gload(c_lo);
+        lstore(0);
+    }
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): in the loop only its own loads are in flight
+    __syncthreads();
+    // scores of chunk c (in stage st) into the exchange buffer c & 1; keys past
+    // a row's position or N, and rows past NH, give P = dS = 0
+    auto score = [&](int c, int st, auto masked) {
+        const f16* qs = chunk_s + st * L::STAGE + (hf * 16 + l16) * RW + g * 8;
+        const float* sts = stats_s + st * L::STATS + hf * 16 + 4 * g;
+        const floatx4 l2 = *reinterpret_cast<const floatx4*>(sts);
+        const floatx4 dd = *reinterpret_cast<const floatx4*>(sts + BRC);
+        intx4 ps = {0, 0, 0, 0};
+        if (masked) ps = *reinterpret_cast<const intx4*>(pos_s + st * BRC + hf * 16 + 4 * g);
+        floatx4 s[2], dp[2];
+        {
+            half8 qa[KS], ga[KS];
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+                qa[ks] = *reinterpret_cast<const half8*>(qs + ks * 32);
+                ga[ks] = *reinterpret_cast<const half8*>(qs + L::CHUNK + ks * 32);
+            }
+#pragma unroll
+            for (int k2 = 0; k2 < 2; ++k2) {
+                s[k2] = mfma16(qa[0], kt[k2][0], floatx4{0.0f, 0.0f, 0.0f, 0.0f});
+                dp[k2] = mfma16(ga[0], vt[k2][0], floatx4{0.0f, 0.0f, 0.0f, 0.0f});
+#pragma unroll
+                for (int ks = 1; ks < KS; ++ks) {
+                    s[k2] = mfma16(qa[ks], kt[k2][ks], s[k2]);
+                    dp[k2] = mfma16(ga[ks], vt[k2][ks], dp[k2]);
+                }
+            }
+        }
+        // element j of s[k2]: row row0 + 16 hf + 4 g + j, key k0 + 16 k2 + l16
+        half4* x = x_s + (c & 1) * L::XW + wave * 4 * 64 + lane;
+#pragma unroll
+        for (int k2 = 0; k2 < 2; ++k2) {
+            const int key = k0 + 16 * k2 + l16;
+            float pv[4], dsv[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                float pe = fast_exp2(__builtin_fmaf(s[k2][j], c2, -l2[j]));
+                if (masked && ((CAUSAL && key > ps[j]) || key >= N)) pe = 0.0f;
+                pv[j] = pe;
+                dsv[j] = pe * (dp[k2][j] - dd[j]);
+            }
+            x[k2 * 64] = half4{(f16)pv[0], (f16)pv[1], (f16)pv[2], (f16)pv[3]};
+            x[(2 + k2) * 64] = half4{(f16)dsv[0], (f16)dsv[1], (f16)dsv[2], (f16)dsv[3]};
+        }
+    };
+    // dV, dK of chunk c
+    auto multiply = [&](int c, int st) {
+        const half4* x = x_s + (c & 1) * L::XW + kp * 4 * 64 + lane;
+        half8 pa[2], da[2];  // slots: row 4 g + s of block 0, then of block 1
+#pragma unroll
+        for (int k2 = 0; k2 < 2; ++k2) {
+            pa[k2] = cat4(x[k2 * 64], x[(16 + k2) * 64]);
+            da[k2] = cat4(x[(2 + k2) * 64], x[(18 + k2) * 64]);
+        }
+        const f16* qp = chunk_s + st * L::STAGE + (g * 4 + trow) * RW + hf * (DH / 2) + tcol;
+#pragma unroll
+        for (int d = 0; d < DW; ++d) {
+            const f16* qb = qp + d * 16;
+            const f16* gb = qb + L::CHUNK;
+            const half8 gt = cat4(lds_read_tr(gb), lds_read_tr(gb + 16 * RW));
+            const half8 qt = cat4(lds_read_tr(qb), lds_read_tr(qb + 16 * RW));
+#pragma unroll
+            for (int k2 = 0; k2 < 2; ++k2) {
+                dv[k2][d] = mfma16(pa[k2], gt, dv[k2][d]);
+                dk[k2][d] = mfma16(da[k2], qt, dk[k2][d]);
+            }
+        }
+    };
+    auto next = [](int st) { return st == 2 ? 0 : st + 1; };
+    // scores one chunk ahead of the products, in one straight-line block, so
+    // that each one's LDS and MFMA latency hides behind the other
+    int st = 0;
+    if (c_lo < c_hi) {
+        gload(c_lo + 1);
+        score(c_lo, 0, std::true_type{});
+        lstore(1);
+    }
+    __syncthreads();
+    // chunks from c_free on hold no position before the workgroup's last key
+    // (and all keys exist): nothing is masked in them
+    const int c_free = (kb + 1) * BKB > N ? c_hi : !CAUSAL ? 0 : ((kb + 1) * BKB * H - r_lo + BRC - 1) / BRC;
+    auto both = [&](int c, auto masked) {
+        gload(c + 1);  // past the part: staged where nothing reads
+        const int sc = next(st);
+        multiply(c - 1, st);  // first: it writes no LDS, so the scores' reads may move above it
+        score(c, sc, masked);
+        lstore(next(sc));
+        st = sc;
+        __syncthreads();
+    };
+    int c = c_lo + 1;
+    for (; c < min(c_hi, c_free); ++c) both(c, std::true_type{});
+    for (; c < c_hi; ++c) both(c, std::false_type{});
+    if (c_lo < c_hi) multiply(c_hi - 1, st);
+
+    // element j of dk[k2][d]: key k0 + 16 k2 + 4 g + j, dh 16 (DW hf + d) + l16
+    if (nparts == 1) {
+#pragma unroll
+        for (int k2 = 0; k2 < 2; ++k2)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int key = k0 + 16 * k2 + 4 * g + j;
+                if (key >= N) continue;
+                const int64_t at = ((int64_t)b * N + key) * DH + hf * (DH / 2) + l16;
+#pragma unroll
+                for (int d = 0; d < DW; ++d) {
+                    p.dK[at + d * 16] = (f16)(dk[k2][d][j] * p.scale);
+                    p.dV[at + d * 16] = (f16)dv[k2][d][j];
+                }
+            }
+        return;
+    }
+    // fp32 partial in bwd_kv_body's layout: [slot][key wave][dk|dv][k2][d][lane]
+    constexpr int PW = 2 * 2 * DB;
+    const int64_t slot = (int64_t)b * parts_per_batch + slot0 + part;
+    floatx4* mine = reinterpret_cast<floatx4*>(part_ws) + (slot * 4 + kp) * PW * 64;
+#pragma unroll
+    for (int k2 = 0; k2 < 2; ++k2)
+#pragma unroll
+        for (int d = 0; d < DW; ++d) {
+            __builtin_nontemporal_store(dk[k2][d], mine + ((0 * 2 + k2) * DB + hf * DW + d) * 64 + lane);
+            __builtin_nontemporal_store(dv[k2][d], mine + ((1 * 2 + k2) * DB + hf * DW + d) * 64 + lane);
+        }
+}
+
 // Sums the fp32 partials of key blocks with several row parts, in part
 // order, and writes dK (times the softmax scale) and dV.  Grid: one
 // workgroup per (batch, key block) x 16 slices of its 4096 floatx4.
-template <int DH, bool CAUSAL>
+template <int DH, bool CAUSAL, int PL>
 __global__ __launch_bounds__(256) void flash_bwd_kv_reduce(FlashArgs p, const float* part_ws, int parts_per_batch) {
     constexpr int DB = DH / 16, PW = 2 * 2 * DB, SLOT = 4 * PW * 64;  // floatx4 per slot
-    const int N = p.N, H = p.H;
+    const int N = p.N, H = p.H, part_log2 = PL > 0 ? PL : p.part_log2;
     const int nkb = (N + BKB - 1) / BKB;
     const int bk = blockIdx.x / 16, slice = blockIdx.x % 16;
     const int b = bk / nkb, kb = bk % nkb;
     int slot0 = 0;
-    for (int k = 0; k < kb; ++k) slot0 += bwd_kv_parts(k, N, H, CAUSAL);
-    const int nparts = bwd_kv_parts(kb, N, H, CAUSAL);
+    for (int k = 0; k < kb; ++k) slot0 += bwd_kv_parts(k, N, H, CAUSAL, part_log2);
+    const int nparts = bwd_kv_parts(kb, N, H, CAUSAL, part_log2);
     if (nparts == 1) return;  // written directly by its only part
     for (int e = slice * 256 + threadIdx.x; e < SLOT; e += 16 * 256) {
         const floatx4* src = reinterpret_cast<const floatx4*>(part_ws) + ((int64_t)b * parts_per_batch + slot0) * SLOT + e;
@@ -1247,7 +1520,7 @@ __global__ __launch_bounds__(256) void flash_bwd_kv_reduce(FlashArgs p, const fl
 }
 
 // ---------------------------------------------------------------------------
-// Backward dQ for head dims 32, 64 and 128: the key-split forward's structure
+// Backward dQ for head dims 32 and 64 (128: bwd_q_pair_body): the key-split forward's structure
 // without the online softmax (P comes from the saved row statistics).
 // Workgroup: 64 flattened query rows, 4 waves; wave w takes 32-key chunks
 // w, w+4, ... for all 64 rows:
@@ -1433,22 +1706,200 @@ DEV void bwd_q_body(const FlashArgs& p, int blk, char* lds) {
     }
 }
 
+// The same tile for head size 128 on 8 waves: wave w takes key chunks w % 4,
+// w % 4 + 4, ... for 32 of the tile's 64 rows (half w / 4), which fits two
+// waves on a SIMD.  The next chunk's K is requested once the current one is
+// in its LDS slot, the next V once the scores have read the current one.
+template <int DH>
+struct DqPairLayout {
+    static constexpr int QB = 2;                  // 16-row blocks per wave
+    static constexpr int KW = DH + 8, KSLOT = KC * KW;
+    static constexpr int OW = DH + 4, MERGE = 4 * 64 * OW;
+    static constexpr int LDS_BYTES = (MERGE * 4 > 8 * KSLOT * 2) ? MERGE * 4 : 8 * KSLOT * 2;
+};
+
+template <int DH, bool CAUSAL>
+DEV void bwd_q_pair_body(const FlashArgs& p, int blk, char* lds) {
+    using L = DqPairLayout<DH>;
+    constexpr int KS = DH / 32, DB = DH / 16, KW = L::KW, OW = L::OW, QB = L::QB;
+    constexpr int KPER = KC * DH / 8 / 64;  // 16-byte K pieces per lane
+    float* smem_f = reinterpret_cast<float*>(lds);
+    f16* kslot = reinterpret_cast<f16*>(smem_f) + (threadIdx.x >> 6) * L::KSLOT;
+
+    const int H = p.H, N = p.N, NH = N * H;
+    const int nrg = (NH + 63) / 64;
+    const int b = blk % p.B;
+    const int rg = CAUSAL ? nrg - 1 - blk / p.B : blk / p.B;  // heavy rows first
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kw = wave & 3, l16 = lane & 15, g = lane >> 4;
+    const int T0 = rg * 64, R0 = T0 + (wave >> 2) * 32;  // the tile's and the wave's first row
+    const int last = min(R0 + 31, NH - 1);               // R0 > last: no rows
+    const int pmin = R0 / H, pmax = last / H;
+    const int kend = R0 > last ? 0 : CAUSAL ? min(N, pmax + 1) : N;
+    const int nch = (kend + KC - 1) / KC;
+    const float c2 = p.scale_log2;
+
+    const f16* kb_ptr = p.k + (int64_t)b * N * DH;
+    const f16* vb_ptr = p.v + (int64_t)b * N * DH;
+    const uint32_t rows_bytes = (uint32_t)(min(T0 + 63, NH - 1) - T0 + 1) * DH * 2;
+    const __amdgpu_buffer_rsrc_t qres = buf_rsrc(p.q + ((int64_t)b * NH + T0) * DH, rows_bytes);
+    const __amdgpu_buffer_rsrc_t gres = buf_rsrc(p.dO + ((int64_t)b * NH + T0) * DH, rows_bytes);
+    const __amdgpu_buffer_rsrc_t ores = buf_rsrc(p.o + ((int64_t)b * NH + T0) * DH, rows_bytes);
+
+    half8 qf[QB][KS], gf[QB][KS];
+    float l2[QB], dd[QB];
+    int qpos[QB];
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) {
+        const int row = min(R0 + qb * 16 + l16, NH - 1);
+        qpos[qb] = row / H;
+        l2[qb] = p.lse[((int64_t)b * H + row % H) * N + row / H] * kLog2e;
+        float dsum = 0.0f;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const uint32_t off = (uint32_t)((R0 - T0 + qb * 16 + l16) * DH + ks * 32 + g * 8) * 2;
+            qf[qb][ks] = as_half8(buf_load16(qres, off, 0));
+            gf[qb][ks] = as_half8(buf_load16(gres, off, 0));
+            dsum += dot8(gf[qb][ks], as_half8(buf_load16(ores, off, 0)));
+        }
+        dsum += __shfl_xor(dsum, 16, 64);
+        dd[qb] = dsum + __shfl_xor(dsum, 32, 64);
+    }
+    floatx4 acc[DB][QB];
+#pragma unroll
+    for (int d = 0; d < DB; ++d)
+#pragma unroll
+        for (int qb = 0; qb < QB; ++qb) acc[d][qb] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+
+    const uint32_t a_vo = (uint32_t)(l16 * DH + g * 8) * 2;  // + k2*16*DH*2 + ks*64
+    const uint32_t p_vo = (uint32_t)lane * 16;                // + i*1024
+    const int k_lo = (lane / (DH / 8)) * KW + (lane % (DH / 8)) * 8;
+    u32x4 kp[KPER], va[2][KS];
+    auto load_k = [&](int c) {  // descriptors over keys [c*KC, N): keys past N read as zeros
+        const __amdgpu_buffer_rsrc_t kres = buf_rsrc(kb_ptr + (int64_t)c * KC * DH, (uint32_t)(N - c * KC) * DH * 2);
+#pragma unroll
+        for (int i = 0; i < KPER; ++i) kp[i] = buf_load16(kres, p_vo + i * 1024, 0);
+    };
+    auto load_v = [&](int c) {
+        const __amdgpu_buffer_rsrc_t vres = buf_rsrc(vb_ptr + (int64_t)c * KC * DH, (uint32_t)(N - c * KC) * DH * 2);
+#pragma unroll
+        for (int k2 = 0; k2 < 2; ++k2)
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) va[k2][ks] = buf_load16(vres, a_vo + k2 * 16 * DH * 2 + ks * 64, 0);
+    };
+    const int trow = l16 >> 2, tcol = (l16 & 3) * 4;
+    int c = kw;
+    if (c < nch) {
+        load_k(c);
+        load_v(c);
+    }
+    for (; c < nch; c += 4) {
+        const int key0 = c * KC;
+        // K chunk into this wave's slot; its A operands and K^T come back from LDS
+#pragma unroll
+        for (int i = 0; i < KPER; ++i)
+            *reinterpret_cast<u32x4*>(kslot + k_lo + i * (64 / (DH / 8)) * KW) = kp[i];
+        if (c + 4 < nch) load_k(c + 4);
+        floatx4 s[QB][2], dp[QB][2];
+#pragma unroll
+        for (int k2 = 0; k2 < 2; ++k2) {
+            half8 kf[KS];
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks)
+                kf[ks] = *reinterpret_cast<const half8*>(kslot + (k2 * 16 + l16) * KW + ks * 32 + g * 8);
+#pragma unroll
+            for (int qb = 0; qb < QB; ++qb) {
+                s[qb][k2] = mfma16(kf[0], qf[qb][0], floatx4{0.0f, 0.0f, 0.0f, 0.0f});
+                dp[qb][k2] = mfma16(as_half8(va[k2][0]), gf[qb][0], floatx4{0.0f, 0.0f, 0.0f, 0.0f});
+#pragma unroll
+                for (int ks = 1; ks < KS; ++ks) {
+                    s[qb][k2] = mfma16(kf[ks], qf[qb][ks], s[qb][k2]);
+                    dp[qb][k2] = mfma16(as_half8(va[k2][ks]), gf[qb][ks], dp[qb][k2]);
+                }
+            }
+        }
+        if (c + 4 < nch) load_v(c + 4);
+        // element j of s[qb][k2]: key key0 + 16 k2 + 4 g + j, row R0 + 16 qb + l16
+        const bool edge = key0 + KC > N || (CAUSAL && key0 + KC - 1 > pmin);
+        half8 db_[QB];
+#pragma unroll
+        for (int qb = 0; qb < QB; ++qb) {
+            const int lim = (CAUSAL ? min(N - 1, qpos[qb]) : N - 1) - key0 - 4 * g;
+            float dsv[2][4];
+#pragma unroll
+            for (int k2 = 0; k2 < 2; ++k2)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    float pe = fast_exp2(__builtin_fmaf(s[qb][k2][j], c2, -l2[qb]));
+                    if (edge && k2 * 16 + j > lim) pe = 0.0f;
+                    dsv[k2][j] = pe * (dp[qb][k2][j] - dd[qb]);
+                }
+            u32x4 u = {pack_h2(dsv[0][0], dsv[0][1]), pack_h2(dsv[0][2], dsv[0][3]),
+                       pack_h2(dsv[1][0], dsv[1][1]), pack_h2(dsv[1][2], dsv[1][3])};
+            db_[qb] = as_half8(u);
+        }
+#pragma unroll
+        for (int d = 0; d < DB; ++d) {
+            const f16* base0 = kslot + (g * 4 + trow) * KW + d * 16 + tcol;
+            const half8 kt = cat4(lds_read_tr(base0), lds_read_tr(base0 + 16 * KW));
+#pragma unroll
+            for (int qb = 0; qb < QB; ++qb) acc[d][qb] = mfma16(kt, db_[qb], acc[d][qb]);
+        }
+    }
+
+    // sum the four key ranges' dQ^T through LDS: [key range][tile row][OW]
+    int ml = lane;
+    asm volatile("" : "+v"(ml));
+    const int ml16 = ml & 15, mg = ml >> 4;
+    __syncthreads();
+    float* ob = smem_f;
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+        for (int d = 0; d < DB; ++d)
+            *reinterpret_cast<floatx4*>(ob + (kw * 64 + (wave >> 2) * 32 + qb * 16 + ml16) * OW + d * 16 + mg * 4) = acc[d][qb];
+    __syncthreads();
+    constexpr int CPR = DH / 8;
+    for (int rr = ml / CPR; rr < 8; rr += 64 / CPR) {
+        const int q = wave * 8 + rr;
+        const int row = T0 + q;
+        const int dc = (ml % CPR) * 8;
+        floatx4 a0 = *reinterpret_cast<const floatx4*>(ob + q * OW + dc);
+        floatx4 a1 = *reinterpret_cast<const floatx4*>(ob + q * OW + dc + 4);
+#pragma unroll
+        for (int w = 1; w < 4; ++w) {
+            a0 += *reinterpret_cast<const floatx4*>(ob + (w * 64 + q) * OW + dc);
+            a1 += *reinterpret_cast<const floatx4*>(ob + (w * 64 + q) * OW + dc + 4);
+        }
+        if (row < NH) {
+            const float sc = p.scale;
+            u32x4 o = {pack_h2(a0[0] * sc, a0[1] * sc), pack_h2(a0[2] * sc, a0[3] * sc),
+                       pack_h2(a1[0] * sc, a1[1] * sc), pack_h2(a1[2] * sc, a1[3] * sc)};
+            __builtin_nontemporal_store(o, reinterpret_cast<u32x4*>(p.out + ((int64_t)b * NH + row) * DH + dc));
+        }
+    }
+}
+
 // dK/dV (key blocks x row parts) and dQ (row tiles) in one launch: the
 // first n_kv workgroups run the former, heavy key blocks first, the rest
 // the latter, heavy row tiles first.  The two halves are independent (both
 // read only Q, K, V, dO and the row statistics), so the dQ tiles fill the
 // CUs that the short dK/dV parts free.
-// DH = 128 runs one wave per SIMD (450 registers: both bodies hold 128
-// accumulators and as many operand values).  It is a latency chain, about
-// 1.9 us per 32-row chunk of a dK/dV part, but its parts fill the chip where
-// one workgroup per 32 keys (the kernels below) leaves most CUs idle: with
-// the forward, B=2 N=2000 H=8 causal 834 -> 203 us, B=1 N=1740 H=12 1035 ->
-// 125 us, B=1 N=130 H=2 40.5 -> 32.7 us.  Longer parts halve the fp32
-// partials but not the chain: parts of 32 chunks 201, 116 and (B=1 N=600
-// H=4) 85.6 us against 203, 125 and 54.9 us with 16.
-template <int DH, bool CAUSAL>
-__global__ __launch_bounds__(256, DH <= 64 ? 2 : 1) void flash_bwd_kvq(FlashArgs p, float* part_ws, int parts_per_batch, int n_kv) {
-    constexpr int KVB = KvLayout<DH>::LDS_BYTES, QB = DqLayout<DH>::LDS_BYTES;
+// DH = 128 has bodies of its own on 8 waves, two per SIMD: 153 -> 126 us for B=2
+// N=2000 H=8 causal against the 4-wave bodies at one wave per SIMD (450
+// registers), and 834 -> 163 with the forward against the kernels below (one
+// workgroup per 32 keys).  Bound by instruction issue: a 32-row chunk of a
+// dK/dV part takes about 1.4 us for 1024 cycles of MFMA per SIMD; chunks whose
+// loads all hit the L2 take as long, and the unmasked form and v_dot2 row sums
+// took off 6 us.
+// PL: part_log2 where it is known at compile time (16 chunks, the length of the
+// larger calls up to head size 64: 1 % at B=4 N=1024 H=8), or 0.
+template <int DH, bool CAUSAL, int PL>
+__global__ __launch_bounds__(DH <= 64 ? 256 : 512, 2) void flash_bwd_kvq(FlashArgs p, float* part_ws, int parts_per_batch,
+                                                                        int n_kv) {
+    constexpr int KVB = DH <= 64 ? KvLayout<DH>::LDS_BYTES : KvPairLayout<DH>::LDS_BYTES;
+    constexpr int QB = DH <= 64 ? DqLayout<DH>::LDS_BYTES : DqPairLayout<DH>::LDS_BYTES;
     __shared__ __attribute__((aligned(16))) char lds[KVB > QB ? KVB : QB];
     if ((int)blockIdx.x < n_kv) {
         // Workgroup i runs on XCD i % 8.  When the batches divide the XCDs
@@ -1461,7 +1912,8 @@ __global__ __launch_bounds__(256, DH <= 64 ? 2 : 1) void flash_bwd_kvq(FlashArgs
             const int x = blk % 8, i = blk / 8;
             blk = (x / xpb) * parts_per_batch + i * xpb + x % xpb;
         }
-        bwd_kv_body<DH, CAUSAL>(p, part_ws, parts_per_batch, blk, lds);
+        if constexpr (DH <= 64) bwd_kv_body<DH, CAUSAL, PL>(p, part_ws, parts_per_batch, blk, lds);
+        else bwd_kv_pair_body<DH, CAUSAL>(p, part_ws, parts_per_batch, blk, lds);
     } else {
         // the same XCD assignment for the dQ tiles: XCD x takes the row tiles
         // of batch x / (8 / B) (heavy first), so that one XCD's L2 holds the
@@ -1473,7 +1925,8 @@ __global__ __launch_bounds__(256, DH <= 64 ? 2 : 1) void flash_bwd_kvq(FlashArgs
             const int x = blk % 8, i = blk / 8;
             blk = (i * xpb + x % xpb) * p.B + x / xpb;  // bwd_q_body: batch blk % B, tile blk / B
         }
-        bwd_q_body<DH, CAUSAL>(p, blk, lds);
+        if constexpr (DH <= 64) bwd_q_body<DH, CAUSAL>(p, blk, lds);
+        else bwd_q_pair_body<DH, CAUSAL>(p, blk, lds);
     }
 }
 
@@ -1894,13 +2347,10 @@ hipError_t launch_fwd(const FlashArgs& a, bool causal, int mode, hipStream_t st)
             constexpr int QB = FWD_KS_QB;
             const int64_t nrg_ks = ((int64_t)a.N * a.H + 16 * QB - 1) / (16 * QB);
             dim3 gk((unsigned)((nrg_ks + 1) / 2 * a.B));
-            FlashArgs s = a;
-            if (s.out_rstride == 0) {
-                s.out_rstride = DH;
-                s.out_bstride = (int64_t)a.N * a.H * DH;
-            }
-            if (causal) hipLaunchKernelGGL((flash_fwd_ks<DH, QB, true>), gk, dim3(512), 0, st, s);
-            else hipLaunchKernelGGL((flash_fwd_ks<DH, QB, false>), gk, dim3(512), 0, st, s);
+            if (a.out_rstride && !causal) return hipErrorInvalidValue;  // prefill is causal
+            if (a.out_rstride) hipLaunchKernelGGL((flash_fwd_ks<DH, QB, true, true>), gk, dim3(512), 0, st, a);
+            else if (causal) hipLaunchKernelGGL((flash_fwd_ks<DH, QB, true>), gk, dim3(512), 0, st, a);
+            else hipLaunchKernelGGL((flash_fwd_ks<DH, QB, false>), gk, dim3(512), 0, st, a);
             return hipGetLastError();
         }
     }
@@ -1937,22 +2387,28 @@ hipError_t launch_bwd(const FlashArgs& a, bool causal, bool have_lse, hipStream_
 }
 
 // dK/dV by key blocks and row parts, then dQ by row tiles (head dims 32, 64, 128).
-template <int DH>
-hipError_t launch_bwd_split(const FlashArgs& a, bool causal, float* parts, int parts_per_batch,
-                            hipStream_t st) {
+template <int DH, bool CAUSAL, int PL>
+hipError_t launch_bwd_parts(const FlashArgs& a, float* parts, int parts_per_batch, hipStream_t st) {
     const int NH = a.N * a.H;
     const int n_kv = a.B * parts_per_batch;
     dim3 gm((unsigned)(n_kv + (NH + 63) / 64 * a.B));
     const int nkb = (a.N + BKB - 1) / BKB;
     dim3 gr((unsigned)(a.B * nkb * 16));
-    if (causal) {
-        hipLaunchKernelGGL((flash_bwd_kvq<DH, true>), gm, dim3(256), 0, st, a, parts, parts_per_batch, n_kv);
-        hipLaunchKernelGGL((flash_bwd_kv_reduce<DH, true>), gr, dim3(256), 0, st, a, parts, parts_per_batch);
-    } else {
-        hipLaunchKernelGGL((flash_bwd_kvq<DH, false>), gm, dim3(256), 0, st, a, parts, parts_per_batch, n_kv);
-        hipLaunchKernelGGL((flash_bwd_kv_reduce<DH, false>), gr, dim3(256), 0, st, a, parts, parts_per_batch);
-    }
+    hipLaunchKernelGGL((flash_bwd_kvq<DH, CAUSAL, PL>), gm, dim3(DH <= 64 ? 256 : 512), 0, st, a, parts, parts_per_batch,
+                       n_kv);
+    hipLaunchKernelGGL((flash_bwd_kv_reduce<DH, CAUSAL, PL>), gr, dim3(256), 0, st, a, parts, parts_per_batch);
     return hipGetLastError();
+}
+template <int DH>
+hipError_t launch_bwd_split(const FlashArgs& a, bool causal, float* parts, int parts_per_batch,
+                            hipStream_t st) {
+    if constexpr (DH <= 64) {
+        if (a.part_log2 == 4)
+            return causal ? launch_bwd_parts<DH, true, 4>(a, parts, parts_per_batch, st)
+                          : launch_bwd_parts<DH, false, 4>(a, parts, parts_per_batch, st);
+    }
+    return causal ? launch_bwd_parts<DH, true, 0>(a, parts, parts_per_batch, st)
+                  : launch_bwd_parts<DH, false, 0>(a, parts, parts_per_batch, st);
 }
 
 }  // namespace
@@ -2009,8 +2465,12 @@ int flash_backward(FlashArgs a, int dh, bool mfma, bool causal, hipStream_t st) 
     auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
     const int nkb = (a.N + BKB - 1) / BKB;
     int parts_per_batch = 0;
-    if (split)
-        for (int kb = 0; kb < nkb; ++kb) parts_per_batch += bwd_kv_parts(kb, a.N, a.H, causal);
+    if (split) {
+        int64_t chunks = 0;
+        for (int kb = 0; kb < nkb; ++kb) chunks += bwd_kv_chunks(kb, a.N, a.H, causal);
+        a.part_log2 = bwd_part_log2(dh, chunks * a.B);
+        for (int kb = 0; kb < nkb; ++kb) parts_per_batch += bwd_kv_parts(kb, a.N, a.H, causal, a.part_log2);
+    }
     const size_t stats_b = (split || wide) ? 0 : al(2 * rows * sizeof(float));  // formed in-kernel
     const size_t part_b = split ? al((size_t)a.B * parts_per_batch * 4 * (2 * 2 * (dh / 16)) * 64 * 16) : 0;
     const size_t fwd_b = ((split || wide) && !have_lse) ? al(rows * dh * 2) + al(rows * sizeof(float)) : 0;

@@ -50,8 +50,9 @@ struct FlashArgs {
     float scale_log2;  // scale * log2(e)
     float scale;
     int spin_limit;    // iterations of a bounded in-kernel wait before it gives up
-    int64_t out_bstride;  // forward, flash_out_strided head sizes only: elements between the O of consecutive
+    int64_t out_bstride;  // causal forward, flash_out_strided head sizes only: elements between the O of consecutive
     int out_rstride;      // batches and query rows; 0, 0 = contiguous (B, N, H*Dh)
+    int part_log2;        // backward: chunks per dK/dV row part
 };
 // flash_wide.hip: MFMA forward / backward for the other multiples of 16 up
 // to 256.  The backward takes the forward's O and LSE in a.o / a.lse (no

@@ -145,11 +145,12 @@ def test_flash_backward_dh32_split_parts(dev, orc, causal):
 
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("use_lse", [True, False])
-@pytest.mark.parametrize("B,N,H", [(2, 300, 8), (1, 127, 4), (1, 129, 5), (8, 64, 8)])
+@pytest.mark.parametrize("B,N,H", [(2, 300, 8), (1, 127, 4), (1, 129, 5), (8, 64, 8), (1, 60, 2), (3, 33, 1), (1, 700, 6)])
 def test_flash_backward_dh128(dev, orc, B, N, H, causal, use_lse):
     """Head size 128 at the edges of its tiles: several row parts per key
-    block, one key short of and one key past a 128-key block, heads that do
-    not divide the 32-row chunks, one part (written without partials)."""
+    block (of 4 and of 8 chunks), one key short of and one key past a 128-key
+    block, heads that do not divide the 32-row chunks, one part (written
+    without partials), query tiles whose second half holds no rows."""
     import evk_amd as evk
     import torch
     Dh = 128
