@@ -180,6 +180,24 @@ DEV float wave_sum(float v) {
     return v;
 }
 
+// v += v of the lane that DPP control CTRL names (0xB1, 0x4E: lanes 1 and 2
+// apart in a quad; 0x141: the mirrored lane of 8; 0x140: of 16)
+template <int CTRL>
+DEV void dpp_add(float& v) {
+    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
+}
+
+// sum over groups of W adjacent lanes (W a power of two up to 32)
+template <int W>
+DEV float lanes_sum(float v) {
+    if (W >= 2) dpp_add<0xB1>(v);
+    if (W >= 4) dpp_add<0x4E>(v);
+    if (W >= 8) dpp_add<0x141>(v);
+    if (W >= 16) dpp_add<0x140>(v);
+    if (W >= 32) v += __shfl_xor(v, 16, 64);
+    return v;
+}
+
 // tanh GELU of gelu.comp (evk_ai.cpp:679-699)
 DEV float gelu_f(float x) {
     const float ka = 0.7978845608028654f, kb = 0.044715f;

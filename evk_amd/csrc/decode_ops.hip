@@ -8,6 +8,7 @@
 #include <math.h>
 
 #include <algorithm>
+#include <cmath>
 
 namespace evkhip {
 
@@ -16,9 +17,18 @@ namespace {
 // ---------------------------------------------------------------------------
 // Single-query attention.  Grid (heads, nsplit); 256 threads.  A workgroup
 // covers cache rows [split*chunk, +chunk) of one head: LPK = DH/8 lanes per
-// key (16 bytes each), 256/LPK keys per pass (DH = 256: 32 lanes, 8 keys).  Partial (m, l, o) go to
-// workspace; the last workgroup of a head merges the splits in split order.
+// key (16 bytes each), 256/LPK keys per pass, U passes requested at once and
+// the next U while those are scored (U = 1 where a split is one pass).
+// Latency bounds a short cache and the bytes in flight a long one; with one
+// pass at a time and a fence per workgroup, us before -> now, the step's two
+// cache writes included: 16 caches of 160 rows of 256 14.3 -> 9.8, 38 of 739
+// 56 -> 12, one of 4000 rows of 12 heads of 64 62 -> 11, 32 of 2001 rows of 8
+// heads of 128 121 -> 47 (5.5 TB/s).  Partial (m, l, o) go to workspace at agent scope; the last
+// workgroup of a head merges the splits in split order, every partial it
+// needs requested in batches of SQ_MB.
 // ---------------------------------------------------------------------------
+constexpr int SQ_U = 4, SQ_MB = 16;
+constexpr int SQ_SPLITS = 256;  // at most: one thread each in the merge
 struct SqArgs {
     const f16* q;
     const f16* kc;
@@ -34,14 +44,13 @@ struct SqArgs {
 
 constexpr float kLog2e = 1.4426950408889634f;
 
-template <int DH>
+template <int DH, int U>
 __global__ __launch_bounds__(256) void sq_attention(SqArgs a) {
     constexpr int LPK = DH / 8;             // lanes per key
     constexpr int KPP = 256 / LPK;          // keys per pass
     static_assert(KPP >= 4, "at least one key slot per wave");
     __shared__ float s_m[4], s_w[4];
     __shared__ float s_o[4][DH];
-    __shared__ unsigned s_last;
     // h: (sequence, head) pair; q, out and the workspace are indexed by it,
     // the caches by the sequence's cache and the head's columns
     const int h = blockIdx.x, split = blockIdx.y, nsplit = gridDim.y;
@@ -62,32 +71,51 @@ __global__ __launch_bounds__(256) void sq_attention(SqArgs a) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) o[e] = 0.0f;
 
-    for (int jb = j0; jb < j1; jb += KPP) {
-        const int j = jb + kslot;
-        float s = -INFINITY;
-        half8 vh;
-        if (j < j1) {
-            const f16* kr = kc + (int64_t)j * a.row_stride + sub * 8;
-            half8 kh = *reinterpret_cast<const half8*>(kr);
-            vh = *reinterpret_cast<const half8*>(vc + (int64_t)j * a.row_stride + sub * 8);
+    auto load = [&](int jb, half8 (&k)[U], half8 (&v)[U]) {  // rows past the range: its last one, masked below
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int64_t at = (int64_t)min(jb + u * KPP + kslot, j1 - 1) * a.row_stride + sub * 8;
+            k[u] = *reinterpret_cast<const half8*>(kc + at);
+            v[u] = *reinterpret_cast<const half8*>(vc + at);
+        }
+    };
+    half8 kh[U], vh[U];
+    if (j0 < j1) load(j0, kh, vh);
+    for (int jb = j0; jb < j1; jb += KPP * U) {
+        half8 kn[U], vn[U];
+        const bool more = jb + KPP * U < j1;
+        if (more) load(jb + KPP * U, kn, vn);
+        // online softmax per lane group (all LPK lanes of a key hold the same s)
+        float s[U], mn = m;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
             float d = 0.0f;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) d += qv[e] * (float)kh[e];
-#pragma unroll
-            for (int off = LPK / 2; off > 0; off >>= 1) d += __shfl_xor(d, off, 64);
-            s = d * a.scale_log2;
-        } else {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) vh[e] = (f16)0.0f;
+            for (int e = 0; e < 8; ++e) d += qv[e] * (float)kh[u][e];
+            d = lanes_sum<LPK>(d);
+            s[u] = jb + u * KPP + kslot < j1 ? d * a.scale_log2 : -INFINITY;
+            mn = fmaxf(mn, s[u]);
         }
-        // online softmax per lane group (all LPK lanes of a key hold the same s)
-        float mn = fmaxf(m, s);
-        float base = mn == -INFINITY ? 0.0f : mn;
-        float al = exp2f(m - base), pe = exp2f(s - base);
-        l = l * al + pe;
+        const float base = mn == -INFINITY ? 0.0f : mn;
+        const float al = exp2f(m - base);
+        l *= al;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) o[e] = o[e] * al + pe * (float)vh[e];
+        for (int e = 0; e < 8; ++e) o[e] *= al;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const float pe = exp2f(s[u] - base);
+            l += pe;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) o[e] += pe * (float)vh[u][e];
+        }
         m = mn;
+        if (more) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                kh[u] = kn[u];
+                vh[u] = vn[u];
+            }
+        }
     }
     // Merge the key slots of the workgroup: within a wave (slots sharing sub)
     // then across waves through LDS.
@@ -122,34 +150,46 @@ __global__ __launch_bounds__(256) void sq_attention(SqArgs a) {
         if (nsplit == 1) {
             a.out[(int64_t)h * DH + tid] = (f16)(ll > 0.0f ? oo / ll : 0.0f);
         } else {
-            part[2 + tid] = oo;
-            if (tid == 0) { part[0] = mm; part[1] = ll; }
+            st_ag(part + 2 + tid, oo);
+            if (tid == 0) {
+                st_ag(part, mm);
+                st_ag(part + 1, ll);
+            }
         }
     }
-    if (nsplit == 1) return;
-    __threadfence();
+    if (nsplit == 1 || !arrive_last(a.counters + h, nsplit)) return;
+    // Weights of the splits, one thread each; then GR groups of DH threads sum
+    // every GR-th split's o and meet in LDS in group order.
+    constexpr int GR = 256 / DH;
+    __shared__ float s_wt[SQ_SPLITS], s_sum[GR][DH];
+    const float* ph = a.part + (int64_t)h * nsplit * (2 + DH);
+    const float m_sp = tid < nsplit ? ld_ag(ph + tid * (2 + DH)) : -INFINITY;
+    const float l_sp = tid < nsplit ? ld_ag(ph + tid * (2 + DH) + 1) : 0.0f;
+    float mm = wave_max(m_sp);
+    if (lane == 0) s_m[wave] = mm;
     __syncthreads();
-    if (tid == 0) {
-        unsigned prev = atomicAdd(a.counters + h, 1u);
-        s_last = prev == (unsigned)(nsplit - 1);
-        if (s_last) a.counters[h] = 0u;
+    mm = fmaxf(fmaxf(s_m[0], s_m[1]), fmaxf(s_m[2], s_m[3]));
+    const float wt = exp2f(m_sp - (mm == -INFINITY ? 0.0f : mm));
+    const float lw = wave_sum(l_sp * wt);
+    s_wt[tid] = wt;
+    if (lane == 0) s_w[wave] = lw;
+    __syncthreads();
+    const float ll = s_w[0] + s_w[1] + s_w[2] + s_w[3];
+    const int gr = tid / DH, dim = tid % DH;
+    float oo = 0.0f;
+    for (int sp = gr; sp < nsplit; sp += GR * SQ_MB) {
+        float t[SQ_MB];
+#pragma unroll
+        for (int u = 0; u < SQ_MB; ++u) t[u] = sp + u * GR < nsplit ? ld_ag(ph + (sp + u * GR) * (2 + DH) + 2 + dim) : 0.0f;
+#pragma unroll
+        for (int u = 0; u < SQ_MB; ++u) oo += t[u] * (sp + u * GR < nsplit ? s_wt[sp + u * GR] : 0.0f);
     }
+    s_sum[gr][dim] = oo;
     __syncthreads();
-    if (!s_last) return;
-    __threadfence();
     if (tid < DH) {
-        const float* ph = a.part + (int64_t)h * nsplit * (2 + DH);
-        float mm = -INFINITY;
-        for (int sp = 0; sp < nsplit; ++sp)
-            mm = fmaxf(mm, __hip_atomic_load(ph + sp * (2 + DH), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-        float base = mm == -INFINITY ? 0.0f : mm;
-        float ll = 0.0f, oo = 0.0f;
-        for (int sp = 0; sp < nsplit; ++sp) {
-            const float* q = ph + sp * (2 + DH);
-            float f = exp2f(__hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - base);
-            ll += __hip_atomic_load(q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) * f;
-            oo += __hip_atomic_load(q + 2 + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) * f;
-        }
+        oo = 0.0f;
+#pragma unroll
+        for (int g = 0; g < GR; ++g) oo += s_sum[g][tid];
         a.out[(int64_t)h * DH + tid] = (f16)(ll > 0.0f ? oo / ll : 0.0f);
     }
 }
@@ -443,13 +483,16 @@ int sq_attention_launch(const f16* q, const f16* kc, const f16* vc, f16* out, in
         hipError_t e = hipGetLastError();
         return e == hipSuccess ? EVKHIP_OK : check_hip(e, "sq_attention_scalar launch");
     }
-    // split so that each workgroup streams at least 64 rows and the grid has
-    // about two workgroups per CU
+    // A split walks `step` rows at a time (about a microsecond each), and the
+    // merge takes about as long per SQ_MB splits: chunk / step + splits / SQ_MB
+    // is least at splits = sqrt(SQ_MB L / step), within two workgroups per CU.
     const int cus = device_cu_count();
     int nsplit = 1, chunk = std::max(L, 1);
-    if (L > 64) {
-        nsplit = std::max(1, std::min((L + 63) / 64, (2 * cus + heads - 1) / heads));
-        chunk = (L + nsplit - 1) / nsplit;
+    const int step = 256 / (dh / 8) * SQ_U;
+    if (L > std::max(step, 64)) {  // up to 64 rows: no workspace
+        const int few = (int)std::ceil(std::sqrt((double)SQ_MB * L / step));
+        nsplit = std::max(1, std::min({(L + step - 1) / step, (2 * cus + heads - 1) / heads, few, SQ_SPLITS}));
+        chunk = ((L + nsplit - 1) / nsplit + step - 1) / step * step;  // whole steps
         nsplit = (L + chunk - 1) / chunk;
     }
     a.chunk = chunk;
@@ -476,13 +519,19 @@ int sq_attention_launch(const f16* q, const f16* kc, const f16* vc, f16* out, in
     }
     a.part = g_sq_part;
     a.counters = g_sq_cnt;
-    dim3 grid(heads, nsplit);
+    const bool one = chunk <= 256 / (dh / 8);  // a split is one pass
+    auto launch = [&](auto D) {
+        constexpr int DH = decltype(D)::value;
+        const dim3 grid(heads, nsplit);
+        if (one) hipLaunchKernelGGL((sq_attention<DH, 1>), grid, dim3(256), 0, st, a);
+        else hipLaunchKernelGGL((sq_attention<DH, SQ_U>), grid, dim3(256), 0, st, a);
+    };
     switch (dh) {
-        case 16: hipLaunchKernelGGL(sq_attention<16>, grid, dim3(256), 0, st, a); break;
-        case 32: hipLaunchKernelGGL(sq_attention<32>, grid, dim3(256), 0, st, a); break;
-        case 64: hipLaunchKernelGGL(sq_attention<64>, grid, dim3(256), 0, st, a); break;
-        case 128: hipLaunchKernelGGL(sq_attention<128>, grid, dim3(256), 0, st, a); break;
-        default: hipLaunchKernelGGL(sq_attention<256>, grid, dim3(256), 0, st, a); break;
+        case 16: launch(std::integral_constant<int, 16>{}); break;
+        case 32: launch(std::integral_constant<int, 32>{}); break;
+        case 64: launch(std::integral_constant<int, 64>{}); break;
+        case 128: launch(std::integral_constant<int, 128>{}); break;
+        default: launch(std::integral_constant<int, 256>{}); break;
     }
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? EVKHIP_OK : check_hip(e, "sq_attention launch");

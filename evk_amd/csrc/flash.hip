@@ -902,13 +902,6 @@ DEV float dot8_pairs(const half8& x, const half8& y) {
     return acc;
 }
 
-// v += v of the lane that DPP control CTRL names (0xB1, 0x4E: lanes 1 and 2
-// apart in a quad; 0x141: the mirrored lane of 8; 0x140: of 16)
-template <int CTRL>
-DEV void dpp_add(float& v) {
-    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
-}
-
 constexpr int BKB = 128;       // keys per workgroup (4 waves x 32)
 constexpr int BRC = 32;        // flattened query rows per chunk
 // Chunks per row part, as a power of two: as long as leaves about 128 parts

@@ -406,3 +406,25 @@ def test_reference_training_shape_d256(dev, orc, use_lse):
     ones = np.full((B, N, D), f16(1.0), np.uint16)
     o1, _ = fwd(evk, dev, q, k, ones, True)
     assert np.abs(f32(o1) - 1.0).max() <= 1e-3
+
+
+@pytest.mark.parametrize("dh", [16, 32, 64, 128, 256])
+@pytest.mark.parametrize("L", [1, 64, 65, 513, 2049])
+def test_sq_attention_splits(dev, orc, dh, L):
+    """Cache lengths at the edges of a pass, of a step and of a split, for
+    every vector head size; a row of scores that dwarfs the others (one
+    split's weight 1, the rest 0) for the second sequence; two calls in a row
+    (the counters reset)."""
+    import torch
+    import evk_amd as evk
+    B, heads = 2, 3
+    D, maxlen = heads * dh, L + 5
+    q, kc, vc = orc.normal_f16((B, D), 361 + L), orc.normal_f16((B, maxlen, D), 362 + L), orc.normal_f16((B, maxlen, D), 363)
+    kc[1, L // 2] = q[1]  # q . q is about dh, the other scores about sqrt(dh)
+    Q, K, V = to_dev(q, dev), to_dev(kc, dev), to_dev(vc, dev)
+    for _ in range(2):
+        O = torch.empty((B, D), dtype=torch.float16, device=dev)
+        evk.single_query_attention(Q, K, V, O, L, heads)
+        torch.cuda.synchronize()
+        for b in range(B):
+            assert_close_f16(from_dev(O)[b], orc.sq_attention(q[b], kc[b], vc[b], L, heads), what=f"dh={dh} L={L} b={b}")
