@@ -303,12 +303,24 @@ DEV float dot8(const u32x4& a, const u32x4& b) {
     return acc;
 }
 
+// Partial products dO . O of a row's DH / 8 pieces: on adjacent lanes where
+// their number divides a half wave (summed there), else in LDS rows of an odd
+// number of floats that the row's thread walks.  (Rows of DH / 8 floats put a
+// wave's reads on one bank: for DH = 256 each of the 32 reads was a 32-way
+// conflict.)
+template <int DH>
+struct RowDots {
+    static constexpr int PPR = DH / 8;
+    static constexpr bool LANES = (PPR & (PPR - 1)) == 0;
+    static constexpr int STRIDE = PPR | 1, BYTES = LANES ? 0 : WKC * STRIDE * 4;
+};
+
 // LDS of a flash_bwd_wide workgroup, either role: two double-buffered
 // 32-row tiles, then (dK/dV) the tiles' lse2 and D, the block exchange and
 // the per-piece dO . O products of the next tile
 template <int DH>
 constexpr int bwd_wide_lds() {
-    return 2 * 2 * WKC * WideTile<DH>::W * 2 + 2 * 2 * WKC * 4 + XBYTES + WideTile<DH>::PIECES * 4;
+    return 2 * 2 * WKC * WideTile<DH>::W * 2 + 2 * 2 * WKC * 4 + XBYTES + RowDots<DH>::BYTES;
 }
 
 template <int DH, bool CAUSAL>
@@ -354,19 +366,30 @@ __device__ void bwd_dkdv_wide(const FlashArgs& p, int bx, char* lds) {
     // D = rowsum(dO * O).  The LSE is loaded as it is and scaled when it goes
     // to LDS: arithmetic on it at the load would make the wave wait there for
     // every load in flight, the next tile's included.  O comes in the dO
-    // tile's piece layout; each thread stores the dot products of its pieces
-    // and, after the next barrier, the first WKC threads add their row's
-    // DH / 8 products in order.
-    constexpr int PPR = DH / 8;  // pieces per row
+    // tile's piece layout (RowDots).  Rows advance by WKC a tile without
+    // dividing by H, and the mask compares rows: with a division per score the
+    // tile spent more on it than on everything else the VALU does (B=2 N=456
+    // H=4 Dh=96 forward and backward 119 -> 90 us, B=4 N=1000 H=2 Dh=256 217 ->
+    // 180, both changes together).
+    using RD = RowDots<DH>;
+    constexpr int PPR = RD::PPR;
     WideTile<DH> lq, lg, lo;
     float lsv = 0.0f;
-    auto load_tile = [&](int t) {
+    int st_head = (rstart + (int)(threadIdx.x % WKC)) % H, st_pos = (rstart + (int)(threadIdx.x % WKC)) / H;
+    const int h_step = WKC % H, p_step = WKC / H;
+    auto load_tile = [&](int t) {  // t = 0, 1, ... in order
         const int r0 = rstart + t * WKC;
         lq.load(qres, r0);
         lg.load(gres, r0);
         lo.load(ores, r0);
         const int r = r0 + (int)threadIdx.x;
-        lsv = buf_load_f32(lres, oob_or(threadIdx.x < WKC && r < NH, (uint32_t)((r % H) * N + r / H) * 4u));
+        lsv = buf_load_f32(lres, oob_or(threadIdx.x < WKC && r < NH, (uint32_t)(st_head * N + st_pos) * 4u));
+        st_head += h_step;
+        st_pos += p_step;
+        if (st_head >= H) {
+            st_head -= H;
+            st_pos += 1;
+        }
     };
     auto stage_tile = [&](int st) {
         lq.store(sQ[st]);
@@ -374,18 +397,27 @@ __device__ void bwd_dkdv_wide(const FlashArgs& p, int bx, char* lds) {
 #pragma unroll
         for (int i = 0; i < WideTile<DH>::PER; ++i) {
             const int pc = threadIdx.x + 256 * i;
-            if (WideTile<DH>::PIECES % 256 == 0 || pc < WideTile<DH>::PIECES) sPart[pc] = dot8(lg.r[i], lo.r[i]);
+            const bool ok = WideTile<DH>::PIECES % 256 == 0 || pc < WideTile<DH>::PIECES;
+            float d = ok ? dot8(lg.r[i], lo.r[i]) : 0.0f;
+            if constexpr (RD::LANES) {
+                d = lanes_sum<PPR>(d);
+                if (ok && pc % PPR == 0) sD[st][pc / PPR] = d;
+            } else {
+                if (ok) sPart[pc / PPR * RD::STRIDE + pc % PPR] = d;
+            }
         }
         if (threadIdx.x < WKC) sL[st][threadIdx.x] = lsv * kLog2e;
     };
     auto finish_d = [&](int st) {
-        if (threadIdx.x < WKC) {
+        if (!RD::LANES && threadIdx.x < WKC) {
             float d = 0.0f;
 #pragma unroll
-            for (int c = 0; c < PPR; ++c) d += sPart[threadIdx.x * PPR + c];
+            for (int c = 0; c < PPR; ++c) d += sPart[threadIdx.x * RD::STRIDE + c];
             sD[st][threadIdx.x] = d;
         }
     };
+    // a row r meets this thread's key from position mykey on: r >= r_from
+    const int r_from = !key_ok ? NH : CAUSAL ? mykey * H : 0;
     if (nrt > 0) load_tile(0);
     // drain the key operands' and the first tile's loads together: inside
     // the loop only the next tile's loads are then in flight (see
@@ -411,7 +443,7 @@ __device__ void bwd_dkdv_wide(const FlashArgs& p, int bx, char* lds) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const int rl = rb * 16 + 4 * g + j, r = r0 + rl;
-                const bool ok = r < NH && key_ok && (!CAUSAL || mykey <= r / H);
+                const bool ok = r < NH && r >= r_from;
                 const float pv = ok ? __builtin_amdgcn_exp2f(__builtin_fmaf(s[rb][j], c2, -sL[cur][rl])) : 0.0f;
                 pe[rb][j] = pv;
                 ds[rb][j] = pv * (dp[rb][j] - sD[cur][rl]);

@@ -428,3 +428,18 @@ def test_sq_attention_splits(dev, orc, dh, L):
         torch.cuda.synchronize()
         for b in range(B):
             assert_close_f16(from_dev(O)[b], orc.sq_attention(q[b], kc[b], vc[b], L, heads), what=f"dh={dh} L={L} b={b}")
+
+
+@pytest.mark.parametrize("Dh,H,N", [(48, 40, 9), (256, 5, 37), (176, 33, 20), (16, 3, 70)])
+@pytest.mark.parametrize("causal", [True, False])
+def test_wide_backward_head_counts(dev, orc, Dh, H, N, causal):
+    """Wide-head backward where the 32-row tiles and the heads do not divide
+    each other (more heads than a tile has rows among them): the rows' heads
+    and positions advance tile by tile, and head sizes with and without a
+    power-of-two number of pieces form the row sums differently."""
+    import evk_amd as evk
+    q, g = orc.normal_f16((2, N, H * Dh), 371 + N), orc.normal_f16((2, N, H * Dh), 374 + N)
+    k, v = orc.normal_f16((2, N, Dh), 372 + N), orc.normal_f16((2, N, Dh), 373 + N)
+    got = bwd(evk, dev, q, k, v, g, causal, True)
+    for x, want, what in zip(got, orc.attention_bwd(q, k, v, g, causal), ("dQ", "dK", "dV")):
+        assert_close_f16(x, want, what=f"{what} Dh={Dh} H={H} N={N}")
