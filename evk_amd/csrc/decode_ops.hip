@@ -84,7 +84,13 @@ __global__ __launch_bounds__(256) void sq_attention(SqArgs a) {
     for (int jb = j0; jb < j1; jb += KPP * U) {
         half8 kn[U], vn[U];
         const bool more = jb + KPP * U < j1;
-        if (more) load(jb + KPP * U, kn, vn);
+        if (more) {
+            load(jb + KPP * U, kn, vn);
+        } else {  // weight 0 times the last row again is not 0 where that row holds an infinity
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (jb + u * KPP + kslot >= j1) vh[u] = half8{};
+        }
         // online softmax per lane group (all LPK lanes of a key hold the same s)
         float s[U], mn = m;
 #pragma unroll

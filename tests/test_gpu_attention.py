@@ -430,6 +430,23 @@ def test_sq_attention_splits(dev, orc, dh, L):
             assert_close_f16(from_dev(O)[b], orc.sq_attention(q[b], kc[b], vc[b], L, heads), what=f"dh={dh} L={L} b={b}")
 
 
+@pytest.mark.parametrize("L", [1, 30, 63, 100, 700])
+def test_sq_attention_infinity_in_last_row(dev, orc, L):
+    """An infinity in a sequence's last value row reaches the output as one:
+    a workgroup's passes that end past the rows read the last one again, with
+    weight 0, and 0 times infinity is not 0.  A NaN past the rows stays out."""
+    import evk_amd as evk
+    dh, maxlen = 64, L + 3
+    q, kc, vc = orc.normal_f16((dh,), 381 + L), orc.normal_f16((maxlen, dh), 382), orc.normal_f16((maxlen, dh), 383)
+    want = orc.sq_attention(q, kc, vc, L, 1).copy()
+    kc[L:], vc[L:] = 0x7E00, 0x7E00
+    vc[L - 1, 5] = 0x7C00
+    got = sq(evk, dev, q, kc, vc, L, 1)
+    assert got[5] == 0x7C00
+    got[5] = want[5] = 0
+    assert_close_f16(got, want, what=f"L={L}")
+
+
 @pytest.mark.parametrize("Dh,H,N", [(48, 40, 9), (256, 5, 37), (176, 33, 20), (16, 3, 70)])
 @pytest.mark.parametrize("causal", [True, False])
 def test_wide_backward_head_counts(dev, orc, Dh, H, N, causal):
