@@ -147,6 +147,21 @@ struct RagTile {
     }
 };
 
+// Four rotary pairs by their (cos, sin), as rope_k rotates (fp32, one fp16
+// rounding).
+DEV half8 rope8(const half8& x, const float2* t) {
+    const floatx4 t0 = reinterpret_cast<const floatx4*>(t)[0], t1 = reinterpret_cast<const floatx4*>(t)[1];
+    const float cs[4] = {t0[0], t0[2], t1[0], t1[2]}, sn[4] = {t0[1], t0[3], t1[1], t1[3]};
+    half8 r;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const float x0 = (float)x[2 * u], x1 = (float)x[2 * u + 1];
+        r[2 * u] = (f16)(x0 * cs[u] - x1 * sn[u]);
+        r[2 * u + 1] = (f16)(x0 * sn[u] + x1 * cs[u]);
+    }
+    return r;
+}
+
 // Workgroup w runs on XCD w % 8; each XCD takes a contiguous range of tiles
 // (the first total % 8 XCDs one more than the others).
 DEV int xcd_tile(int w, int total) {
@@ -397,6 +412,30 @@ __global__ __launch_bounds__(64 * NWV * KG, 1) void gemm_mfma(GemmArgs p, int ti
         stage([](float v, const f16*) { return v; });
     }
     wave_lds();
+    if constexpr (!TA && !TB) {
+        if (p.epi == GEMM_QKV) {
+            // a lane's chunks are 8 columns of one head, all at the same place
+            // of a row; memory-bound on the five outputs.  As a pass of its own
+            // behind this product the same work took 4.4 us (1000 x 768); a
+            // prefill of 12 such layers 847 -> 824 us.
+            const QkvDest& o = p.qkv;
+            const int d = N / 3, col = n0 + wn0 + (lane % CPR) * 8;
+            if (col >= N) return;
+            const int which = col / d, c = col % d, h = c / o.dh, j = c % o.dh;
+            f16* const head = (which == 0 ? o.q : which == 1 ? o.k : o.v) + (int64_t)h * M * o.dh + j;
+            f16* const cache = (which == 1 ? o.kc : o.vc) + c;
+#pragma unroll
+            for (int q = 0; q < CQ; ++q) {
+                const int r = (lane + 64 * q) / CPR, row = m0 + wm0 + r;
+                if (row >= M) continue;
+                half8 x = *reinterpret_cast<const half8*>(ot + r * OUT_LD + (lane % CPR) * 8);
+                if (which < 2) x = rope8(x, o.rope + ((int64_t)row * o.dh + j) / 2);
+                *reinterpret_cast<half8*>(head + (int64_t)row * o.dh) = x;
+                if (which > 0) *reinterpret_cast<half8*>(cache + (int64_t)row * d) = x;
+            }
+            return;
+        }
+    }
     each_chunk([&](int, f16* c, const f16* o, int left) {
         const u32x4 v = *reinterpret_cast<const u32x4*>(o);
         if constexpr (RAG) {

@@ -6,6 +6,13 @@
 namespace evkhip {
 
 // ---- gemm.hip ----
+// GEMM_QKV: where the columns of X.Wqkv (M rows: positions 0..M-1; N = 3 d) go
+struct QkvDest {
+    const float2* rope;  // (cos, sin) of pair p of row i at [i * dh / 2 + p]
+    f16 *q, *k, *v;      // per head: (heads, M, dh), q and k rotated
+    f16 *kc, *vc;        // cache rows 0..M-1: (M, d)
+    int dh;              // head size, a multiple of 8
+};
 struct GemmArgs {
     const f16* A;
     const f16* B;
@@ -14,10 +21,13 @@ struct GemmArgs {
     int64_t sA, sB, sC;  // per-batch element strides (0 = broadcast)
     int acc;             // C = fp16(C + A B)
     int epi;             // GEMM_*, without acc
+    QkvDest qkv;         // GEMM_QKV (C is not written)
 };
 // Ops folded into the store of a product, with the roundings of the separate
-// ops: C = fp16(C + fp16(A B)) and C = fp16(gelu(fp16(A B))).
-enum { GEMM_STORE = 0, GEMM_RESIDUAL = 1, GEMM_GELU = 2 };
+// ops: C = fp16(C + fp16(A B)), C = fp16(gelu(fp16(A B))), and rope of the q
+// and k columns of fp16(A B), regrouped per head and into the cache (A and B
+// row-major, N % 24 == 0).
+enum { GEMM_STORE = 0, GEMM_RESIDUAL = 1, GEMM_GELU = 2, GEMM_QKV = 3 };
 // Caller-provided split-K scratch of the skinny (M <= 16) path: partials and
 // arrival counters.  With it, gemm_dispatch allocates nothing.
 struct GemvScratch {

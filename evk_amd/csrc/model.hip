@@ -27,7 +27,7 @@ __global__ __launch_bounds__(256) void copy_k(const u32x4* src, u32x4* dst, int6
 
 // rope_k's angles of positions 0..n-1: (cos, sin) of pair p of row i at
 // table[i * dh / 2 + p].  One launch for all layers of a prefill: powf and
-// sincosf take longer than the data that prefill_split_k moves.
+// sincosf take longer than the rotation itself.
 __global__ __launch_bounds__(256) void rope_table_k(float2* table, int n, int dh, float base) {
     const int gid = blockIdx.x * 256 + threadIdx.x;
     const int pairs = dh / 2;
@@ -37,44 +37,6 @@ __global__ __launch_bounds__(256) void rope_table_k(float2* table, int n, int dh
     float sn, cs;
     sincosf((float)i * inv_freq, &sn, &cs);
     table[gid] = float2{cs, sn};
-}
-
-// Batched prefill: rows i of qkv (n, 3d) are positions i.  q and k are
-// rotated as rope_k does (pairs within a head, fp32, one fp16 rounding),
-// q, k, v are regrouped per head as (heads, n, dh) for the flash kernels, and
-// the k, v rows go to the cache at their positions.  One thread per 8 columns
-// (dh % 8 == 0), 16-byte accesses.  1000 x 768: 6.9 us with a thread per pair
-// that formed its angle itself, 4.4 now.
-__global__ __launch_bounds__(256) void prefill_split_k(const f16* qkv, const float2* table, int n, int d, int dh,
-                                                       f16* Qh, f16* Kh, f16* Vh, f16* Kc, f16* Vc) {
-    const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int pieces = d / 8;
-    if (gid >= (int64_t)n * pieces) return;
-    const int c = 8 * (int)(gid % pieces), i = (int)(gid / pieces);
-    const int h = c / dh, j = c % dh;
-    const f16* row = qkv + (int64_t)i * 3 * d + c;
-    const half8 q = *reinterpret_cast<const half8*>(row), k = *reinterpret_cast<const half8*>(row + d),
-                v = *reinterpret_cast<const half8*>(row + 2 * d);
-    const floatx4* t = reinterpret_cast<const floatx4*>(table + ((int64_t)i * dh + j) / 2);
-    const floatx4 t0 = t[0], t1 = t[1];
-    const float cs[4] = {t0[0], t0[2], t1[0], t1[2]}, sn[4] = {t0[1], t0[3], t1[1], t1[3]};
-    auto rotate = [&](const half8& x) {
-        half8 r;
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const float x0 = (float)x[2 * u], x1 = (float)x[2 * u + 1];
-            r[2 * u] = (f16)(x0 * cs[u] - x1 * sn[u]);
-            r[2 * u + 1] = (f16)(x0 * sn[u] + x1 * cs[u]);
-        }
-        return r;
-    };
-    const int64_t o = ((int64_t)h * n + i) * dh + j, oc = (int64_t)i * d + c;
-    const half8 kr = rotate(k);
-    *reinterpret_cast<half8*>(Qh + o) = rotate(q);
-    *reinterpret_cast<half8*>(Kh + o) = kr;
-    *reinterpret_cast<half8*>(Vh + o) = v;
-    *reinterpret_cast<half8*>(Kc + oc) = kr;
-    *reinterpret_cast<half8*>(Vc + oc) = v;
 }
 
 // (heads, n, dh) -> (n, heads * dh), 16 bytes per thread
@@ -882,10 +844,10 @@ int run_tokens_fused(const evkhip_model_cfg& c, const f16* E, const f16* Wout, u
 // rms_norm over the n rows, X.Wqkv on the MFMA GEMM, rope and the cache rows,
 // causal flash attention per head (heads as the batch), X.Wo, residual,
 // rms_norm, gelu(X.W1).W2, residual; then the last row's logits and greedy id.
-// The residuals and the gelu are part of the GEMMs' stores, and the attention
-// writes its rows where X.Wo reads them: eight launches a layer, not twelve
-// (1000 tokens, 12 layers of 768: 1029 -> 847 us with the GEMM instances that
-// came with it).  Same op sequence and fp16 rounding points as the token loop; the
+// Rope, the cache rows, the residuals and the gelu are part of the GEMMs'
+// stores, and the attention writes its rows where X.Wo reads them: seven
+// launches a layer, not twelve (1000 tokens, 12 layers of 768: 1029 -> 824 us
+// with the GEMM instances that came with it).  Same op sequence and fp16 rounding points as the token loop; the
 // GEMMs sum in another order.  Returns 1 when the shape is not taken (the token loop
 // serves it), an evkhip error code otherwise.
 int run_prefill_batched(const evkhip_model_cfg& c, const f16* E, const f16* Wout, uint64_t per_layer, f16* cache_h,
@@ -895,9 +857,9 @@ int run_prefill_batched(const evkhip_model_cfg& c, const f16* E, const f16* Wout
         (int64_t)n * hid * 2 >= INT32_MAX)
         return 1;
     const size_t nd = (size_t)n * d, nh = (size_t)n * hid;
-    // X, Hn, QKV (3), Qh, Kh, Vh, Oh, A: 10 n d; HG: n hidden; the rope table:
-    // n dh floats.  (d and hidden are multiples of 8: 16-byte aligned pieces.)
-    const size_t need = 10 * nd + nh + 2 * (size_t)n * dh;
+    // X, Hn, Qh, Kh, Vh, Oh, A: 7 n d; HG: n hidden; the rope table: n dh
+    // floats.  (d and hidden are multiples of 8: 16-byte aligned pieces.)
+    const size_t need = 7 * nd + nh + 2 * (size_t)n * dh;
     if (need * sizeof(f16) > ((size_t)1 << 31)) return 1;
     if (need > g_pws.elems) {
         if (g_pws.buf) EVK_HIP(hipFree(g_pws.buf));
@@ -908,16 +870,17 @@ int run_prefill_batched(const evkhip_model_cfg& c, const f16* E, const f16* Wout
     }
     f16* X = g_pws.buf;
     f16* Hn = X + nd;
-    f16* QKV = Hn + nd;  // 3 nd
-    f16* Qh = QKV + 3 * nd;
+    f16* Qh = Hn + nd;
     f16* Kh = Qh + nd;
     f16* Vh = Kh + nd;
     f16* Oh = Vh + nd;
     f16* A = Oh + nd;
     f16* HG = A + nd;
     float2* table = reinterpret_cast<float2*>(HG + nh);
-    auto gemm = [&](const f16* a, const f16* b, f16* out, int M, int N, int K, int epi = GEMM_STORE) {
+    auto gemm = [&](const f16* a, const f16* b, f16* out, int M, int N, int K, int epi = GEMM_STORE,
+                    const QkvDest& qkv = QkvDest{}) {
         GemmArgs g{};
+        g.qkv = qkv;
         g.A = a;
         g.B = b;
         g.C = out;
@@ -940,8 +903,7 @@ int run_prefill_batched(const evkhip_model_cfg& c, const f16* E, const f16* Wout
         f16* Kc = cache_h + (uint64_t)l * 2 * c.max_seq * d;
         f16* Vc = Kc + (uint64_t)c.max_seq * d;
         CHECK(rms_norm_launch(X, Hn, n, d, c.eps, st));
-        CHECK(gemm(Hn, Wqkv, QKV, (int)n, 3 * d, d));
-        hipLaunchKernelGGL(prefill_split_k, dim3(g_rows), dim3(256), 0, st, QKV, table, (int)n, d, dh, Qh, Kh, Vh, Kc, Vc);
+        CHECK(gemm(Hn, Wqkv, nullptr, (int)n, 3 * d, d, GEMM_QKV, QkvDest{table, Qh, Kh, Vh, Kc, Vc, dh}));
         FlashArgs fa{};
         fa.q = Qh;
         fa.k = Kh;
