@@ -451,9 +451,6 @@ __global__ __launch_bounds__(512) void flash_fwd(FlashArgs p, int round) {
 // row maxima of a rescale cross the wave's 16-lane rows by permlane swaps.
 // ---------------------------------------------------------------------------
 constexpr int KC = 32;  // keys per chunk
-#ifndef FWD_KS_QB
-#define FWD_KS_QB 4  // 16-row query blocks per wave (rows per workgroup / 16)
-#endif
 
 // Maximum over the four 16-lane rows of a wave (lanes 16 and 32 apart):
 // two row swaps on the VALU instead of cross-lane LDS permutes.
@@ -474,14 +471,18 @@ struct KsLayout {
     static constexpr int VPER = KC * DH / 8 / 64;  // 16-byte V pieces per lane
     static constexpr int OW = DH + 4;            // merge row stride (floats)
     // the merge area follows the V slots: a wave stores its partials as soon
-    // as its own loop ends, while other waves still use their slots.  Each
-    // wave stores the three 16-row blocks it does not finish, and m, l of all
-    // its rows.
+    // as its own loop ends, while other waves still use their slots.  Wave w
+    // finishes 16-row block w; each wave stores the blocks it does not finish
+    // (three of four, or in fixed slots where there are fewer blocks than
+    // waves), and m, l of all its rows.
     static constexpr int VBYTES = 4 * VSLOT * 2;
-    static constexpr int MERGE = 4 * (QB - 1) * 16 * OW + 2 * 4 * ROWS;  // floats
+    static constexpr int SLOTS = QB == 4 ? 3 : QB;
+    static constexpr int MERGE = 4 * SLOTS * 16 * OW + 2 * 4 * ROWS;  // floats
+    static __device__ __forceinline__ int slot(int wave, int qb) { return QB == 4 && qb > wave ? qb - 1 : qb; }
     static constexpr int LDS_BYTES = VBYTES + MERGE * 4;
 };
 
+// QB: 16-row query blocks per tile, 4 or 2 (launch_fwd).
 // STRIDED: O rows at out_bstride / out_rstride instead of contiguous.
 template <int DH, int QB, bool CAUSAL, bool STRIDED = false>
 __global__ __launch_bounds__(512, 1) void flash_fwd_ks(FlashArgs p) {
@@ -579,7 +580,8 @@ __global__ __launch_bounds__(512, 1) void flash_fwd_ks(FlashArgs p) {
     int qpos[QB];
     {
         constexpr int QPIECES = ROWS * DH / 8;           // 16-byte pieces of the tile
-        constexpr int QPER = QPIECES / 256;
+        constexpr int QPER = (QPIECES + 255) / 256;       // pieces past the tile: zeros into unused V slots
+        static_assert(QPER * 256 / (DH / 8) <= 4 * KC, "the pieces fit the V slots");
         f16* qs = vslot_all;                              // [ROWS][DH + 8]
         const int ht = threadIdx.x & 255;
         u32x4 qv[QPER];
@@ -708,10 +710,15 @@ __global__ __launch_bounds__(512, 1) void flash_fwd_ks(FlashArgs p) {
             auto mx3 = [](half2_t a, half2_t b, half2_t c) {
                 return __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, b), c);
             };
-            static_assert(QB == 4, "16 packed values");
-            const half2_t h5[6] = {mx3(hv[0], hv[1], hv[2]), mx3(hv[3], hv[4], hv[5]), mx3(hv[6], hv[7], hv[8]),
-                                   mx3(hv[9], hv[10], hv[11]), mx3(hv[12], hv[13], hv[14]), hv[15]};
-            const half2_t h = mx3(mx3(h5[0], h5[1], h5[2]), mx3(h5[3], h5[4], h5[5]), h5[0]);
+            static_assert(QB == 4 || QB == 2, "16 or 8 packed values");
+            half2_t h;
+            if constexpr (QB == 4) {
+                const half2_t h5[6] = {mx3(hv[0], hv[1], hv[2]), mx3(hv[3], hv[4], hv[5]), mx3(hv[6], hv[7], hv[8]),
+                                       mx3(hv[9], hv[10], hv[11]), mx3(hv[12], hv[13], hv[14]), hv[15]};
+                h = mx3(mx3(h5[0], h5[1], h5[2]), mx3(h5[3], h5[4], h5[5]), h5[0]);
+            } else {
+                h = mx3(mx3(hv[0], hv[1], hv[2]), mx3(hv[3], hv[4], hv[5]), mx3(hv[6], hv[7], hv[0]));
+            }
             need |= __builtin_fmaxf((float)h[0], (float)h[1]) > (float)(1 << (int)RESCALE_LOG2);
         }
         if (__builtin_expect(__any(need), 0)) {
@@ -784,13 +791,12 @@ __global__ __launch_bounds__(512, 1) void flash_fwd_ks(FlashArgs p) {
                                   __HIP_MEMORY_SCOPE_AGENT);
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
     };
-    static_assert(QB == 4, "one 16-row block per wave of the half");
-    float* ob = smem_f + L::VBYTES / 4;          // [wave][3 blocks][16][OW]
-    float* mw = ob + 4 * (QB - 1) * 16 * L::OW;  // [wave][ROWS]
+    static_assert(QB <= 4, "at most one 16-row block per wave of the half");
+    float* ob = smem_f + L::VBYTES / 4;          // [wave][SLOTS][16][OW]
+    float* mw = ob + 4 * L::SLOTS * 16 * L::OW;  // [wave][ROWS]
     float* lw = mw + 4 * ROWS;                   // [wave][ROWS]
-    // wave w finishes the rows of its block qb = w; it stores the other
-    // blocks' partial state for the waves that finish them (block qb in its
-    // slot qb, or qb - 1 past its own) and keeps its own
+    // wave w < QB finishes the rows of its block qb = w; it stores the other
+    // blocks' partial state for the waves that finish them and keeps its own
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
         const int q = qb * 16 + ml16;
@@ -799,14 +805,15 @@ __global__ __launch_bounds__(512, 1) void flash_fwd_ks(FlashArgs p) {
             lw[wave * ROWS + q] = lacc[qb][0];
         }
         if (qb != wave) {
-            const int k = qb < wave ? qb : qb - 1;
+            const int k = L::slot(wave, qb);
 #pragma unroll
             for (int d = 0; d < DB; ++d)
-                *reinterpret_cast<floatx4*>(ob + ((wave * (QB - 1) + k) * 16 + ml16) * L::OW + d * 16 + mg * 4) =
+                *reinterpret_cast<floatx4*>(ob + ((wave * L::SLOTS + k) * 16 + ml16) * L::OW + d * 16 + mg * 4) =
                     oacc[d][qb];
         }
     }
     half_sync(4);
+    if (QB < 4 && wave >= QB) return;  // no block of its own; past the last barrier
     // lane (mg, ml16): row q = 16 wave + ml16, dh 16 d + 4 mg + j.  Every LDS
     // read of the merge (m, l of the four waves, the three other waves'
     // blocks) is issued before any is used.
@@ -817,12 +824,12 @@ __global__ __launch_bounds__(512, 1) void flash_fwd_ks(FlashArgs p) {
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
         const int w = j < wave ? j : j + 1;        // the j-th other wave
-        const int k = wave < w ? wave : wave - 1;  // this block's slot in wave w
+        const int k = L::slot(w, wave);            // this block's slot in wave w
         mv[j] = mw[w * ROWS + q];
         lv[j] = lw[w * ROWS + q];
 #pragma unroll
         for (int d = 0; d < DB; ++d)
-            r[j][d] = *reinterpret_cast<const floatx4*>(ob + ((w * (QB - 1) + k) * 16 + ml16) * L::OW + d * 16 + mg * 4);
+            r[j][d] = *reinterpret_cast<const floatx4*>(ob + ((w * L::SLOTS + k) * 16 + ml16) * L::OW + d * 16 + mg * 4);
     }
     // the wave's own block qb = wave, from registers (static indices)
     floatx4 a[DB];
@@ -2327,6 +2334,12 @@ __global__ __launch_bounds__(256) void flash_bwd_pre_scalar(FlashArgs p, int Dh)
 char* g_bwd_ws = nullptr;
 size_t g_bwd_ws_bytes = 0;
 
+// Workgroups of flash_fwd_ks: pairs of tiles of 16 qb rows.
+inline int64_t fwd_ks_pairs(const FlashArgs& a, int qb) {
+    const int64_t tiles = ((int64_t)a.N * a.H + 16 * qb - 1) / (16 * qb);
+    return (tiles + 1) / 2 * a.B;
+}
+
 template <int DH>
 hipError_t launch_fwd(const FlashArgs& a, bool causal, int mode, hipStream_t st) {
     const int nrg = (a.N * a.H + FR - 1) / FR;
@@ -2337,13 +2350,22 @@ hipError_t launch_fwd(const FlashArgs& a, bool causal, int mode, hipStream_t st)
     if constexpr (DH <= 64) {
         // buffer offsets are 32-bit: one batch of K (or V) must stay below 2 GiB
         if (mode == 0 && (int64_t)a.N * DH * 2 < (int64_t)INT32_MAX) {
-            constexpr int QB = FWD_KS_QB;
-            const int64_t nrg_ks = ((int64_t)a.N * a.H + 16 * QB - 1) / (16 * QB);
-            dim3 gk((unsigned)((nrg_ks + 1) / 2 * a.B));
             if (a.out_rstride && !causal) return hipErrorInvalidValue;  // prefill is causal
-            if (a.out_rstride) hipLaunchKernelGGL((flash_fwd_ks<DH, QB, true, true>), gk, dim3(512), 0, st, a);
-            else if (causal) hipLaunchKernelGGL((flash_fwd_ks<DH, QB, true>), gk, dim3(512), 0, st, a);
-            else hipLaunchKernelGGL((flash_fwd_ks<DH, QB, false>), gk, dim3(512), 0, st, a);
+            auto launch = [&](auto qbc) {
+                constexpr int QB = decltype(qbc)::value;
+                const dim3 g((unsigned)fwd_ks_pairs(a, QB));
+                if (a.out_rstride) hipLaunchKernelGGL((flash_fwd_ks<DH, QB, true, true>), g, dim3(512), 0, st, a);
+                else if (causal) hipLaunchKernelGGL((flash_fwd_ks<DH, QB, true>), g, dim3(512), 0, st, a);
+                else hipLaunchKernelGGL((flash_fwd_ks<DH, QB, false>), g, dim3(512), 0, st, a);
+            };
+            // Tiles of 32 rows while 64-row pairs leave half of the CUs idle:
+            // twice the workgroups, each wave with half the products and
+            // exponentials per chunk.  us, 64 rows -> 32, causal and not:
+            // 12 heads of 64 with 1000 keys 10.5 -> 8.8, 13.7 -> 12.7; B=1
+            // N=600 H=4 8.2 -> 6.3, 9.9 -> 8.3; Dh 32, B=8 N=1000 7.9 -> 6.0,
+            // 9.9 -> 6.9.  With more pairs 64-row tiles read K and V less often.
+            if (2 * fwd_ks_pairs(a, 4) <= device_cu_count()) launch(std::integral_constant<int, 2>{});
+            else launch(std::integral_constant<int, 4>{});
             return hipGetLastError();
         }
     }

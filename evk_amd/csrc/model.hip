@@ -847,8 +847,8 @@ int run_tokens_fused(const evkhip_model_cfg& c, const f16* E, const f16* Wout, u
 // Rope, the cache rows, the residuals and the gelu are part of the GEMMs'
 // stores, and the attention writes its rows where X.Wo reads them: seven
 // launches a layer, not twelve (1000 tokens, 12 layers of 768: 1029 -> 824 us
-// with the GEMM instances that came with it).  Same op sequence and fp16 rounding points as the token loop; the
-// GEMMs sum in another order.  Returns 1 when the shape is not taken (the token loop
+// with the GEMM instances that came with it).  Same op sequence and fp16
+// rounding points as the token loop; the GEMMs sum in another order.  Returns 1 when the shape is not taken (the token loop
 // serves it), an evkhip error code otherwise.
 int run_prefill_batched(const evkhip_model_cfg& c, const f16* E, const f16* Wout, uint64_t per_layer, f16* cache_h,
                         const uint16_t* feed, uint16_t* ids, uint32_t n, f16* logits, hipStream_t st) {

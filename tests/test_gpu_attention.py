@@ -430,6 +430,23 @@ def test_sq_attention_splits(dev, orc, dh, L):
             assert_close_f16(from_dev(O)[b], orc.sq_attention(q[b], kc[b], vc[b], L, heads), what=f"dh={dh} L={L} b={b}")
 
 
+@pytest.mark.parametrize("Dh", [32, 64])
+@pytest.mark.parametrize("B,N,H", [(1, 1, 1), (1, 15, 1), (2, 33, 1), (3, 257, 3), (128, 100, 1), (129, 100, 1), (64, 65, 4)])
+@pytest.mark.parametrize("causal", [True, False])
+def test_forward_tile_heights(dev, orc, Dh, B, N, H, causal):
+    """Tiles of 32 and of 64 query rows, both sides of the line between them
+    on 256 CUs; fewer rows than a tile, an odd number of tiles, a partial last
+    one, and a score that moves a row's reference late (large last key)."""
+    import evk_amd as evk
+    q, k, v = orc.normal_f16((B, N, H * Dh), 391 + N), orc.normal_f16((B, N, Dh), 392 + N), orc.normal_f16((B, N, Dh), 393 + N)
+    k[0, -1] = f16(4.0 * f32(k[0, -1]))
+    o, lse = fwd(evk, dev, q, k, v, causal)
+    for b in sorted({0, B // 2, B - 1}):
+        want, wl = orc.attention_fwd(q[b:b + 1], k[b:b + 1], v[b:b + 1], causal)
+        assert_close_f16(o[b:b + 1], want, what=f"o b={b}")
+        assert np.abs(lse[b] - wl[0]).max() <= 1e-3
+
+
 @pytest.mark.parametrize("L", [1, 30, 63, 100, 700])
 def test_sq_attention_infinity_in_last_row(dev, orc, L):
     """An infinity in a sequence's last value row reaches the output as one:

@@ -512,3 +512,26 @@ def test_greedy_long_rows(dev, orc, V, base, count):
                 best, bj = key, j
         want.append(base + bj)
     assert list(got) == want
+
+
+@pytest.mark.parametrize("heads,dh", [(3, 48), (5, 32), (3, 64), (1, 128), (1, 256)])
+@pytest.mark.parametrize("n", [16, 17, 65])
+def test_prefill_cache_rows(dev, orc, heads, dh, n):
+    """The QKV product's store (rope, heads, cache rows): heads that straddle
+    column tiles, partial row tiles, every cache row of both layers, and rows
+    past the prompt left alone."""
+    import evk_amd as evk
+    import torch
+    kw = dict(vocab=136, d=heads * dh, heads=heads, layers=2, hidden=72, max_seq=n + 2)
+    ocfg, cfg = orc.model_cfg(**kw), evk.model_cfg(**kw)
+    w = orc.model_weights(ocfg, seed=401 + dh, std=0.1)
+    prompt = orc.tokens_u16(n, 402 + n, 136)
+    cache = torch.zeros(evk.model_cache_elems(cfg), dtype=torch.float16, device=dev)
+    tok, logits = torch.zeros(1, dtype=torch.int16, device=dev), torch.empty(136, dtype=torch.float16, device=dev)
+    evk.model_prefill(cfg, to_dev(w, dev), cache, torch.from_numpy(prompt.view(np.int16)).to(dev), 0, tok, logits)
+    torch.cuda.synchronize()
+    _, want_cache, want_logits = orc.model_generate(ocfg, w, prompt, 0, return_logits=True)
+    got = from_dev(cache).reshape(2, 2, n + 2, heads * dh)
+    assert_close_f16(got, want_cache.reshape(got.shape), what="cache")
+    assert not got[:, :, n:].any()
+    assert_close_f16(from_dev(logits), want_logits[0], what="logits")
