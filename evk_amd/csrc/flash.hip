@@ -484,8 +484,12 @@ struct KsLayout {
 
 // QB: 16-row query blocks per tile, 4 or 2 (launch_fwd).
 // STRIDED: O rows at out_bstride / out_rstride instead of contiguous.
-template <int DH, int QB, bool CAUSAL, bool STRIDED = false>
+// SOLO (QB 2): a workgroup runs one tile, its eight waves every eighth chunk
+// of the keys, instead of a pair of tiles on four waves each.
+template <int DH, int QB, bool CAUSAL, bool STRIDED = false, bool SOLO = false>
 __global__ __launch_bounds__(512, 1) void flash_fwd_ks(FlashArgs p) {
+    static_assert(!SOLO || QB == 2, "a slot for every block of every wave");
+    constexpr int KW = SOLO ? 8 : 4;  // waves that share a tile's keys
     using L = KsLayout<DH, QB>;
     constexpr int ROWS = L::ROWS;
     constexpr int KS = L::KS, DB = L::DB, VW = L::VW, VPER = L::VPER;
@@ -506,8 +510,8 @@ __global__ __launch_bounds__(512, 1) void flash_fwd_ks(FlashArgs p) {
     // runs (id mod 8) then share the K/V of few batches in its L2
     const int b = blockIdx.x % p.B, pq = blockIdx.x / p.B;
     const int half = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
-    const int rg = half == 0 ? nrg - 1 - pq : pq;
-    const bool active = half == 0 || rg != nrg - 1 - pq;  // odd nrg: the middle tile runs once
+    const int rg = SOLO || half == 0 ? nrg - 1 - pq : pq;
+    const bool active = SOLO || half == 0 || rg != nrg - 1 - pq;  // odd nrg: the middle tile runs once
     float* smem_f = smem_all + half * (L::LDS_BYTES / 4);
     f16* vslot_all = reinterpret_cast<f16*>(smem_f);
     const int lane = threadIdx.x & 63;
@@ -565,8 +569,8 @@ __global__ __launch_bounds__(512, 1) void flash_fwd_ks(FlashArgs p) {
     // start is bound by the burst of first requests from every CU, and the
     // heavy tile carries the workgroup's critical path (Q staged 2.4 -> 1.9
     // us, 13.0 -> 12.5 us per C2 launch).
-    int c = wave;
-    const bool late = CAUSAL && half == 1;
+    int c = SOLO ? 4 * half + wave : wave;
+    const bool late = CAUSAL && !SOLO && half == 1;
     // Every wave issues these requests (the late ones get the empty
     // descriptor): with no branch around them the staging's wait counts
     // stay exact, and the Q staging waits for the Q loads alone, not for the
@@ -644,7 +648,7 @@ __global__ __launch_bounds__(512, 1) void flash_fwd_ks(FlashArgs p) {
             const int idx = lane + 64 * i;
             *reinterpret_cast<u32x4*>(vslot + (idx / (DH / 8)) * VW + (idx % (DH / 8)) * 8) = vr[i];
         }
-        if (c + 4 < nch) load_v(c + 4);
+        if (c + KW < nch) load_v(c + KW);
         // V^T fragments read back at once (after the slot's writes, in
         // order): their latency hides behind the score MFMAs
         half8 vt[DB];
@@ -664,7 +668,7 @@ __global__ __launch_bounds__(512, 1) void flash_fwd_ks(FlashArgs p) {
                     s[kb][qb] = mfma16(as_half8(kr[kb][ks]), qf[qb][ks], ks == 0 ? floatx4{0.0f, 0.0f, 0.0f, 0.0f} : s[kb][qb]);
         // the K registers are free once the score MFMAs have read them: the
         // next chunk's K goes straight into them (no copy)
-        if (c + 4 < nch) load_k(c + 4);
+        if (c + KW < nch) load_k(c + KW);
         // element j of s[kb][qb]: key key0 + 16 kb + 4 g + j, query row R0 + 16 qb + l16
         if constexpr (MASK) {
 #pragma unroll
@@ -759,8 +763,8 @@ __global__ __launch_bounds__(512, 1) void flash_fwd_ks(FlashArgs p) {
         }
     };
     const int c_mask = __builtin_amdgcn_readfirstlane(min(nch, cu));
-    for (; c < c_mask; c += 4) chunk(c, std::false_type{});
-    for (; c < nch; c += 4) chunk(c, std::true_type{});
+    for (; c < c_mask; c += KW) chunk(c, std::false_type{});
+    for (; c < nch; c += KW) chunk(c, std::true_type{});
 
     // ---- merge the four waves' partial softmax states ----
     // Each wave stores its state as it stands (m, l and O relative to its own
@@ -804,7 +808,7 @@ __global__ __launch_bounds__(512, 1) void flash_fwd_ks(FlashArgs p) {
             mw[wave * ROWS + q] = mref(qb);
             lw[wave * ROWS + q] = lacc[qb][0];
         }
-        if (qb != wave) {
+        if (qb != wave || (SOLO && half == 1)) {
             const int k = L::slot(wave, qb);
 #pragma unroll
             for (int d = 0; d < DB; ++d)
@@ -812,24 +816,26 @@ __global__ __launch_bounds__(512, 1) void flash_fwd_ks(FlashArgs p) {
                     oacc[d][qb];
         }
     }
-    half_sync(4);
-    if (QB < 4 && wave >= QB) return;  // no block of its own; past the last barrier
+    if constexpr (SOLO) __syncthreads();
+    else half_sync(4);
+    if ((QB < 4 && wave >= QB) || (SOLO && half == 1)) return;  // no block of its own; past the last barrier
     // lane (mg, ml16): row q = 16 wave + ml16, dh 16 d + 4 mg + j.  Every LDS
     // read of the merge (m, l of the four waves, the three other waves'
     // blocks) is issued before any is used.
     const int q = wave * 16 + ml16;
     const float mo = mw[wave * ROWS + q], lo = lw[wave * ROWS + q];
-    float mv[3], lv[3];
-    floatx4 r[3][DB];
+    float mv[KW - 1], lv[KW - 1];
+    floatx4 r[KW - 1][DB];
 #pragma unroll
-    for (int j = 0; j < 3; ++j) {
-        const int w = j < wave ? j : j + 1;        // the j-th other wave
-        const int k = L::slot(w, wave);            // this block's slot in wave w
-        mv[j] = mw[w * ROWS + q];
-        lv[j] = lw[w * ROWS + q];
+    for (int j = 0; j < KW - 1; ++j) {
+        const int w = j < wave ? j : j + 1;          // the j-th other wave
+        const int at = SOLO && w >= 4 ? L::LDS_BYTES / 4 : 0;  // the other half's area
+        const int k = L::slot(w & 3, wave);          // this block's slot in wave w
+        mv[j] = mw[at + (w & 3) * ROWS + q];
+        lv[j] = lw[at + (w & 3) * ROWS + q];
 #pragma unroll
         for (int d = 0; d < DB; ++d)
-            r[j][d] = *reinterpret_cast<const floatx4*>(ob + ((w * L::SLOTS + k) * 16 + ml16) * L::OW + d * 16 + mg * 4);
+            r[j][d] = *reinterpret_cast<const floatx4*>(ob + at + (((w & 3) * L::SLOTS + k) * 16 + ml16) * L::OW + d * 16 + mg * 4);
     }
     // the wave's own block qb = wave, from registers (static indices)
     floatx4 a[DB];
@@ -840,13 +846,15 @@ __global__ __launch_bounds__(512, 1) void flash_fwd_ks(FlashArgs p) {
             for (int d = 0; d < DB; ++d) a[d] = oacc[d][qb];
         }
     });
-    const float m = fmaxf(fmaxf(mo, mv[0]), fmaxf(mv[1], mv[2]));
+    float m = mo;
+#pragma unroll
+    for (int j = 0; j < KW - 1; ++j) m = fmaxf(m, mv[j]);
     const float so = mo == -INFINITY ? 0.0f : fast_exp2(mo - m);
     float l = so * lo;
 #pragma unroll
     for (int d = 0; d < DB; ++d) a[d] *= so;
 #pragma unroll
-    for (int j = 0; j < 3; ++j) {
+    for (int j = 0; j < KW - 1; ++j) {
         const float sc = mv[j] == -INFINITY ? 0.0f : fast_exp2(mv[j] - m);
         l += sc * lv[j];
 #pragma unroll
@@ -2334,11 +2342,9 @@ __global__ __launch_bounds__(256) void flash_bwd_pre_scalar(FlashArgs p, int Dh)
 char* g_bwd_ws = nullptr;
 size_t g_bwd_ws_bytes = 0;
 
-// Workgroups of flash_fwd_ks: pairs of tiles of 16 qb rows.
-inline int64_t fwd_ks_pairs(const FlashArgs& a, int qb) {
-    const int64_t tiles = ((int64_t)a.N * a.H + 16 * qb - 1) / (16 * qb);
-    return (tiles + 1) / 2 * a.B;
-}
+// Tiles of 16 qb rows of a batch, and flash_fwd_ks's pairs of them over all batches.
+inline int64_t fwd_ks_tiles(const FlashArgs& a, int qb) { return ((int64_t)a.N * a.H + 16 * qb - 1) / (16 * qb); }
+inline int64_t fwd_ks_pairs(const FlashArgs& a, int qb) { return (fwd_ks_tiles(a, qb) + 1) / 2 * a.B; }
 
 template <int DH>
 hipError_t launch_fwd(const FlashArgs& a, bool causal, int mode, hipStream_t st) {
@@ -2351,21 +2357,32 @@ hipError_t launch_fwd(const FlashArgs& a, bool causal, int mode, hipStream_t st)
         // buffer offsets are 32-bit: one batch of K (or V) must stay below 2 GiB
         if (mode == 0 && (int64_t)a.N * DH * 2 < (int64_t)INT32_MAX) {
             if (a.out_rstride && !causal) return hipErrorInvalidValue;  // prefill is causal
-            auto launch = [&](auto qbc) {
+            auto launch = [&](auto qbc, auto solo) {
                 constexpr int QB = decltype(qbc)::value;
-                const dim3 g((unsigned)fwd_ks_pairs(a, QB));
-                if (a.out_rstride) hipLaunchKernelGGL((flash_fwd_ks<DH, QB, true, true>), g, dim3(512), 0, st, a);
-                else if (causal) hipLaunchKernelGGL((flash_fwd_ks<DH, QB, true>), g, dim3(512), 0, st, a);
-                else hipLaunchKernelGGL((flash_fwd_ks<DH, QB, false>), g, dim3(512), 0, st, a);
+                constexpr bool SOLO = decltype(solo)::value;
+                const dim3 g((unsigned)(SOLO ? fwd_ks_tiles(a, QB) * a.B : fwd_ks_pairs(a, QB)));
+                if (a.out_rstride) hipLaunchKernelGGL((flash_fwd_ks<DH, QB, true, true, SOLO>), g, dim3(512), 0, st, a);
+                else if (causal) hipLaunchKernelGGL((flash_fwd_ks<DH, QB, true, false, SOLO>), g, dim3(512), 0, st, a);
+                else hipLaunchKernelGGL((flash_fwd_ks<DH, QB, false, false, SOLO>), g, dim3(512), 0, st, a);
             };
+            // A 32-row tile on all eight waves of a workgroup while every
+            // tile gets a CU of its own (a pair on one CU would leave another
+            // idle).  us, pairs -> one tile, causal and not: 8 heads of 64
+            // with 1024 keys 8.5 -> 7.9, 12.3 -> 8.3; B=1 N=4000 H=2 21.0 ->
+            // 20.4, 37.6 -> 20.8; Dh 32, B=8 N=1000 6.0 -> 5.2, 6.9 -> 5.2.
+            const int64_t cus = device_cu_count();
+            if (fwd_ks_tiles(a, 2) * a.B <= cus) {
+                launch(std::integral_constant<int, 2>{}, std::true_type{});
+                return hipGetLastError();
+            }
             // Tiles of 32 rows while 64-row pairs leave half of the CUs idle:
             // twice the workgroups, each wave with half the products and
             // exponentials per chunk.  us, 64 rows -> 32, causal and not:
             // 12 heads of 64 with 1000 keys 10.5 -> 8.8, 13.7 -> 12.7; B=1
             // N=600 H=4 8.2 -> 6.3, 9.9 -> 8.3; Dh 32, B=8 N=1000 7.9 -> 6.0,
             // 9.9 -> 6.9.  With more pairs 64-row tiles read K and V less often.
-            if (2 * fwd_ks_pairs(a, 4) <= device_cu_count()) launch(std::integral_constant<int, 2>{});
-            else launch(std::integral_constant<int, 4>{});
+            if (2 * fwd_ks_pairs(a, 4) <= cus) launch(std::integral_constant<int, 2>{}, std::false_type{});
+            else launch(std::integral_constant<int, 4>{}, std::false_type{});
             return hipGetLastError();
         }
     }

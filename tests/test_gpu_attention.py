@@ -431,11 +431,12 @@ def test_sq_attention_splits(dev, orc, dh, L):
 
 
 @pytest.mark.parametrize("Dh", [32, 64])
-@pytest.mark.parametrize("B,N,H", [(1, 1, 1), (1, 15, 1), (2, 33, 1), (3, 257, 3), (128, 100, 1), (129, 100, 1), (64, 65, 4)])
+@pytest.mark.parametrize("B,N,H", [(1, 1, 1), (1, 15, 1), (2, 33, 1), (3, 257, 3), (128, 100, 1), (129, 100, 1), (64, 65, 4), (64, 100, 1),
+                                   (65, 100, 1), (2, 700, 2)])
 @pytest.mark.parametrize("causal", [True, False])
 def test_forward_tile_heights(dev, orc, Dh, B, N, H, causal):
-    """Tiles of 32 and of 64 query rows, both sides of the line between them
-    on 256 CUs; fewer rows than a tile, an odd number of tiles, a partial last
+    """Tiles of 32 query rows on eight and on four waves and of 64 rows, both
+    sides of the lines between them on 256 CUs; fewer rows than a tile, an odd number of tiles, a partial last
     one, and a score that moves a row's reference late (large last key)."""
     import evk_amd as evk
     q, k, v = orc.normal_f16((B, N, H * Dh), 391 + N), orc.normal_f16((B, N, Dh), 392 + N), orc.normal_f16((B, N, Dh), 393 + N)
