@@ -20,6 +20,7 @@
 //                 lane owns one key column; dV^T += dO^T P and dK^T += Q^T dS
 //                 read dO^T / Q^T from a per-wave transposed LDS tile.
 // Softmax runs in the exp2 domain: s2 = s * scale * log2(e).
+#include "flash_parts.h"
 #include "kernels.h"
 
 #include <algorithm>
@@ -915,32 +916,6 @@ DEV float dot8_pairs(const half8& x, const half8& y) {
     for (int e = 0; e < 8; e += 2)
         acc = __builtin_amdgcn_fdot2(half2_t{x[e], x[e + 1]}, half2_t{y[e], y[e + 1]}, acc, false);
     return acc;
-}
-
-constexpr int BKB = 128;       // keys per workgroup (4 waves x 32)
-constexpr int BRC = 32;        // flattened query rows per chunk
-// Chunks per row part, as a power of two: as long as leaves about 128 parts
-// (fewer fp32 partials to write and read) and short enough that a small call
-// still spreads over the chip.  Head sizes up to 64 stop at 16: two workgroups
-// share a CU there, and longer parts lengthen the launch.  Forward and
-// backward, us with this rule and with parts of 16 throughout: Dh 128, B=2
-// N=2000 H=8 163 and 177, B=16 N=160 H=4 27.5 and 40.1, B=1 N=130 H=2 22.3
-// and 26.6; Dh 64, B=1 N=600 H=4 24.5 and 33.7, B=16 N=160 H=4 20.9 and 32.3;
-// Dh 32, B=1 N=888 H=1 19.9 and 27.7.
-inline int bwd_part_log2(int dh, int64_t chunks) {
-    const int most = dh <= 64 ? 4 : 6;
-    int l = 2;
-    while (l < most && (chunks >> (l + 1)) >= 96) ++l;
-    return l;
-}
-
-// Chunks of flattened rows that key block kb of a batch interacts with.
-__host__ __device__ inline int bwd_kv_chunks(int kb, int N, int H, bool causal) {
-    const int64_t r_lo = causal ? (int64_t)kb * BKB * H : 0;
-    return (int)(((int64_t)N * H - r_lo + BRC - 1) / BRC);
-}
-__host__ __device__ inline int bwd_kv_parts(int kb, int N, int H, bool causal, int part_log2) {
-    return (bwd_kv_chunks(kb, N, H, causal) + (1 << part_log2) - 1) >> part_log2;
 }
 
 template <int DH>
@@ -1901,8 +1876,8 @@ DEV void bwd_q_pair_body(const FlashArgs& p, int blk, char* lds) {
 // dK/dV part takes about 1.4 us for 1024 cycles of MFMA per SIMD; chunks whose
 // loads all hit the L2 take as long, and the unmasked form and v_dot2 row sums
 // took off 6 us.
-// PL: part_log2 where it is known at compile time (16 chunks, the length of the
-// larger calls up to head size 64: 1 % at B=4 N=1024 H=8), or 0.
+// PL: part_log2 where it is known at compile time (16 chunks, the length of most
+// calls up to head size 64: 1 % at B=4 N=1024 H=8), or 0.
 template <int DH, bool CAUSAL, int PL>
 __global__ __launch_bounds__(DH <= 64 ? 256 : 512, 2) void flash_bwd_kvq(FlashArgs p, float* part_ws, int parts_per_batch,
                                                                         int n_kv) {
@@ -1914,9 +1889,15 @@ __global__ __launch_bounds__(DH <= 64 ? 256 : 512, 2) void flash_bwd_kvq(FlashAr
         // evenly, XCD x takes the dK/dV parts of batch x / (8 / B) only
         // (every (8 / B)-th part, heavy key blocks first), so the key blocks
         // that re-read a batch's Q, dO and O rows find them in that XCD's L2.
+        // Key blocks of one part each differ in length by the causal mask:
+        // the heavy ones of every batch go first (B=128 N=2048 H=8 causal
+        // 8520 -> 7226 us against batch after batch), and where the XCDs
+        // divide the batches a batch stays on one XCD this way too.
         int blk = blockIdx.x;
         const int xpb = p.B > 0 && 8 % p.B == 0 ? 8 / p.B : 0;
-        if (xpb > 0 && parts_per_batch % xpb == 0 && n_kv == p.B * parts_per_batch) {
+        if (parts_per_batch == (p.N + BKB - 1) / BKB) {
+            blk = blk % p.B * parts_per_batch + blk / p.B;
+        } else if (xpb > 0 && parts_per_batch % xpb == 0 && n_kv == p.B * parts_per_batch) {
             const int x = blk % 8, i = blk / 8;
             blk = (x / xpb) * parts_per_batch + i * xpb + x % xpb;
         }
@@ -2428,7 +2409,8 @@ hipError_t launch_bwd_parts(const FlashArgs& a, float* parts, int parts_per_batc
     dim3 gr((unsigned)(a.B * nkb * 16));
     hipLaunchKernelGGL((flash_bwd_kvq<DH, CAUSAL, PL>), gm, dim3(DH <= 64 ? 256 : 512), 0, st, a, parts, parts_per_batch,
                        n_kv);
-    hipLaunchKernelGGL((flash_bwd_kv_reduce<DH, CAUSAL, PL>), gr, dim3(256), 0, st, a, parts, parts_per_batch);
+    if (parts_per_batch > nkb)  // else every key block was written by its only part
+        hipLaunchKernelGGL((flash_bwd_kv_reduce<DH, CAUSAL, PL>), gr, dim3(256), 0, st, a, parts, parts_per_batch);
     return hipGetLastError();
 }
 template <int DH>
@@ -2495,16 +2477,11 @@ int flash_backward(FlashArgs a, int dh, bool mfma, bool causal, hipStream_t st) 
     const bool wide = mfma && flash_wide_head(dh) && flash_wide_fits(a.N, a.H, dh);
     // arena layout (256-byte aligned pieces)
     auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
-    const int nkb = (a.N + BKB - 1) / BKB;
-    int parts_per_batch = 0;
-    if (split) {
-        int64_t chunks = 0;
-        for (int kb = 0; kb < nkb; ++kb) chunks += bwd_kv_chunks(kb, a.N, a.H, causal);
-        a.part_log2 = bwd_part_log2(dh, chunks * a.B);
-        for (int kb = 0; kb < nkb; ++kb) parts_per_batch += bwd_kv_parts(kb, a.N, a.H, causal, a.part_log2);
-    }
+    BwdKvPlan kv{};
+    if (split) kv = bwd_kv_plan(dh, a.B, a.N, a.H, causal);
+    a.part_log2 = kv.part_log2;
     const size_t stats_b = (split || wide) ? 0 : al(2 * rows * sizeof(float));  // formed in-kernel
-    const size_t part_b = split ? al((size_t)a.B * parts_per_batch * 4 * (2 * 2 * (dh / 16)) * 64 * 16) : 0;
+    const size_t part_b = al(kv.bytes);
     const size_t fwd_b = ((split || wide) && !have_lse) ? al(rows * dh * 2) + al(rows * sizeof(float)) : 0;
     const size_t need = stats_b + part_b + fwd_b;
     if (need > g_bwd_ws_bytes) {
@@ -2533,9 +2510,9 @@ int flash_backward(FlashArgs a, int dh, bool mfma, bool causal, hipStream_t st) 
             a.o = o_ws;
             a.lse = l_ws;
         }
-        e = (dh == 32)   ? launch_bwd_split<32>(a, causal, parts, parts_per_batch, st)
-            : (dh == 64) ? launch_bwd_split<64>(a, causal, parts, parts_per_batch, st)
-                         : launch_bwd_split<128>(a, causal, parts, parts_per_batch, st);
+        e = (dh == 32)   ? launch_bwd_split<32>(a, causal, parts, kv.per_batch, st)
+            : (dh == 64) ? launch_bwd_split<64>(a, causal, parts, kv.per_batch, st)
+                         : launch_bwd_split<128>(a, causal, parts, kv.per_batch, st);
     } else if (wide) {
         if (!have_lse) {
             // recompute the forward's O and LSE into the arena

@@ -478,3 +478,39 @@ def test_wide_backward_head_counts(dev, orc, Dh, H, N, causal):
     got = bwd(evk, dev, q, k, v, g, causal, True)
     for x, want, what in zip(got, orc.attention_bwd(q, k, v, g, causal), ("dQ", "dK", "dV")):
         assert_close_f16(x, want, what=f"{what} Dh={Dh} H={H} N={N}")
+
+
+@pytest.mark.parametrize("Dh,B,N,H", [(128, 1, 5000, 91), (128, 515, 130, 9), (128, 1030, 40, 3), (64, 1, 3000, 120), (64, 1024, 128, 20),
+                                      (32, 1, 3000, 121), (32, 300, 500, 33)])
+@pytest.mark.parametrize("causal", [True, False])
+def test_backward_parts_of_long_sequences(dev, Dh, B, N, H, causal):
+    """Row parts longer than an ordinary call's, and key blocks of one part
+    each (no partials): against 64-bit gradients.  P, dS and the results round
+    to fp16 (2.8e-4 of their size each, rms) and a reference keeps none of it:
+    2e-3 is about four times the three together."""
+    import torch
+    import evk_amd as evk
+    gen = torch.Generator(device=dev).manual_seed(N + H)
+    new = lambda *s: torch.empty(*s, dtype=torch.float16, device=dev).normal_(generator=gen)  # noqa: E731
+    q, g, k, v = new(B, N, H * Dh), new(B, N, H * Dh), new(B, N, Dh), new(B, N, Dh)
+    o, dq, dk, dv = torch.empty_like(q), torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
+    lse = torch.empty(B, H, N, device=dev)
+    evk.flash_attention(q, k, v, o, causal=causal, lse=lse)
+    evk.flash_attention_bwd(q, k, v, o, g, dq, dk, dv, causal=causal, lse=lse)
+    torch.cuda.synchronize()
+    hidden = torch.ones(N, N, dtype=torch.bool, device=dev).triu(1)
+    for b in sorted({0, B // 2, B - 1}):
+        K, V = k[b].double(), v[b].double()
+        wk, wv, wq = torch.zeros_like(K), torch.zeros_like(V), []
+        for h in range(H):
+            Q, G = (t[b, :, h * Dh:(h + 1) * Dh].double() for t in (q, g))
+            s = Q @ K.t() / Dh ** 0.5
+            if causal:
+                s = s.masked_fill(hidden, -float("inf"))
+            P = torch.softmax(s, -1)
+            ds = P * (G @ V.t() - (G * (P @ V)).sum(-1, keepdim=True)) / Dh ** 0.5
+            wq.append(ds @ K)
+            wk += ds.t() @ Q
+            wv += P.t() @ G
+        for got, want, what in ((dq[b], torch.cat(wq, -1), "dq"), (dk[b], wk, "dk"), (dv[b], wv, "dv")):
+            assert (got.double() - want).norm() <= 2e-3 * want.norm(), (what, b)
