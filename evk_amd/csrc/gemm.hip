@@ -7,12 +7,16 @@
 // lengths, 2-byte aligned pointers, operands past the 2 GiB a buffer
 // descriptor spans) through registers.
 //
+// Element kernel (gemm_short): such rows with a short K, one thread for each
+// element of C.
+//
 // Skinny kernel (M <= 16, B row-major): bandwidth-bound, streams B once with
 // 16-byte coalesced loads, fp32 accumulation in registers, split-K across
 // workgroups with a deterministic last-arriving-workgroup reduction.
 #include "kernels.h"
 
 #include <algorithm>
+#include <cmath>
 #include <utility>
 
 namespace evkhip {
@@ -750,7 +754,39 @@ __global__ __launch_bounds__(256) void gemv_mf(GemmArgs p, float* __restrict__ p
     gemv_finish_m16(p, part, cnt, c0);
 }
 
+// ---- short K, any alignment: one thread per element of C.  Launch-bound up
+// to a few thousand elements; a chain of K loads of each operand otherwise ----
+__global__ __launch_bounds__(256) void gemm_short(GemmArgs p, int ta, int tb) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= (int64_t)p.M * p.N) return;
+    const int bz = blockIdx.y, row = (int)(i / p.N), col = (int)(i % p.N);
+    const f16* a = p.A + (int64_t)bz * p.sA + (ta ? (int64_t)row : (int64_t)row * p.K);
+    const f16* b = p.B + (int64_t)bz * p.sB + (tb ? (int64_t)col * p.K : (int64_t)col);
+    const int64_t step_a = ta ? p.M : 1, step_b = tb ? 1 : p.N;
+    float v = 0.0f;
+#pragma unroll 4
+    for (int k = 0; k < p.K; ++k) v += (float)a[k * step_a] * (float)b[k * step_b];
+    f16* c = p.C + (int64_t)bz * p.sC + i;
+    *c = (f16)(p.acc ? v + (float)*c : v);
+}
 
+// Whether gemm_short serves a product that the register-staged MFMA form would
+// otherwise take.  Both sides in us, fitted to 150 products with K from 1 to
+// 65 (hot operands): a thread's chain and the launched threads and products
+// against a workgroup's one or two K tiles (0.8 more where B is stored (N,K)),
+// and the tiles past the 512 or so that run at once.  5 x 5 x 5 3.3 -> 1.9 us,
+// 4096 of them 13.8 -> 3.8, 100000 x 3 x 7 8.7 -> 3.3, 300 x 301 x 9 3.9 -> 2.9;
+// the MFMA form from K = 17 on (300 x 301 both 3.9) and for 2000 x 2001
+// outputs from K = 1 on (10.1 -> 6.2).
+bool short_k_wins(const GemmArgs& a, int batch, bool tb) {
+    if (a.K > 80) return false;  // past the fit
+    const double mn = (double)a.M * a.N, k = a.K;
+    const double threads = std::ceil(mn / 256) * 256 * batch;
+    const double tiles = (double)((a.M + 63) / 64) * ((a.N + 63) / 64) * batch;
+    const double elements_us = 1.6 + 0.09 * k + 1.6e-6 * threads + 0.27e-6 * k * mn * batch;
+    const double tiles_us = 3.5 + (tb ? 0.8 : 0.0) + 2.7e-3 * std::max(0.0, tiles - 512) * (1 + k / 80);
+    return elements_us < tiles_us;
+}
 
 // The instances of gemm_mfma and what one costs, for choosing among them:
 // a CU that holds j tiles at once (j <= resident, what LDS allows) spends
@@ -980,7 +1016,11 @@ int gemm_dispatch(const GemmArgs& a, int batch, bool ta, bool tb, bool vec_ok, h
     // 131136 x 256 x 8192 1240 -> 1222 us, A stored (K,M) 1425 -> 1176 us.
     const bool direct = vec_ok && (int64_t)a.M * a.K * 2 < INT32_MAX && (int64_t)a.K * a.N * 2 < INT32_MAX &&
                         (int64_t)a.M * a.N < INT32_MAX;
-    if (direct) {
+    if (!vec_ok && a.epi == GEMM_STORE && short_k_wins(a, batch, tb)) {
+        const dim3 grid((unsigned)(((int64_t)a.M * a.N + 255) / 256), batch);
+        hipLaunchKernelGGL(gemm_short, grid, dim3(256), 0, st, a, (int)ta, (int)tb);
+        e = hipGetLastError();
+    } else if (direct) {
         e = launch_plan(choose_plan(a, batch, ta ? kColPlans : kRowPlans), a, batch, ta, tb, st);
     } else {
         e = launch_plan_rag(choose_plan(a, batch, kRagPlans), a, batch, ta, tb, st);

@@ -297,3 +297,24 @@ def test_each_instance(dev, orc, ta, tb, M, N, K):
     A = f32(a[:, rows].T if ta else a[rows])
     want = (A @ f32(b.T if tb else b) + f32(c0[rows])).astype(np.float16).view(np.uint16)
     assert_close_f16(got[rows], want, what=f"{ta}{tb} {M}x{N}x{K}")
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)])
+@pytest.mark.parametrize("B,M,N,K", [(1, 1, 1, 1), (4100, 5, 5, 5), (3, 37, 33, 13), (2, 300, 301, 17), (1, 3000, 3, 23), (1, 257, 255, 80),
+                                     (300, 3, 7, 81), (1, 1001, 1003, 2)])
+def test_short_k(dev, orc, ta, tb, B, M, N, K):
+    """Odd rows with a short K, accumulating, on both sides of the line between
+    a thread per element and MFMA tiles; sentinels around C."""
+    import torch
+    import evk_amd as evk
+    a = orc.uniform_f16((B, K, M) if ta else (B, M, K), 121 + M)
+    b = orc.uniform_f16((B, N, K) if tb else (B, K, N), 122 + N)
+    c0 = orc.uniform_f16((B, M, N), 123)
+    buf = torch.full((c0.size + 16,), 7.0, dtype=torch.float16, device=dev)
+    C = buf[5:5 + c0.size].view(c0.shape)
+    C.copy_(to_dev(c0, dev))
+    evk.matmul(to_dev(a, dev), to_dev(b, dev), C, ta, tb, True)
+    torch.cuda.synchronize()
+    want = orc.matmul(a, b, c=c0, transpose_a=ta, transpose_b=tb, acc_c=True)
+    assert_close_f16(from_dev(C), want, what=f"{ta}{tb} {B}x{M}x{N}x{K}")
+    assert bool((buf[:5] == 7).all()) and bool((buf[5 + c0.size:] == 7).all())
