@@ -357,9 +357,10 @@ DEV void each8(int64_t n, F&& f) {
 DEV half8 ld_n(const f16* p, int n) {
     if (n == 8) return ld_h8(p);
     half8 v = {};
+    if (n > 0) {  // the last value again past the end: no branch, hence no wait, between the loads
 #pragma unroll
-    for (int e = 0; e < 7; ++e)
-        if (e < n) v[e] = p[e];
+        for (int e = 0; e < 8; ++e) v[e] = p[min(e, n - 1)];
+    }
     return v;
 }
 DEV void st_n(f16* p, const half8& v, int n) {
@@ -388,15 +389,23 @@ __global__ __launch_bounds__(256) void add_k(const f16* a, const f16* b, f16* c,
     });
 }
 
-// One thread per 8 values of a row (dim / 8 rounded up pieces a row).
+// One thread per W values of a row (W = 8 or 1; dim / W rounded up pieces a row).
+template <int W>
 __global__ __launch_bounds__(256) void embed_k(const f16* table, const uint16_t* idx, f16* out, int64_t n_idx,
                                                 int dim, int pieces, int vocab) {
     const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (gid >= n_idx * pieces) return;
     const int64_t i = gid / pieces;
-    const int d = (int)(gid % pieces) * 8, k = min(8, dim - d);
+    const int d = (int)(gid % pieces) * W;
     const int tok = min((int)idx[i], vocab - 1);
-    st_n(out + i * dim + d, ld_n(table + (int64_t)tok * dim + d, k), k);
+    const f16* src = table + (int64_t)tok * dim + d;
+    f16* dst = out + i * dim + d;
+    if constexpr (W == 1) {
+        *dst = *src;
+    } else {
+        const int k = min(8, dim - d);
+        st_n(dst, ld_n(src, k), k);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -593,9 +602,15 @@ int add_launch(const f16* a, const f16* b, f16* c, int64_t n, hipStream_t st) {
 int embed_launch(const f16* table, const uint16_t* idx, f16* out, int64_t n_idx, int dim, int vocab,
                  hipStream_t st) {
     if (n_idx == 0 || dim == 0) return EVKHIP_OK;
-    const int pieces = (dim + 7) / 8;
-    hipLaunchKernelGGL(embed_k, dim3((unsigned)((n_idx * pieces + 255) / 256)), dim3(256), 0, st, table, idx, out,
-                       n_idx, dim, pieces, vocab);
+    // 8 values a thread unless a row's last, partial piece would cost more
+    // than the others save: short rows of a length off 8, or few of them.  us,
+    // one value and 8 a thread: 20000 x 7 1.9 and 3.0, 100000 x 31 5.6 and 6.7,
+    // 100 x 255 1.8 and 2.6; 20000 x 65 3.2 and 2.7, 1000 x 1001 2.8 and 2.4.
+    const bool by_value = dim % 8 && (dim < 32 || n_idx * dim < (1 << 19));
+    const int pieces = by_value ? dim : (dim + 7) / 8;
+    const dim3 grid((unsigned)((n_idx * pieces + 255) / 256));
+    if (by_value) hipLaunchKernelGGL(embed_k<1>, grid, dim3(256), 0, st, table, idx, out, n_idx, dim, pieces, vocab);
+    else hipLaunchKernelGGL(embed_k<8>, grid, dim3(256), 0, st, table, idx, out, n_idx, dim, pieces, vocab);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? EVKHIP_OK : check_hip(e, "embed launch");
 }

@@ -491,6 +491,22 @@ def test_embed_row_lengths(dev, orc, dim):
     assert np.array_equal(from_dev(O), table[np.minimum(idx, 49)])
 
 
+@pytest.mark.parametrize("n,dim", [(1, 255), (520, 1001), (15888, 33), (16913, 31), (523, 1002), (524, 1001)])
+def test_embed_value_or_piece(dev, orc, n, dim):
+    """Rows off 8 values, one value a thread (short or few) and in pieces of 8
+    with a partial last one: both sides of the line; sentinels behind."""
+    import torch
+    import evk_amd as evk
+    table = orc.normal_f16((40, dim), 361)
+    idx = (np.arange(n) * 7 % 45).astype(np.uint16)  # ids past the table: its last row
+    buf = torch.full((n * dim + 8,), 7.0, dtype=torch.float16, device=dev)
+    O = buf[:n * dim].view(n, dim)
+    evk.embed(to_dev(table, dev), torch.from_numpy(idx.view(np.int16)).to(dev), O)
+    torch.cuda.synchronize()
+    assert np.array_equal(from_dev(O), table[np.minimum(idx, 39)])
+    assert bool((buf[n * dim:] == 7).all())
+
+
 @pytest.mark.parametrize("V,base,count", [(40000, 0, 40000), (40001, 3, 39990), (33000, 1, 32769), (100, 7, 9), (8, 0, 0)])
 def test_greedy_long_rows(dev, orc, V, base, count):
     """Rows longer than one pass of the workgroup, ranges off a 16-byte
