@@ -415,31 +415,31 @@ __global__ __launch_bounds__(256) void embed_k(const f16* table, const uint16_t*
 // token_base.  Any reduction tree over this order gives the same winner.
 // ---------------------------------------------------------------------------
 
-// One workgroup per sequence; a thread requests GR_LD 16-byte pieces of the
-// row before it looks at any (the row may start at any fp16 address): 32000
-// logits 39.7 -> 6.1 us against 2-byte loads by 256 threads.
-constexpr int GR_NT = 1024, GR_LD = 4;
-
-__global__ __launch_bounds__(GR_NT) void greedy_k(const f16* logits, uint16_t* out, int S, int V, int position,
-                                                   int token_base, int token_count) {
-    __shared__ float s_v[GR_NT / 64];
-    __shared__ uint32_t s_r[GR_NT / 64];
+// One workgroup of NT threads per sequence; a thread requests LD pieces of W
+// values (8 or 1) before it looks at any; the row may start at any fp16
+// address.  greedy_launch chooses.
+template <int NT, int W, int LD>
+__global__ __launch_bounds__(NT) void greedy_k(const f16* logits, uint16_t* out, int S, int V, int position,
+                                                int token_base, int token_count) {
+    __shared__ float s_v[NT / 64];
+    __shared__ uint32_t s_r[NT / 64];
     const int b = blockIdx.x, tid = threadIdx.x;
     const f16* row = logits + ((int64_t)b * S + position) * V + token_base;
     float bv = -3.402823466e+38f;
     uint32_t br = 0u;  // rank of j = 0 (token_base)
-    for (int j0 = tid * 8; j0 < token_count; j0 += GR_NT * 8 * GR_LD) {
-        half8 v[GR_LD];
+    for (int j0 = tid * W; j0 < token_count; j0 += NT * W * LD) {
+        half8 v[LD];
 #pragma unroll
-        for (int u = 0; u < GR_LD; ++u) {
-            const int j = j0 + u * GR_NT * 8;
-            v[u] = ld_n(row + j, max(0, min(8, token_count - j)));
+        for (int u = 0; u < LD; ++u) {
+            const int j = j0 + u * NT * W;
+            if constexpr (W == 8) v[u] = ld_n(row + j, max(0, min(8, token_count - j)));
+            else v[u][0] = row[min(j, token_count - 1)];
         }
 #pragma unroll
-        for (int u = 0; u < GR_LD; ++u)
+        for (int u = 0; u < LD; ++u)
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const int j = j0 + u * GR_NT * 8 + e;
+            for (int e = 0; e < W; ++e) {
+                const int j = j0 + u * NT * W + e;
                 const float x = (float)v[u][e];
                 const uint32_t r = greedy_rank((uint32_t)j);
                 if (j < token_count && x > -3.402823466e+38f && greedy_better(x, r, bv, br)) {
@@ -457,7 +457,7 @@ __global__ __launch_bounds__(GR_NT) void greedy_k(const f16* logits, uint16_t* o
     if ((tid & 63) == 0) { s_v[tid >> 6] = bv; s_r[tid >> 6] = br; }
     __syncthreads();
     if (tid == 0) {
-        for (int w = 1; w < GR_NT / 64; ++w)
+        for (int w = 1; w < NT / 64; ++w)
             if (greedy_better(s_v[w], s_r[w], bv, br)) { bv = s_v[w]; br = s_r[w]; }
         out[b] = (uint16_t)(token_base + greedy_index(br));
     }
@@ -618,7 +618,24 @@ int embed_launch(const f16* table, const uint16_t* idx, f16* out, int64_t n_idx,
 int greedy_launch(const f16* logits, uint16_t* out, int B, int S, int V, int position, int token_base,
                   int token_count, hipStream_t st) {
     if (B == 0) return EVKHIP_OK;
-    hipLaunchKernelGGL(greedy_k, dim3(B), dim3(GR_NT), 0, st, logits, out, S, V, position, token_base, token_count);
+    auto launch = [&](auto nt, auto w, auto ld) {
+        constexpr int NT = decltype(nt)::value, W = decltype(w)::value, LD = decltype(ld)::value;
+        hipLaunchKernelGGL((greedy_k<NT, W, LD>), dim3(B), dim3(NT), 0, st, logits, out, S, V, position, token_base,
+                           token_count);
+    };
+    using std::integral_constant;
+    // The latency of one row's loads and of the comparisons behind them, or
+    // many rows' workgroups.  us for rows of 32, 2000, 8192 and 32000 values,
+    // one row: 256 x 1 2.2, 3.4, 7.4, 22.9; 256 x 8 2.7, 2.8, 4.7, 12.7; 512 x
+    // 2 x 8 3.2, 3.2, 3.7, 7.6; 1024 x 2 x 8 3.5, 3.6, 4.2, 6.4.  2048 rows:
+    // 3.4, 5.1, 11.2, 52; 3.9, 4.9, 9.8, 30; 6.3, 7.0, 10.2, 28; 12, 12, 17, 31.
+    constexpr integral_constant<int, 1> one{};
+    constexpr integral_constant<int, 2> two{};
+    constexpr integral_constant<int, 8> eight{};
+    if (token_count <= 512) launch(integral_constant<int, 256>{}, one, one);
+    else if (token_count <= 4096) launch(integral_constant<int, 256>{}, eight, one);
+    else if (token_count <= 8192 || B > device_cu_count()) launch(integral_constant<int, 512>{}, eight, two);
+    else launch(integral_constant<int, 1024>{}, eight, two);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? EVKHIP_OK : check_hip(e, "greedy_sample launch");
 }

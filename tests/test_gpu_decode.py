@@ -530,6 +530,18 @@ def test_greedy_long_rows(dev, orc, V, base, count):
     assert list(got) == want
 
 
+@pytest.mark.parametrize("B", [2, 300])
+@pytest.mark.parametrize("count", [1, 511, 512, 513, 4096, 4097, 8192, 8193, 20001])
+def test_greedy_workgroup_sizes(dev, orc, B, count):
+    """Both sides of each line between the workgroup forms (and of one row per
+    CU), from a start off a 16-byte boundary, the winner often among ties."""
+    import evk_amd as evk
+    pool = f16([-1.0, 0.0, -0.0, 0.5, 2.0, -np.inf, np.nan, 1.0])
+    logits = pool[np.random.RandomState(count).randint(0, 8, size=(B, 1, count + 3))]
+    logits[1, 0, 3:] = 0xFC00  # no candidate
+    assert np.array_equal(greedy_dev(evk, dev, logits, 0, 3, count), orc.greedy_sample(logits, 0, 3, count))
+
+
 @pytest.mark.parametrize("heads,dh", [(3, 48), (5, 32), (3, 64), (1, 128), (1, 256)])
 @pytest.mark.parametrize("n", [16, 17, 65])
 def test_prefill_cache_rows(dev, orc, heads, dh, n):
