@@ -567,7 +567,9 @@ int kv_cache_write_launch(const f16* src, f16* cache, int batch, int n, int D, i
 int rms_norm_launch(const f16* in, f16* out, int64_t rows, int D, float eps, hipStream_t st) {
     if (rows == 0) return EVKHIP_OK;
     const dim3 grid((unsigned)((rows + 3) / 4));
-    if (D % 8 || D > 4096) hipLaunchKernelGGL(rms_norm_k, grid, dim3(256), 0, st, in, out, rows, D, eps);
+    // up to 64 values a lane has one of them either way, without pieces of 8
+    // that most lanes do not hold (100000 x 16: 16.0 us, in registers 17.8)
+    if (D <= 64 || D % 8 || D > 4096) hipLaunchKernelGGL(rms_norm_k, grid, dim3(256), 0, st, in, out, rows, D, eps);
     else if (D <= 512) hipLaunchKernelGGL(rms_norm_reg_k<1>, grid, dim3(256), 0, st, in, out, rows, D, eps);
     else if (D <= 1024) hipLaunchKernelGGL(rms_norm_reg_k<2>, grid, dim3(256), 0, st, in, out, rows, D, eps);
     else if (D <= 2048) hipLaunchKernelGGL(rms_norm_reg_k<4>, grid, dim3(256), 0, st, in, out, rows, D, eps);

@@ -482,28 +482,33 @@ __global__ __launch_bounds__(EW_NT) void rms_norm_bwd_k(const f16* in, const f16
     }
 }
 
-// rms_norm_bwd_k with the row in registers: D % 8 == 0, D <= 512 * NV, rows at
-// any alignment; each value is read and written once (2560 x 768: 19.6 -> 6.3 us)
-template <int NV>
+// rms_norm_bwd_k with the row in registers: pieces of W values (8 or 2), D a
+// multiple of W and at most 64 W NV, rows at any alignment; each value is read
+// and written once (2560 x 768: 19.6 -> 6.3 us)
+template <int W>
+DEV void ld_w(const f16* p, f16 (&v)[W]) {
+    __builtin_memcpy(v, p, 2 * W);
+}
+template <int NV, int W>
 __global__ __launch_bounds__(EW_NT) void rms_norm_bwd_reg_k(const f16* in, const f16* gout, f16* gin, float eps, int D,
                                                             int64_t rows) {
     const int64_t row = (int64_t)blockIdx.x * ROWS_PER_WG + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     if (row >= rows) return;
-    half8 x[NV] = {}, g[NV] = {}, o[NV] = {};
+    f16 x[NV][W] = {}, g[NV][W] = {}, o[NV][W] = {};
 #pragma unroll
     for (int u = 0; u < NV; ++u) {
-        const int c = (lane + 64 * u) * 8;
+        const int c = (lane + 64 * u) * W;
         if (c >= D) continue;
-        x[u] = ld_h8(in + row * D + c);
-        g[u] = ld_h8(gout + row * D + c);
-        o[u] = ld_h8(gin + row * D + c);
+        ld_w(in + row * D + c, x[u]);
+        ld_w(gout + row * D + c, g[u]);
+        ld_w(gin + row * D + c, o[u]);
     }
     float ss = 0.0f;
 #pragma unroll
     for (int u = 0; u < NV; ++u)
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
+        for (int e = 0; e < W; ++e) {
             x[u][e] = (f16)fminf(fmaxf(hf(x[u][e]), -65504.0f), 65504.0f);
             ss += hf(x[u][e]) * hf(x[u][e]);
         }
@@ -513,16 +518,16 @@ __global__ __launch_bounds__(EW_NT) void rms_norm_bwd_reg_k(const f16* in, const
 #pragma unroll
     for (int u = 0; u < NV; ++u)
 #pragma unroll
-        for (int e = 0; e < 8; ++e) dot += hf(g[u][e]) * (hf(x[u][e]) * inv);
+        for (int e = 0; e < W; ++e) dot += hf(g[u][e]) * (hf(x[u][e]) * inv);
     dot = wave_sum(dot);
     const float sc = dot / (float)D;
 #pragma unroll
     for (int u = 0; u < NV; ++u) {
-        const int c = (lane + 64 * u) * 8;
+        const int c = (lane + 64 * u) * W;
         if (c >= D) continue;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) o[u][e] = (f16)(hf(o[u][e]) + (hf(g[u][e]) * inv - hf(x[u][e]) * inv * inv * sc));
-        st_h8(gin + row * D + c, o[u]);
+        for (int e = 0; e < W; ++e) o[u][e] = (f16)(hf(o[u][e]) + (hf(g[u][e]) * inv - hf(x[u][e]) * inv * inv * sc));
+        __builtin_memcpy(gin + row * D + c, o[u], 2 * W);
     }
 }
 
@@ -792,10 +797,14 @@ int softmax_bwd_launch(const f16* probs, const f16* gout, f16* gin, float scale,
 int rms_norm_bwd_launch(const f16* in, const f16* gout, f16* gin, float eps, int D, int64_t rows, hipStream_t st) {
     if (rows == 0 || D == 0) return EVKHIP_OK;
     const dim3 grid(row_grid(rows)), nt(EW_NT);
-    if (D % 8 || D > 2048) hipLaunchKernelGGL(rms_norm_bwd_k, grid, nt, 0, st, in, gout, gin, eps, D, rows);
-    else if (D <= 512) hipLaunchKernelGGL(rms_norm_bwd_reg_k<1>, grid, nt, 0, st, in, gout, gin, eps, D, rows);
-    else if (D <= 1024) hipLaunchKernelGGL(rms_norm_bwd_reg_k<2>, grid, nt, 0, st, in, gout, gin, eps, D, rows);
-    else hipLaunchKernelGGL(rms_norm_bwd_reg_k<4>, grid, nt, 0, st, in, gout, gin, eps, D, rows);
+    // Up to 64 values a lane has one of them either way, and the walking kernel
+    // none of the idle lanes' work of pieces of 8; up to 128 pieces of 2 (us,
+    // walking, 2 and 8: 20000 x 64 6.1, -, 8.0; 20000 x 128 7.7, 5.8, 8.3).
+    if (D <= 64 || D % 8 || D > 2048) hipLaunchKernelGGL(rms_norm_bwd_k, grid, nt, 0, st, in, gout, gin, eps, D, rows);
+    else if (D <= 128) hipLaunchKernelGGL((rms_norm_bwd_reg_k<1, 2>), grid, nt, 0, st, in, gout, gin, eps, D, rows);
+    else if (D <= 512) hipLaunchKernelGGL((rms_norm_bwd_reg_k<1, 8>), grid, nt, 0, st, in, gout, gin, eps, D, rows);
+    else if (D <= 1024) hipLaunchKernelGGL((rms_norm_bwd_reg_k<2, 8>), grid, nt, 0, st, in, gout, gin, eps, D, rows);
+    else hipLaunchKernelGGL((rms_norm_bwd_reg_k<4, 8>), grid, nt, 0, st, in, gout, gin, eps, D, rows);
     return launched("rms_norm_backward launch");
 }
 int mse_loss_launch(const f16* pred, const f16* tgt, f16* grad, f16* result, int64_t n, hipStream_t st) {

@@ -455,6 +455,13 @@ def test_rms_norm_row_lengths(dev, orc, D, off):
     assert ulp_close(from_dev(Y), orc.rms_norm(x, 1e-4))
 
 
+@pytest.mark.parametrize("off", [0, 1])
+@pytest.mark.parametrize("D", [56, 64, 72])
+def test_rms_norm_narrow_rows(dev, orc, D, off):
+    """Both sides of the line between the walking and the register kernels."""
+    test_rms_norm_row_lengths(dev, orc, D, off)
+
+
 @pytest.mark.parametrize("off", [0, 5])
 @pytest.mark.parametrize("n", [1, 7, 8, 9, 2047, 2049])
 def test_elementwise_tails(dev, orc, n, off):

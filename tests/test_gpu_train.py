@@ -258,3 +258,10 @@ def test_rms_norm_backward_row_lengths(dev, orc, D, off):
     evk.rms_norm_backward(X, G, A, 1e-4)
     sync()
     assert_close_f16(from_dev(A), orc.rms_norm_backward(x, g, a, 1e-4), what=f"rms_norm_backward D={D}")
+
+
+@pytest.mark.parametrize("off", [0, 1])
+@pytest.mark.parametrize("D", [56, 64, 72, 120, 128, 136])
+def test_rms_norm_backward_narrow_rows(dev, orc, D, off):
+    """Both sides of the lines between the walking kernel, pieces of 2 and of 8."""
+    test_rms_norm_backward_row_lengths(dev, orc, D, off)
