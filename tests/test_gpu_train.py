@@ -265,3 +265,9 @@ def test_rms_norm_backward_row_lengths(dev, orc, D, off):
 def test_rms_norm_backward_narrow_rows(dev, orc, D, off):
     """Both sides of the lines between the walking kernel, pieces of 2 and of 8."""
     test_rms_norm_backward_row_lengths(dev, orc, D, off)
+
+
+@pytest.mark.parametrize("n,dim,vocab,distinct", [(2, 5, 9, 1), (7, 257, 40, 9), (10, 768, 60, 3), (11, 768, 60, 3)])
+def test_embed_backward_few_ids(dev, orc, n, dim, vocab, distinct):
+    """Both sides of the line to the walking kernel, repeated and invalid ids."""
+    test_embed_backward_order(dev, orc, n, dim, vocab, distinct)
