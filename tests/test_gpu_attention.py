@@ -514,3 +514,73 @@ def test_backward_parts_of_long_sequences(dev, Dh, B, N, H, causal):
             wv += P.t() @ G
         for got, want, what in ((dq[b], torch.cat(wq, -1), "dq"), (dk[b], wk, "dk"), (dv[b], wv, "dv")):
             assert (got.double() - want).norm() <= 2e-3 * want.norm(), (what, b)
+
+
+def gradients_f64(Q, K, V, G, pos, causal):
+    """dQ rows and the rows' shares of dK and dV: flattened rows Q, G at positions pos."""
+    import torch
+    Q, K, V, G = (t.double() for t in (Q, K, V, G))
+    s = Q @ K.t() / Q.shape[1] ** 0.5
+    if causal:
+        s = s.masked_fill(torch.arange(K.shape[0], device=Q.device)[None] > pos[:, None], -float("inf"))
+    P = torch.softmax(s, -1)
+    dp = G @ V.t()
+    ds = P * (dp - (P * dp).sum(-1, keepdim=True)) / Q.shape[1] ** 0.5
+    return ds @ K, ds.t() @ Q, P.t() @ G
+
+
+@pytest.mark.parametrize("exponent", [-12, -15, -17])
+@pytest.mark.parametrize("Dh", [32, 64, 128])
+def test_backward_small_gradients(dev, Dh, exponent):
+    """dO small and subnormal (all of it at 2^-17) against large V, so that the
+    row sums of dO.O and dO.V matter and dQ, dK are normal numbers: no product
+    of a subnormal may be lost.  dV, subnormal itself, to its fp16 spacing."""
+    import torch
+    import evk_amd as evk
+    N, H = 256, 16
+    gen = torch.Generator(device=dev).manual_seed(Dh)
+    new = lambda scale, *s: (torch.empty(*s, device=dev).normal_(generator=gen) * scale).half()  # noqa: E731
+    q, k, v, g = new(1, 1, N, H * Dh), new(1, 1, N, Dh), new(256, 1, N, Dh), new(2.0 ** exponent, 1, N, H * Dh)
+    o, dq, dk, dv = torch.empty_like(q), torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
+    lse = torch.empty(1, H, N, device=dev)
+    evk.flash_attention(q, k, v, o, causal=True, lse=lse)
+    evk.flash_attention_bwd(q, k, v, o, g, dq, dk, dv, causal=True, lse=lse)
+    torch.cuda.synchronize()
+    pos = torch.arange(N * H, device=dev) // H
+    wq, wk, wv = gradients_f64(q.view(-1, Dh), k[0], v[0], g.view(-1, Dh), pos, True)
+    for got, want, what in ((dq.view(-1, Dh), wq, "dq"), (dk[0], wk, "dk")):
+        assert (got.double() - want).norm() <= 2e-3 * want.norm(), what
+    assert (dv[0].double() - wv).abs().max() <= 2.0 ** -24 + 2e-3 * wv.abs().max()
+
+
+@pytest.mark.parametrize("Dh,causal,use_lse", [(32, True, True), (32, False, False), (64, True, False), (64, False, True), (128, True, True),
+                                               (128, False, False)])
+def test_backward_batch_of_q_over_2gib(dev, Dh, causal, use_lse):
+    """One batch of Q of 2 GiB: past the 32-bit buffer descriptors of the row
+    parts, on the kernels of 32 keys a workgroup.  Every gradient against 64
+    bits; tolerance as in test_backward_parts_of_long_sequences."""
+    import torch
+    import evk_amd as evk
+    N = 64
+    H = 2 ** 30 // (N * Dh) + 1
+    assert N * H * Dh * 2 > 2 ** 31
+    gen = torch.Generator(device=dev).manual_seed(Dh)
+    new = lambda *s: torch.empty(*s, dtype=torch.float16, device=dev).normal_(generator=gen)  # noqa: E731
+    q, g, k, v = new(1, N, H * Dh), new(1, N, H * Dh), new(1, N, Dh), new(1, N, Dh)
+    o, dq, dk, dv = torch.empty_like(q), torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
+    lse = torch.empty(1, H, N, device=dev)
+    evk.flash_attention(q, k, v, o, causal=causal, lse=lse)
+    evk.flash_attention_bwd(q, k, v, o, g, dq, dk, dv, causal=causal, lse=lse if use_lse else None)
+    torch.cuda.synchronize()
+    rows, wk, wv = N * H, 0.0, 0.0
+    for r0 in range(0, rows, 1 << 20):
+        r1 = min(rows, r0 + (1 << 20))
+        pos = torch.arange(r0, r1, device=dev) // H
+        wq, sk, sv = gradients_f64(q.view(-1, Dh)[r0:r1], k[0], v[0], g.view(-1, Dh)[r0:r1], pos, causal)
+        err, size = (dq.view(-1, Dh)[r0:r1].double() - wq).norm(), wq.norm()
+        assert err <= 2e-3 * size, ("dq", r0)
+        wk, wv = wk + sk, wv + sv
+    for got, want, what in ((dk[0], wk, "dk"), (dv[0], wv, "dv")):
+        assert (got.double() - want).norm() <= 2e-3 * want.norm(), what
+    del q, g, o, dq
+    torch.cuda.empty_cache()

@@ -570,3 +570,24 @@ def test_prefill_cache_rows(dev, orc, heads, dh, n):
     assert_close_f16(got, want_cache.reshape(got.shape), what="cache")
     assert not got[:, :, n:].any()
     assert_close_f16(from_dev(logits), want_logits[0], what="logits")
+
+
+@pytest.mark.parametrize("heads,dh,n", [(44, 64, 260), (80, 32, 150)])
+def test_prefill_64_row_tiles(dev, orc, heads, dh, n):
+    """Prompts whose attention takes pairs of 64-row tiles and stores its rows
+    strided (more than 128 pairs): an odd number of tiles, a partial last one.
+    The second layer's cache rows depend on every row of the first's attention."""
+    import evk_amd as evk
+    import torch
+    assert ((n + 63) // 64 + 1) // 2 * heads > 128
+    kw = dict(vocab=136, d=heads * dh, heads=heads, layers=2, hidden=72, max_seq=n)
+    ocfg, cfg = orc.model_cfg(**kw), evk.model_cfg(**kw)
+    w = orc.model_weights(ocfg, seed=411 + dh, std=0.03)
+    prompt = orc.tokens_u16(n, 412 + n, 136)
+    cache = torch.zeros(evk.model_cache_elems(cfg), dtype=torch.float16, device=dev)
+    tok, logits = torch.zeros(1, dtype=torch.int16, device=dev), torch.empty(136, dtype=torch.float16, device=dev)
+    evk.model_prefill(cfg, to_dev(w, dev), cache, torch.from_numpy(prompt.view(np.int16)).to(dev), 0, tok, logits)
+    torch.cuda.synchronize()
+    _, want_cache, want_logits = orc.model_generate(ocfg, w, prompt, 0, return_logits=True)
+    assert_close_f16(from_dev(cache), want_cache.reshape(-1), what="cache")
+    assert_close_f16(from_dev(logits), want_logits[0], what="logits")

@@ -75,10 +75,9 @@ def test_large_tile_paths(dev, orc, M, N, K):
 
 @pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)])
 def test_k_groups_ragged(dev, orc, ta, tb):
-    """Grids that fit the CUs once with a long K (64x64 tiles, K >= 1024) run
-    four K groups per workgroup whose sums meet in LDS: ragged M, N and a K
-    that is not a multiple of the 64-deep tile (the last group's range is
-    shorter), every operand order."""
+    """Grids that fit the CUs once with a long K run two K groups per workgroup
+    whose sums meet in LDS: ragged M, N and a K that is not a multiple of the
+    64-deep tile (the last group's range is shorter), every operand order."""
     import evk_amd as evk
     M, N, K = 200, 136, 1096
     a = orc.uniform_f16((K, M) if ta else (M, K), 61 + ta)
@@ -205,9 +204,9 @@ def test_config5_qkv_shape(dev, orc):
 
 
 @pytest.mark.parametrize("ta", [False, True])
-def test_operand_over_2gib_takes_tiled_path(dev, orc, ta):
-    """A 2.15 GB A operand (past the 32-bit buffer-descriptor range of the
-    MFMA kernel) runs the 64-bit-addressed tiled kernel; sampled rows of C and
+def test_operand_over_2gib(dev, orc, ta):
+    """A 2.15 GB A operand (past the 32-bit buffer descriptors of the LDS-direct
+    loads) runs on 64-bit addresses through registers; sampled rows of C and
     whole-matrix column sums are checked against fp32 on the host.  Inputs
     are drawn on the device from a seeded torch generator (2 GB is too much
     to push from the host in a test)."""
@@ -241,7 +240,7 @@ def test_operand_over_2gib_takes_tiled_path(dev, orc, ta):
 def test_any_row_length(dev, orc, ta, tb, M, N, K):
     """Row lengths that are no multiple of a 16-byte chunk, in every operand
     order: tile edges, a K tail of one element, grids of one and of many
-    tiles, the four-group K split (K >= 1024)."""
+    tiles, the two-group K split (K >= 1024)."""
     import evk_amd as evk
     a = orc.uniform_f16((K, M) if ta else (M, K), 91 + M)
     b = orc.uniform_f16((N, K) if tb else (K, N), 92 + N)
@@ -318,3 +317,41 @@ def test_short_k(dev, orc, ta, tb, B, M, N, K):
     want = orc.matmul(a, b, c=c0, transpose_a=ta, transpose_b=tb, acc_c=True)
     assert_close_f16(from_dev(C), want, what=f"{ta}{tb} {B}x{M}x{N}x{K}")
     assert bool((buf[:5] == 7).all()) and bool((buf[5 + c0.size:] == 7).all())
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)])
+def test_large_odd_rows(dev, orc, ta, tb):
+    """Odd rows on 128 x 128 tiles through registers (the grids of the other
+    such tests are small enough for 64 x 64), accumulating."""
+    import evk_amd as evk
+    M, N, K = 3001, 2003, 70
+    a = orc.uniform_f16((K, M) if ta else (M, K), 131)
+    b = orc.uniform_f16((N, K) if tb else (K, N), 132)
+    c0 = orc.uniform_f16((M, N), 133)
+    got = run_mm(evk, dev, a, b, None, ta, tb, True, c0)
+    want = (f32(a.T if ta else a) @ f32(b.T if tb else b) + f32(c0)).astype(np.float16).view(np.uint16)
+    assert_close_f16(got, want, what=f"{ta}{tb}")
+
+
+def test_output_past_2_31_elements(dev):
+    """More than 2^31 elements of C from small operands: rows at both ends and
+    around the 2^31st element, and the sum of every row."""
+    import torch
+    import evk_amd as evk
+    M, N, K = 70000, 32000, 64
+    assert M * N > 2**31
+    g = torch.Generator(device=dev).manual_seed(8)
+    A = torch.rand((M, K), generator=g, device=dev, dtype=torch.float16) - 0.5
+    B = torch.rand((K, N), generator=g, device=dev, dtype=torch.float16) - 0.5
+    C = torch.full((M, N), 7.0, dtype=torch.float16, device=dev)
+    evk.matmul(A, B, C)
+    torch.cuda.synchronize()
+    rows = torch.tensor([0, 1, 2**31 // N - 1, 2**31 // N, 2**31 // N + 1, M - 2, M - 1], device=dev)
+    want = A[rows].double() @ B.double()
+    assert (C[rows].double() - want).abs().max() <= 2e-3
+    # fp16 rounding of up to 2^-11 |c| an element, sqrt(N) of them: far below 0.2
+    for r0 in range(0, M, 10000):
+        got = C[r0:r0 + 10000].float().sum(1).double()
+        assert (got - A[r0:r0 + 10000].double() @ B.double().sum(1)).abs().max() <= 0.2
+    del A, B, C
+    torch.cuda.empty_cache()
