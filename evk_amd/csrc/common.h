@@ -206,8 +206,9 @@ DEV float gelu_f(float x) {
 }
 
 // tanh on the hardware exponential and reciprocal: 1 - 2 / (e^(2|u|) + 1) with
-// u's sign, about 1e-7 absolute everywhere (what 1 + tanh u needs: it takes
-// the same rounding as with tanhf next to -1).  For whole tensors, where
+// u's sign, 1.4e-7 absolute (tanhf 6e-8).  The fp16 results are as good: over
+// every finite input gelu is off the nearest value at 269 of them (272 with
+// tanhf), its gradient at 433 (433).  For whole tensors, where
 // tanhf's branches and polynomial take longer than the memory accesses; the
 // decode kernels keep gelu_f.
 DEV float tanh_fast(float u) {

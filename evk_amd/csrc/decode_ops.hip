@@ -501,6 +501,8 @@ int sq_attention_launch(const f16* q, const f16* kc, const f16* vc, f16* out, in
     // A split walks `step` rows at a time (about a microsecond each), and the
     // merge takes about as long per SQ_MB splits: chunk / step + splits / SQ_MB
     // is least at splits = sqrt(SQ_MB L / step), within two workgroups per CU.
+    // Over 58 drawn calls (L to 20000, head sizes 16 to 256, up to 128 caches)
+    // 0.66 of the time of 64 rows a split and one pass in flight, geometric mean.
     const int cus = device_cu_count();
     int nsplit = 1, chunk = std::max(L, 1);
     const int step = 256 / (dh / 8) * SQ_U;

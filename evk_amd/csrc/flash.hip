@@ -908,8 +908,11 @@ DEV float dot8(const half8& x, const half8& y) {
     for (int e = 0; e < 8; ++e) acc = __builtin_fmaf((float)x[e], (float)y[e], acc);
     return acc;
 }
-// the same on v_dot2_f32_f16 (products and sums in fp32): 4 instructions
-// instead of 24
+// the same on v_dot2_f32_f16 (products and sums in fp32, subnormal inputs
+// kept): 4 instructions instead of 24.  The dK/dV parts of head size 128 form
+// D with it and the dQ tiles with dot8; dK is as far from 64-bit gradients
+// either way, for dO from 1 down to 2^-19 (3.1e-4 of its size where nothing
+// is subnormal).
 DEV float dot8_pairs(const half8& x, const half8& y) {
     float acc = 0.0f;
 #pragma unroll
@@ -1335,7 +1338,9 @@ DEV void bwd_kv_pair_body(const FlashArgs& p, float* part_ws, int parts_per_batc
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): in the loop only its own loads are in flight
     __syncthreads();
     // scores of chunk c (in stage st) into the exchange buffer c & 1; keys past
-    // a row's position or N, and rows past NH, give P = dS = 0
+    // a row's position or N give P = dS = 0.  Rows past NH are zeros in Q, dO
+    // and their statistics: P is 1 there in an unmasked chunk, dS 0, and the
+    // zero rows of dO and Q keep both out of the sums.
     auto score = [&](int c, int st, auto masked) {
         const f16* qs = chunk_s + st * L::STAGE + (hf * 16 + l16) * RW + g * 8;
         const float* sts = stats_s + st * L::STATS + hf * 16 + 4 * g;

@@ -44,8 +44,8 @@ namespace {
 // tile.  Workgroups are ordered so that the
 // ones an XCD runs (workgroup id mod 8) cover a compact block of C tiles and
 // share A/B panels in that XCD's L2.  The epilogue stages each wave's fp16
-// tile in LDS and writes 16-byte row chunks (accumulating calls add C per
-// element instead, with one rounding of the fp32 sum).
+// tile in LDS and writes 16-byte row chunks; a call that adds to C reads it in
+// such chunks too, and rounds the fp32 sum once.
 constexpr int MB_K = 64;  // BK
 
 typedef __attribute__((address_space(3))) void lds_void;
@@ -793,20 +793,25 @@ bool short_k_wins(const GemmArgs& a, int batch, bool tb) {
 // fixed + steps * (step1 .. step_r, linear in j) us on them, steps being the
 // 64-deep K tiles of one K group; the launch ends with its fullest CU, and
 // the part of a last round that leaves CUs idle runs up to `slack` faster
-// (less traffic beside it).  The constants are a least-squares fit to 300
-// random products (17 <= M <= 8192, N up to 12288, K up to 8192, every
-// operand order) whose operands come from outside the L2, as between the
-// layers of a model: the instance it picks is within 1.6 % of the fastest of
-// 17 on average.  Before, three tile sizes were chosen by tile count alone;
+// (less traffic beside it).  The constants are a least-squares fit to random
+// products (17 <= M <= 8192, N up to 12288, K up to 8192, every operand order)
+// whose operands come from outside the L2, as between the layers of a model.
+// Over 160 others of that range the instance it picks takes 0.6 % longer than
+// the fastest on average, 26 % at worst (profiles/gemm_instance_times.txt).
+// Four K groups of 64 x 64 with two stages are not among them: up to 34 %
+// faster for a few tiles with a long K whose operands are in the L2 (24 x 24 x
+// 4096 16.8 -> 13.0 us), 8 to 80 % slower where they are not (16.7 -> 21.2).
+// Before, three tile sizes were chosen by tile count alone;
 // 128 x 128 ran on 4 waves with four LDS stages, one wave per SIMD.  8 waves,
 // or two K groups of 4 or 8, put two or more on a SIMD so that one's LDS
 // reads and waits overlap the other's MFMAs; two stages instead of four let
 // two workgroups share a CU, and more stages pay where a grid fits the CUs
 // once and the operands' latency shows.
-//   us, before -> now: 2560 x 3072 x 768 28.7 -> 17.3, its weight gradient
-//   (3072 x 768 over 2560) 39.5 -> 25.1, 1000 x 2304 x 768 13.8 -> 10.1,
-//   512 x 4096 x 4096 58.5 -> 28.0, 2048^3 32.4 -> 24.0, 40 x 11008 x 4096
-//   21.0 -> 18.1, 2560 x 768 x 32000 (B transposed) 247 -> 173
+//   us over rotating operands, before -> now: 2560 x 3072 x 768 28.8 -> 16.1,
+//   its weight gradient (3072 x 768 over 2560) 37.8 -> 25.1, 1000 x 2304 x 768
+//   13.9 -> 10.1, 512 x 4096 x 4096 57.1 -> 25.7, 2048^3 31.9 -> 22.4, 40 x
+//   11008 x 4096 28.3 -> 23.1, 2560 x 768 x 32000 (B transposed) 226 -> 161
+//   (195 behind the loss in a training step)
 struct GemmPlan {
     int bm, bn, waves, kg, stages, resident;
     float launch, fixed, step1, step_r, slack;
@@ -1009,11 +1014,14 @@ int gemm_dispatch(const GemmArgs& a, int batch, bool ta, bool tb, bool vec_ok, h
     // The LDS-direct loads address each operand through a buffer descriptor
     // and take whole, aligned 16-byte chunks; every other operand (odd row
     // lengths, pointers off a 16-byte boundary, 2 GiB and more) goes through
-    // registers (kRagPlans).  Against the kernels that served
+    // registers (kRagPlans), and so does a C of 2^31 elements and more, though
+    // no descriptor spans C.  Against the kernels that served
     // such calls before, one thread per element (odd rows) and a tiled one
     // with register transposes (2 GiB): 1000 x 1001 x 777 336 -> 18.2 us,
     // 3000 x 1501 x 801 1116 -> 53 us, 51 x 50 x 1481 179 -> 13.7 us;
-    // 131136 x 256 x 8192 1240 -> 1222 us, A stored (K,M) 1425 -> 1176 us.
+    // 131136 x 256 x 8192 1326 -> 724 us, x 4096 x 8192 12.7 -> 10.3 ms, A
+    // stored (K,M) 131136 x 2048 x 8192 8.0 -> 5.7 ms; 70000 x 32000 x 768 6.5
+    // -> 4.5 ms.
     const bool direct = vec_ok && (int64_t)a.M * a.K * 2 < INT32_MAX && (int64_t)a.K * a.N * 2 < INT32_MAX &&
                         (int64_t)a.M * a.N < INT32_MAX;
     if (!vec_ok && a.epi == GEMM_STORE && short_k_wins(a, batch, tb)) {

@@ -261,7 +261,10 @@ __global__ __launch_bounds__(EW_NT) void causal_mask_k(f16* scores, int64_t n, i
 // not, so a batch of EB_LD rows is requested at once.  One thread per
 // dimension walking all of idx (a chain of dependent memory accesses, three
 // workgroups for 768 dimensions) took 1275 us for 2560 rows of 768 with the
-// token frequencies of text, 32000 tokens; this takes about 40.
+// token frequencies of text, 32000 tokens; this takes 20 alone and 28 in a
+// training step.  Every workgroup reads the token's sums up front, only the
+// first row's uses and writes them (read once it is known to be the first:
+// up to 5 % slower).
 constexpr int EB_NT = 256, EB_IDS = 8, EB_CHUNK = EB_NT * EB_IDS, EB_LD = 16;
 
 // A handful of ids: a thread per dimension walks them, one or two memory round
